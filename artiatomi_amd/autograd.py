@@ -116,7 +116,10 @@ def _bb_descent(grad_at, s0: torch.Tensor, steps: int, first_step_px: float, max
         g_new = grad_at(s_new)
         ds, dg = s_new - s, g_new - g
         den = (ds * dg).sum(1, keepdim=True)
-        alpha = torch.where(den > 0, (ds * ds).sum(1, keepdim=True) / den.clamp_min(1e-300), alpha)
+        # at the optimum dg is rounding alone and den may be any small number: a step length grows at
+        # most 100-fold, so that such a row stays near its optimum
+        alpha = torch.where(den > 0, torch.minimum((ds * ds).sum(1, keepdim=True) / den.clamp_min(1e-300),
+                                                   100.0 * alpha), alpha)
         s, g = s_new, g_new
         if callback:
             callback(k + 2, s)

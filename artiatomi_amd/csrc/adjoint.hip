@@ -9,6 +9,7 @@
 //                  shift moves the detector origin by -shift_x*u - shift_y*v (Projection.cpp:183-195)
 //                  and with it every sample: dq_k/ds = scale * (-u + (dt_in/ds) n) per sub-ray.
 #include "artia_internal.hpp"
+#include "flat_walk.hpp"
 #include "fp_common.hpp"
 #include "tube_walk.hpp"
 
@@ -60,6 +61,13 @@ __global__ void __launch_bounds__(256) fp_adjoint_kernel(VolG v, TiltG g, const 
     const double px = (double)x + ((sub & 2) ? 0.75 : 0.25);
     const double py = (double)y + ((sub & 1) ? 0.75 : 0.25);
     if (!subray_samples(v, g, px, py, step, s)) return;
+    if (g.n[1] == 0.0f) {   // uniform
+        const FlatDir d = flat_dir(s.dq);
+        FlatWalker w;
+        w.init(d, s.q0, s.count);
+        flat_scatter_direct(v, grad, d, s.q0, r, w, []() { return true; });
+        return;
+    }
     for_each_cell(s.q0, s.dq, s.count, [&](const int cell[3], int k, int mi) {
         size_t o[8];
         cell_corners<kBig>(v, cell, o);
@@ -75,22 +83,23 @@ __global__ void __launch_bounds__(256) fp_adjoint_kernel(VolG v, TiltG g, const 
 
 // The same transpose with each tile's rays walked through LDS-staged slabs (tube_walk.hpp): the
 // weights are summed per slab in a box of shared memory and added to grad with one atomic per box
-// voxel, not eight per cell.  Tiles are dealt to the XCDs in groups, as in the forward projector.
+// voxel, not eight per cell.  Tiles are dealt to the XCDs in groups, as in the forward projector.  A wave
+// takes one sub-ray of every pixel of the tile, so that its lanes are a pixel apart and rarely add to the
+// same voxel at once.
+template <bool kFlat>
 __global__ void __launch_bounds__(256) fp_adjoint_lds_kernel(VolG v, TiltG g, const float* __restrict__ resid,
                                                              size_t pitch, Roi roi, float scale,
                                                              float* __restrict__ grad, TubePlan tp) {
     __shared__ float chunk[kChunkFloats];
     __shared__ int zr[2];
-    const int lane = (int)(threadIdx.x & 63), wave = (int)(threadIdx.x >> 6);
-    const int sub = lane & 3, pix = lane >> 2;
+    const int pix = (int)(threadIdx.x & 63), sub = (int)(threadIdx.x >> 6);
     const int xcd = (int)(blockIdx.x & 7u), slot = (int)(blockIdx.x >> 3);
     const int grp = (slot / (kXcdGroup * kXcdGroup)) * 8 + xcd, mem = slot % (kXcdGroup * kXcdGroup);
     const int gtx = (grp % tp.groups_x) * kXcdGroup + mem % kXcdGroup;
     const int gty = (grp / tp.groups_x) * kXcdGroup + mem / kXcdGroup;
     if (gtx >= tp.tiles_x || gty >= tp.tiles_y) return;   // whole workgroup
     const int tx0 = roi.x0 + gtx * 8, ty0 = roi.y0 + gty * 8;
-    const int x = tx0 + (wave & 1) * 4 + (pix & 3);
-    const int y = ty0 + (wave >> 1) * 4 + (pix >> 2);
+    const int x = tx0 + (pix & 7), y = ty0 + (pix >> 3);
     const double step = (double)v.vs[0] * 0.15;
     double r = 0.0;
     SubraySamples s;
@@ -104,9 +113,15 @@ __global__ void __launch_bounds__(256) fp_adjoint_lds_kernel(VolG v, TiltG g, co
         const double py = (double)y + ((sub & 1) ? 0.75 : 0.25);
         if (r == 0.0 || !subray_samples(v, g, px, py, step, s)) s.count = 0;
     }
-    const TubeDir td = tube_dir(v, g, step);
     const TubeBox tb = tube_box(v, g, tp, (double)tx0 + 0.25, (double)tx0 + 7.75, (double)ty0 + 0.25,
                                 (double)ty0 + 7.75, 0.0, 0.0);
+    if (kFlat) {
+        float dq[3];
+        tube_step(v, g, step, dq);
+        flat_tube_scatter(v, grad, chunk, zr, tp, tb, dq, s.q0, s.count, r);
+        return;
+    }
+    const TubeDir td = tube_dir(v, g, step);
     tube_scatter(v, grad, chunk, zr, tp, tb, td, s.q0, s.count, [&](float wgt[8], const int cell[3], int k, int mi) {
         double W[8];
         cell_weights(cell_moments(s.q0, td.dq, cell, k, mi), W);
@@ -247,8 +262,12 @@ artia_status artia_fp_adjoint(artia_ctx* ctx, const artia_vol_geom* vg, const ar
         tp.groups_x = (tp.tiles_x + kXcdGroup - 1) / kXcdGroup;
         const int groups = tp.groups_x * ((tp.tiles_y + kXcdGroup - 1) / kXcdGroup);
         const dim3 grid1((unsigned)(((groups + 7) / 8) * 8 * kXcdGroup * kXcdGroup));
-        hipLaunchKernelGGL(fp_adjoint_lds_kernel, grid1, dim3(256), 0, ctx->stream, vd, gd, resid, pitch, r, scale,
-                           vol_grad, tp);
+        if (gd.n[1] == 0.0f)
+            hipLaunchKernelGGL(fp_adjoint_lds_kernel<true>, grid1, dim3(256), 0, ctx->stream, vd, gd, resid, pitch, r,
+                               scale, vol_grad, tp);
+        else
+            hipLaunchKernelGGL(fp_adjoint_lds_kernel<false>, grid1, dim3(256), 0, ctx->stream, vd, gd, resid, pitch, r,
+                               scale, vol_grad, tp);
     } else if (r.x1 > r.x0 && r.y1 > r.y0)
     {
         const bool big = (double)vg->nx * (double)vg->ny * (double)vg->nz >= 1073741824.0;

@@ -18,6 +18,7 @@
 #include <cmath>
 
 #include "device_common.hpp"
+#include "flat_walk.hpp"
 #include "fp_common.hpp"
 #include "image_ops.hpp"
 #include "tube_walk.hpp"
@@ -279,31 +280,36 @@ __global__ void __launch_bounds__(256, 5) march_ref_lds_kernel(VolG v, TiltG g, 
 
 // Sum of the trilinear samples q0 + k*dq, k = 0..count-1 (coordinates shifted by -0.5, texel j
 // centred at j), cell by cell in closed form (cell_sum, fp_common.hpp).
-// kFlat: dq[1] == 0 (the walk, moments and cell sums without the y terms; the same values).
+// kFlat: dq[1] == 0 (the walk of flat_walk.hpp).
 template <bool kBig, bool kFlat, typename T>
 __device__ __forceinline__ double march_sum(const VolG& v, const T* __restrict__ vol, const float q0[3],
                                             const float dq[3], int count) {
     double total = 0.0;
-    if (kBig) {
-        for_each_cell<kFlat>(q0, dq, count, [&](const auto* cell, auto k, auto mi) {
-            const int ic[3] = {(int)cell[0], (int)cell[1], (int)cell[2]};
+    if (kFlat) {
+        const FlatDir d = flat_dir(dq);
+        FlatWalker w;
+        w.init(d, q0, count);
+        flat_walk_direct<kBig>(v, vol, d, q0, w, []() { return true; },
+                               [&](float A, float B, float C, float D, float, float, float, float, float a, float c,
+                                   float m) { total += (double)flat_cell_sum(A, B, C, D, a, c, m, d.K); });
+    } else if (kBig) {
+        for_each_cell(q0, dq, count, [&](const int cell[3], int k, int mi) {
             size_t o[8];
-            cell_corners<true>(v, ic, o);
+            cell_corners<true>(v, cell, o);
             float val[8];
 #pragma unroll
             for (int i = 0; i < 8; i++) val[i] = vox(vol, o[i]);
-            total += cell_sum_values<kFlat>(val, cell_moments<kFlat>(q0, dq, cell, k, mi), mi);
+            total += cell_sum_values(val, cell_moments(q0, dq, cell, k, mi));
         });
     } else {
         const __amdgpu_buffer_rsrc_t rs = volume_rsrc(vol, v);
-        for_each_cell<kFlat>(q0, dq, count, [&](const auto* cell, auto k, auto mi) {
-            const int ic[3] = {(int)cell[0], (int)cell[1], (int)cell[2]};
+        for_each_cell(q0, dq, count, [&](const int cell[3], int k, int mi) {
             uint32_t o[8];
-            cell_corners_bytes<(uint32_t)sizeof(T)>(v, ic, o);
+            cell_corners_bytes<(uint32_t)sizeof(T)>(v, cell, o);
             float val[8];
 #pragma unroll
             for (int i = 0; i < 8; i++) val[i] = buffer_vox(rs, o[i], vol);
-            total += cell_sum_values<kFlat>(val, cell_moments<kFlat>(q0, dq, cell, k, mi), mi);
+            total += cell_sum_values(val, cell_moments(q0, dq, cell, k, mi));
         });
     }
     return total;
@@ -490,14 +496,23 @@ __global__ void __launch_bounds__(256, 6) march_lds_kernel(VolG v, TiltG g, cons
     float dval = 0.0f;
     if (kResid) dval = pixel_dist(L.len, L.hits);
     else if (!kSlicer) march_store_dist(L.len, L.hits, active, sub, x, y, pitch, dist);
-    const TubeDir td = tube_dir(v, g, step);
     const TubeBox tb = tube_box(v, g, tp, (double)tx0 + 0.25, (double)tx0 + 7.75, (double)ty0 + 0.25,
                                 (double)ty0 + 7.75, 0.0, 0.0);
     double total = 0.0;   // summed as march_sum does, then added to the slicer's first sample
-    tube_walk<kFlat, true>(v, vol, chunk, zr, tp, tb, td, L.q0, L.count,
-                     [&](const float val[8], const auto* cell, auto k, auto mi) {
-                         total += cell_sum_values<kFlat>(val, cell_moments<kFlat>(L.q0, td.dq, cell, k, mi), mi);
-                     });
+    if (kFlat) {
+        float dq[3];
+        tube_step(v, g, step, dq);
+        const float K = flat_dir(dq).K;
+        flat_tube_walk<false>(v, vol, chunk, zr, tp, tb, dq, L.q0, L.count,
+                              [&](float A, float B, float C, float D, float, float, float, float, float a, float c,
+                                  float m) { total += (double)flat_cell_sum(A, B, C, D, a, c, m, K); });
+    } else {
+        const TubeDir td = tube_dir(v, g, step);
+        tube_walk<true>(v, vol, chunk, zr, tp, tb, td, L.q0, L.count,
+                        [&](const float val[8], const int* cell, int k, int mi) {
+                            total += cell_sum_values(val, cell_moments(L.q0, td.dq, cell, k, mi));
+                        });
+    }
     double acc = L.acc;
     if (L.count > 0) acc += total;
     if (kResid)
@@ -643,14 +658,22 @@ __global__ void __launch_bounds__(256, 6) slicer_segments_lds_kernel(VolG v, Til
             zb = (int)floor(fmax(qa, qb));
         }
     }
-    const TubeDir td = tube_dir(v, g, step);
     const TubeBox tb = tube_box(v, g, tp, (double)tx0 + 0.25, (double)tx0 + 7.75, (double)ty0 + 0.25,
                                 (double)ty0 + 7.75, 0.0, 0.0);
-    tube_walk_segments<kFlat, true>(v, vol, chunk, zr, tp, tb, td, za, zb, seg,
-                              [&](const float val[8], const auto* cell, auto kk, auto mi) {
-                                  seg.total += cell_sum_values<kFlat>(
-                                      val, cell_moments<kFlat>(seg.q0, td.dq, cell, kk, mi), mi);
-                              });
+    if (kFlat) {
+        float dq[3];
+        tube_step(v, g, step, dq);
+        const float K = flat_dir(dq).K;
+        flat_tube_segments(v, vol, chunk, zr, tp, tb, dq, za, zb, seg,
+                           [&](float A, float B, float C, float D, float, float, float, float, float a, float c,
+                               float m) { seg.total += (double)flat_cell_sum(A, B, C, D, a, c, m, K); });
+    } else {
+        const TubeDir td = tube_dir(v, g, step);
+        tube_walk_segments<true>(v, vol, chunk, zr, tp, tb, td, za, zb, seg,
+                                 [&](const float val[8], const int* cell, int kk, int mi) {
+                                     seg.total += cell_sum_values(val, cell_moments(seg.q0, td.dq, cell, kk, mi));
+                                 });
+    }
 }
 
 // Slab images from the sub-ray sums: stack[k * stride + y * pitch + x] = 0 + the four sub-rays'
@@ -724,7 +747,10 @@ void launch_exact_t(artia_ctx* ctx, const VolG& v, const TiltG& g_in, const T* v
         tp.groups_x = (tp.tiles_x + kXcdGroup - 1) / kXcdGroup;
         const int groups = tp.groups_x * ((tp.tiles_y + kXcdGroup - 1) / kXcdGroup);
         const dim3 grid1((unsigned)(((groups + 7) / 8) * 8 * kXcdGroup * kXcdGroup));
-        if (slicer)
+        if (slicer && flat)
+            hipLaunchKernelGGL((march_lds_kernel<true, false, T, true>), grid1, block, 0, ctx->stream, v, g, vol, r,
+                               pitch, proj, dist, tmin, tmax, tp, epi, W, H);
+        else if (slicer)
             hipLaunchKernelGGL((march_lds_kernel<true, false, T>), grid1, block, 0, ctx->stream, v, g, vol, r, pitch,
                                proj, dist, tmin, tmax, tp, epi, W, H);
         else if (flat)
@@ -735,7 +761,14 @@ void launch_exact_t(artia_ctx* ctx, const VolG& v, const TiltG& g_in, const T* v
                                pitch, proj, dist, tmin, tmax, tp, epi, W, H);
         return;
     }
-    if (slicer) {
+    if (slicer && flat) {
+        if (big)
+            hipLaunchKernelGGL((march_exact_kernel<true, true, false, T, true>), grid, block, 0, ctx->stream, v, g, vol,
+                               r, pitch, proj, dist, tmin, tmax, epi, W, H);
+        else
+            hipLaunchKernelGGL((march_exact_kernel<true, false, false, T, true>), grid, block, 0, ctx->stream, v, g,
+                               vol, r, pitch, proj, dist, tmin, tmax, epi, W, H);
+    } else if (slicer) {
         if (big)
             hipLaunchKernelGGL((march_exact_kernel<true, true, false, T>), grid, block, 0, ctx->stream, v, g, vol, r,
                                pitch, proj, dist, tmin, tmax, epi, W, H);

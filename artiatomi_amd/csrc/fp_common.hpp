@@ -133,6 +133,15 @@ __device__ __forceinline__ bool subray_samples(const VolG& v, const TiltG& g, do
     return true;
 }
 
+// Direction of one axis: the sign of dq and 1 / dq, or no crossings (sign 0) when dq is 0 or so
+// small that 1 / dq overflows (such an axis would cross no face within the walk's samples).
+__device__ __forceinline__ void walk_dir(float dq, int& sgn, float& inv) {
+    const float r = 1.0f / dq;
+    const bool ok = dq != 0.0f && __builtin_isfinite(r);
+    sgn = ok ? (dq > 0.0f ? 1 : -1) : 0;
+    inv = ok ? r : 0.0f;
+}
+
 // Walk over the cells of the texel lattice crossed by the samples q0 + k*dq, k = 0..count-1, in
 // order.  The sample index of the next crossing on axis i is recomputed from the cell index,
 // (face - q0_i) / dq_i, as one fma (its float error, a few 1e-4 samples for rays of thousands of
@@ -143,50 +152,31 @@ __device__ __forceinline__ bool subray_samples(const VolG& v, const TiltG& g, do
 // the next, active() says whether samples remain, so the walk can be resumed (the LDS-staged
 // projector runs it slab by slab).
 //
-// kFlat: the rays have no y component (dq[1] == 0 exactly, every tilt about the y axis whose beam
-// direction rounds to n_y = 0), so the walk never crosses a y face and the y axis drops out of the
-// step.  With dq[1] == 0 both forms visit the same cells with the same sample ranges.
-// Direction of one axis: the sign of dq and 1 / dq, or no crossings (sign 0) when dq is 0 or so
-// small that 1 / dq overflows (such an axis would cross no face within the walk's samples).
-__device__ __forceinline__ void walk_dir(float dq, int& sgn, float& inv) {
-    const float r = 1.0f / dq;
-    const bool ok = dq != 0.0f && __builtin_isfinite(r);
-    sgn = ok ? (dq > 0.0f ? 1 : -1) : 0;
-    inv = ok ? r : 0.0f;
-}
-
-// The walk without the y axis keeps its cell indices and sample counts in float (cell, k, and the m
-// passed to f): integers below 2^24, exact in float, which the cell moments and the crossing
-// indices take without conversions.
-template <bool kFlat>
-struct CellWalkerT {
-    using Index = typename std::conditional<kFlat, float, int>::type;
-    Index cell[3];
+// Rays without a y component take the walk of flat_walk.hpp instead.
+struct CellWalker {
+    int cell[3];
     int sgn[3];
     float inv[3], off[3], kb[3];
     float fcount;
-    Index k;
+    int k;
     int count, guard;
 
-    __device__ __forceinline__ int icell(int i) const { return (int)cell[i]; }
+    __device__ __forceinline__ int icell(int i) const { return cell[i]; }
     // whether the cell's z index lies in [zs, zs + n)
-    __device__ __forceinline__ bool z_in(int zs, int n) const {
-        if (kFlat) return cell[2] >= (Index)zs && cell[2] <= (Index)(zs + n - 1);
-        return (unsigned)((int)cell[2] - zs) <= (unsigned)(n - 1);
-    }
+    __device__ __forceinline__ bool z_in(int zs, int n) const { return (unsigned)(cell[2] - zs) <= (unsigned)(n - 1); }
 
     __device__ __forceinline__ void init(const float q0[3], const float dq[3], int n) {
 #pragma unroll
         for (int i = 0; i < 3; i++) {
-            cell[i] = (Index)floorf(q0[i]);
+            cell[i] = (int)floorf(q0[i]);
             walk_dir(dq[i], sgn[i], inv[i]);
             off[i] = -q0[i] * inv[i];
-            kb[i] = sgn[i] != 0 ? __builtin_fmaf((float)(cell[i] + (Index)(sgn[i] > 0 ? 1 : 0)), inv[i], off[i])
+            kb[i] = sgn[i] != 0 ? __builtin_fmaf((float)(cell[i] + (sgn[i] > 0 ? 1 : 0)), inv[i], off[i])
                                 : INFINITY;
         }
         count = n;
         fcount = (float)n;
-        k = (Index)0;
+        k = 0;
         guard = 0;
     }
     // The same walk with the direction part (sgn, inv) precomputed: when every lane walks parallel
@@ -194,16 +184,16 @@ struct CellWalkerT {
     __device__ __forceinline__ void init_dir(const float q0[3], const int sgn_u[3], const float inv_u[3], int n) {
 #pragma unroll
         for (int i = 0; i < 3; i++) {
-            cell[i] = (Index)floorf(q0[i]);
+            cell[i] = (int)floorf(q0[i]);
             sgn[i] = sgn_u[i];
             inv[i] = inv_u[i];
             off[i] = -q0[i] * inv[i];
-            kb[i] = sgn[i] != 0 ? __builtin_fmaf((float)(cell[i] + (Index)(sgn[i] > 0 ? 1 : 0)), inv[i], off[i])
+            kb[i] = sgn[i] != 0 ? __builtin_fmaf((float)(cell[i] + (sgn[i] > 0 ? 1 : 0)), inv[i], off[i])
                                 : INFINITY;
         }
         count = n;
         fcount = (float)n;
-        k = (Index)0;
+        k = 0;
         guard = 0;
     }
     // The walk of samples k0 .. n-1 of the same sub-ray, starting in the cell of sample k0 (crossing
@@ -212,20 +202,20 @@ struct CellWalkerT {
                                               const float inv_u[3], int k0, int n) {
 #pragma unroll
         for (int i = 0; i < 3; i++) {
-            cell[i] = (Index)floorf(__builtin_fmaf((float)k0, dq[i], q0[i]));
+            cell[i] = (int)floorf(__builtin_fmaf((float)k0, dq[i], q0[i]));
             sgn[i] = sgn_u[i];
             inv[i] = inv_u[i];
             off[i] = -q0[i] * inv[i];
-            kb[i] = sgn[i] != 0 ? __builtin_fmaf((float)(cell[i] + (Index)(sgn[i] > 0 ? 1 : 0)), inv[i], off[i])
+            kb[i] = sgn[i] != 0 ? __builtin_fmaf((float)(cell[i] + (sgn[i] > 0 ? 1 : 0)), inv[i], off[i])
                                 : INFINITY;
         }
         count = n;
         fcount = (float)n;
-        k = (Index)k0;
+        k = k0;
         guard = 0;
     }
     __device__ __forceinline__ bool active() const {
-        return (kFlat ? (float)k < fcount : (int)k < count) && guard < 4 * count + 64;
+        return k < count && guard < 4 * count + 64;
     }
     // One step; moved(i) is called for every axis i the walk advances along.  The next crossing kn
     // is the least of the axes' crossing indices (never NaN: finite, or INFINITY on an axis without
@@ -245,21 +235,13 @@ struct CellWalkerT {
     template <bool kAll, class F, class M>
     __device__ __forceinline__ void step_impl(F&& f, M&& moved) {
         bool adv[3];
-        float kn;
-        if (kFlat) {
-            adv[0] = kb[0] <= kb[2];
-            adv[1] = false;
-            adv[2] = kb[2] <= kb[0];
-            kn = adv[0] ? kb[0] : kb[2];
-        } else {
-            const float kxy = kb[0] <= kb[1] ? kb[0] : kb[1];
-            kn = kxy <= kb[2] ? kxy : kb[2];
+        const float kxy = kb[0] <= kb[1] ? kb[0] : kb[1];
+        const float kn = kxy <= kb[2] ? kxy : kb[2];
 #pragma unroll
-            for (int i = 0; i < 3; i++) adv[i] = kb[i] == kn;
-        }
-        const Index kend = (Index)__builtin_amdgcn_fmed3f(ceilf(kn), 0.0f, fcount);
+        for (int i = 0; i < 3; i++) adv[i] = kb[i] == kn;
+        const int kend = (int)__builtin_amdgcn_fmed3f(ceilf(kn), 0.0f, fcount);
         if (kAll) {
-            const Index mi = kend - k > (Index)0 ? kend - k : (Index)0;
+            const int mi = max(kend - k, 0);
             f(cell, k, mi);
             k += mi;
         } else if (kend > k) {
@@ -268,10 +250,9 @@ struct CellWalkerT {
         }
 #pragma unroll
         for (int i = 0; i < 3; i++) {
-            if (kFlat && i == 1) continue;
             if (adv[i]) {
-                cell[i] += (Index)sgn[i];
-                kb[i] = __builtin_fmaf((float)(cell[i] + (Index)(sgn[i] > 0 ? 1 : 0)), inv[i], off[i]);
+                cell[i] += sgn[i];
+                kb[i] = __builtin_fmaf((float)(cell[i] + (sgn[i] > 0 ? 1 : 0)), inv[i], off[i]);
                 moved(i);
             }
         }
@@ -283,12 +264,10 @@ struct CellWalkerT {
     }
 };
 
-using CellWalker = CellWalkerT<false>;
-
 // The whole walk: f(cell, k, m) for every cell holding samples k..k+m-1, in order.
-template <bool kFlat = false, class F>
+template <class F>
 __device__ __forceinline__ void for_each_cell(const float q0[3], const float dq[3], int count, F&& f) {
-    CellWalkerT<kFlat> w;
+    CellWalker w;
     w.init(q0, dq, count);
     while (w.active()) w.step(f);
 }
@@ -301,34 +280,21 @@ __device__ __forceinline__ void for_each_cell(const float q0[3], const float dq[
 struct CellMoments {
     float a, b, c, S2c, m;
     float pab, pac, pbc, q;   // da db, da dc, db dc, a db dc + b da dc + c da db
-    bool flat;                // db == 0: b is the same for every sample
 };
 
-// kFlat (dq[1] == 0): b is the same for every sample, da db = db dc = 0 and q = b da dc; the
-// values equal the general form's (fma(kc, 0, q0) = q0, fma(x, 0, y) = y for finite operands).
-// cell, k and mi are ints, or (the walk without the y axis) floats holding the same integers.
-template <bool kFlat = false, typename C, typename K>
-__device__ __forceinline__ CellMoments cell_moments(const float q0[3], const float dq[3], const C* cell, K k, K mi) {
+__device__ __forceinline__ CellMoments cell_moments(const float q0[3], const float dq[3], const int* cell, int k,
+                                                    int mi) {
     CellMoments cm;
-    // k + (m - 1) / 2, exact: integer sums below 2^24 halved; in float as m / 2 + (k - 1/2), whose
-    // half-integer terms and sum are exact too
-    const float kc = std::is_same<K, float>::value ? __builtin_fmaf((float)mi, 0.5f, (float)k - 0.5f)
-                                                   : (float)(k + (k + mi) - 1) * 0.5f;
+    const float kc = (float)(k + (k + mi) - 1) * 0.5f;   // k + (m - 1) / 2, exact
     cm.a = __builtin_fmaf(kc, dq[0], q0[0]) - (float)cell[0];
-    cm.b = (kFlat ? q0[1] : __builtin_fmaf(kc, dq[1], q0[1])) - (float)cell[1];
+    cm.b = __builtin_fmaf(kc, dq[1], q0[1]) - (float)cell[1];
     cm.c = __builtin_fmaf(kc, dq[2], q0[2]) - (float)cell[2];
     cm.m = (float)mi;
     cm.S2c = cm.m * __builtin_fmaf(cm.m, cm.m, -1.0f) * (1.0f / 12.0f);   // m, m^2 - 1 and their product exact
+    cm.pab = dq[0] * dq[1];
     cm.pac = dq[0] * dq[2];
-    cm.flat = kFlat || dq[1] == 0.0f;
-    if (kFlat) {
-        cm.pab = cm.pbc = 0.0f;
-        cm.q = cm.b * cm.pac;
-    } else {
-        cm.pab = dq[0] * dq[1];
-        cm.pbc = dq[1] * dq[2];
-        cm.q = __builtin_fmaf(cm.a, cm.pbc, __builtin_fmaf(cm.b, cm.pac, cm.c * cm.pab));
-    }
+    cm.pbc = dq[1] * dq[2];
+    cm.q = __builtin_fmaf(cm.a, cm.pbc, __builtin_fmaf(cm.b, cm.pac, cm.c * cm.pab));
     return cm;
 }
 
@@ -391,24 +357,9 @@ __device__ __forceinline__ float buffer_vox(const __amdgpu_buffer_rsrc_t rs, uin
 // Sum of one cell's m samples, m f(centre) + S2c corr, rounded once to float (relative error
 // 6e-8 per cell); the ray adds the cells in double, so per-cell roundings do not accumulate into a
 // float running sum.
-// db = 0 (cm.flat; always under kFlat): b is the same for every sample and the cell is a
-// bilinear interpolant in (a, c) of its four y-blended edges w_xz = lerp(v_x0z, v_x1z, b): the
-// samples sum to m g(centre) + S2c (w11 - w01 - w10 + w00) da dc.  Every kernel takes this form
-// for such rays, so their sums agree bit for bit whatever walk they run.
-template <bool kFlat = false>
-__device__ __forceinline__ double cell_sum_values(const float val[8], const CellMoments& cm, int mi) {
+__device__ __forceinline__ double cell_sum_values(const float val[8], const CellMoments& cm) {
     const float v000 = val[0], v100 = val[1], v010 = val[2], v110 = val[3];
     const float v001 = val[4], v101 = val[5], v011 = val[6], v111 = val[7];
-    (void)mi;
-    if (kFlat || cm.flat) {
-        const float w00 = lerpf(v000, v010, cm.b), w10 = lerpf(v100, v110, cm.b);
-        const float w01 = lerpf(v001, v011, cm.b), w11 = lerpf(v101, v111, cm.b);
-        const float d0 = w10 - w00, d1 = w11 - w01;
-        const float g = lerpf(__builtin_fmaf(cm.a, d0, w00), __builtin_fmaf(cm.a, d1, w01), cm.c);
-        // S2c da dc = m (m^2 - 1) (da dc / 12): the integer product exact, the ray's da dc / 12 hoisted
-        const float spac = (cm.m * __builtin_fmaf(cm.m, cm.m, -1.0f)) * (cm.pac * (1.0f / 12.0f));
-        return (double)__builtin_fmaf(cm.m, g, (d1 - d0) * spac);
-    }
     // x differences, shared by the x lerps and the mixed differences
     const float x00 = v100 - v000, x10 = v110 - v010, x01 = v101 - v001, x11 = v111 - v011;
     const float c00 = __builtin_fmaf(cm.a, x00, v000), c10 = __builtin_fmaf(cm.a, x10, v010);
@@ -442,25 +393,9 @@ __device__ __forceinline__ void cell_weights(const CellMoments& cm, double W[8])
 // + ABC b c sums to m (d f/da)(centre) + S2c ABC db dc, and likewise for b and c.  Where a corner
 // index is clamped its step vanishes, and with it the derivative along that axis, as for the
 // clamp-addressed read.  Accumulated into G.
-// db = 0 (cm.flat): the x and z derivatives are those of the bilinear interpolant in (a, c) of the
-// y-blended edges w_xz that the cell sum forms (shared with it), the y derivative interpolates the
-// y differences in (a, c), and with da db = db dc = 0 only the y derivative keeps a correction.
-__device__ __forceinline__ void cell_grad_sum(const float val[8], const CellMoments& cm, int mi, double G[3]) {
+__device__ __forceinline__ void cell_grad_sum(const float val[8], const CellMoments& cm, double G[3]) {
     const float v000 = val[0], v100 = val[1], v010 = val[2], v110 = val[3];
     const float v001 = val[4], v101 = val[5], v011 = val[6], v111 = val[7];
-    if (cm.flat) {
-        const float w00 = lerpf(v000, v010, cm.b), w10 = lerpf(v100, v110, cm.b);
-        const float w01 = lerpf(v001, v011, cm.b), w11 = lerpf(v101, v111, cm.b);
-        const float ga = lerpf(w10 - w00, w11 - w01, cm.c);
-        const float gc = lerpf(w01 - w00, w11 - w10, cm.a);
-        const float y00 = v010 - v000, y10 = v110 - v100, y01 = v011 - v001, y11 = v111 - v101;
-        const float gb = lerpf(lerpf(y00, y10, cm.a), lerpf(y01, y11, cm.a), cm.c);
-        const float ABCf = (y11 - y01) - (y10 - y00);
-        G[0] += (double)(cm.m * ga);
-        G[1] += (double)__builtin_fmaf(cm.m, gb, (cm.S2c * ABCf) * cm.pac);
-        G[2] += (double)(cm.m * gc);
-        return;
-    }
     const float ABC = ((v111 - v110) - (v101 - v100)) - ((v011 - v010) - (v001 - v000));
     // d f / d a at the centre: the x-differences interpolated in b, then c (likewise for b and c)
     const float ga = lerpf(lerpf(v100 - v000, v110 - v010, cm.b), lerpf(v101 - v001, v111 - v011, cm.b), cm.c);

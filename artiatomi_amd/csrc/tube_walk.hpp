@@ -74,11 +74,18 @@ struct TubeDir {
     int sgn[3];
 };
 
+__device__ __forceinline__ void tube_step(const VolG& v, const TiltG& g, double step, float dq[3]) {
+#pragma unroll
+    for (int i = 0; i < 3; i++) dq[i] = (float)(step * (double)g.n[i] * ((double)v.rcp[i] * (double)v.dim[i]));
+}
+
 __device__ __forceinline__ TubeDir tube_dir(const VolG& v, const TiltG& g, double step) {
     TubeDir d;
+    float dq[3];
+    tube_step(v, g, step, dq);
 #pragma unroll
     for (int i = 0; i < 3; i++) {
-        d.dq[i] = wave_uniform((float)(step * (double)g.n[i] * ((double)v.rcp[i] * (double)v.dim[i])));
+        d.dq[i] = wave_uniform(dq[i]);
         float inv;
         walk_dir(d.dq[i], d.sgn[i], inv);
         d.inv[i] = wave_uniform(inv);
@@ -291,17 +298,7 @@ __device__ __forceinline__ void stage_box_rows(const VolG& v, const T* __restric
 //   scatter (kScatter true): f(float wgt[8], cell, k, m) returns eight corner weights, which are
 //     added to the slab's box in LDS (shared-memory atomics) and then to grad with one global
 //     atomic per box voxel, instead of eight global atomics per cell.
-// Box offset cell[2] * CXY + cell[0] + K of a cell of the walk without the y axis: float cells
-// (integers; tube_plan keeps |cell[2] * CXY| below 2^24, so every term and sum is exact) in one fma,
-// int cells in one 24-bit multiply-add.
-__device__ __forceinline__ int flat_box_offset(const float* cell, int CXY, int K) {
-    return (int)__builtin_fmaf(cell[2], (float)CXY, cell[0] + (float)K);
-}
-__device__ __forceinline__ int flat_box_offset(const int* cell, int CXY, int K) {
-    return __mul24(cell[2], CXY) + (cell[0] + K);
-}
-
-template <bool kScatter, bool kFlat, bool kRows, typename T, class F>
+template <bool kScatter, bool kRows, typename T, class F>
 __device__ __forceinline__ void tube_slabs(const VolG& v, const T* __restrict__ vol, float* __restrict__ grad,
                                            float* __restrict__ chunk, int* zr, const TubePlan& tp, const TubeBox& tb,
                                            const TubeDir& td, const float q0[3], int count, F&& f) {
@@ -329,7 +326,7 @@ __device__ __forceinline__ void tube_slabs(const VolG& v, const T* __restrict__ 
         for (int i = 0; i < 8; i++)
             if (wgt[i] != 0.0f) unsafeAtomicAdd(grad + o[i], wgt[i]);
     };
-    CellWalkerT<kFlat> w;
+    CellWalker w;
     w.init_dir(q0, td.sgn, td.inv, count);
     const int nslab = zlo <= zhi ? (zhi - zlo) / kSlabCells + 1 : 0;
     for (int j = 0; j < nslab; j++) {
@@ -381,7 +378,7 @@ __device__ __forceinline__ void tube_slabs(const VolG& v, const T* __restrict__ 
             if (kScatter) {
                 while (w.active() && w.z_in(zs, kSlabCells)) {
                     w.step(
-                        [&](const auto* cell, auto k, auto mi) {
+                        [&](const int* cell, int k, int mi) {
                             float val[8];
                             f(val, cell, k, mi);
 #pragma unroll
@@ -394,41 +391,24 @@ __device__ __forceinline__ void tube_slabs(const VolG& v, const T* __restrict__ 
                 // every step reads its cell's corners and calls f, also for a cell without samples
                 // (f adds +-0 then: the gather callbacks add cell and gradient sums), so the loop
                 // body has no branch
-                if (kFlat) {
-                    // y is fixed: the box offset is one 24-bit multiply-add of the x and z indices
-                    // per step instead of a select and add per axis
-                    const int K = (w.icell(1) - Y0) * CX - X0 - Z0 * CXY;
-                    while (w.active() && w.z_in(zs, kSlabCells)) {
-                        w.step_all(
-                            [&](const auto* cell, auto k, auto mi) {
-                                const int oc = flat_box_offset(cell, CXY, K);
-                                float val[8];
+                while (w.active() && w.z_in(zs, kSlabCells)) {
+                    w.step_all(
+                        [&](const int* cell, int k, int mi) {
+                            float val[8];
 #pragma unroll
-                                for (int i = 0; i < 8; i++) val[i] = chunk[oc + off[i]];
-                                f(val, cell, k, mi);
-                            },
-                            [](int) {});
-                    }
-                } else {
-                    while (w.active() && w.z_in(zs, kSlabCells)) {
-                        w.step_all(
-                            [&](const auto* cell, auto k, auto mi) {
-                                float val[8];
-#pragma unroll
-                                for (int i = 0; i < 8; i++) val[i] = chunk[o + off[i]];
-                                f(val, cell, k, mi);
-                            },
-                            [&](int i) { o += i == 0 ? st0 : (i == 1 ? st1 : st2); });
-                    }
+                            for (int i = 0; i < 8; i++) val[i] = chunk[o + off[i]];
+                            f(val, cell, k, mi);
+                        },
+                        [&](int i) { o += i == 0 ? st0 : (i == 1 ? st1 : st2); });
                 }
             }
         } else {
             while (w.active() && (tp.zdir > 0 ? w.icell(2) <= ze : w.icell(2) >= zs)) {
-                w.step([&](const auto* cell, auto k, auto mi) {
+                w.step([&](const int* cell, int k, int mi) {
                     float val[8];
                     if (kScatter) {
                         f(val, cell, k, mi);
-                        const int ic[3] = {(int)cell[0], (int)cell[1], (int)cell[2]};
+                        const int ic[3] = {cell[0], cell[1], cell[2]};
                         const int cx = ic[0] - X0, cy = ic[1] - Y0, cz = ic[2] - Z0;
                         if (staged && (unsigned)cx < (unsigned)(CX - 1) && (unsigned)cy < (unsigned)(CY - 1) &&
                             (unsigned)cz < (unsigned)(CZ - 1)) {
@@ -441,7 +421,7 @@ __device__ __forceinline__ void tube_slabs(const VolG& v, const T* __restrict__ 
                             scatter_global(ic, val);
                         }
                     } else {
-                        const int ic[3] = {(int)cell[0], (int)cell[1], (int)cell[2]};
+                        const int ic[3] = {cell[0], cell[1], cell[2]};
                         chunk_corners(v, vol, chunk, staged, X0, Y0, Z0, CX, CY, CZ, ic, val);
                         f(val, cell, k, mi);
                     }
@@ -462,9 +442,9 @@ __device__ __forceinline__ void tube_slabs(const VolG& v, const T* __restrict__ 
     }
     // cells beyond the slabs (not expected): global memory
     while (w.active()) {
-        w.step([&](const auto* cell, auto k, auto mi) {
+        w.step([&](const int* cell, int k, int mi) {
             float val[8];
-            const int ic[3] = {(int)cell[0], (int)cell[1], (int)cell[2]};
+            const int ic[3] = {cell[0], cell[1], cell[2]};
             if (kScatter) {
                 f(val, cell, k, mi);
                 scatter_global(ic, val);
@@ -486,9 +466,9 @@ __device__ __forceinline__ void tube_slabs(const VolG& v, const T* __restrict__ 
 // each other along the rays, so one pass over the slabs of cell layers serves all of them; za..zb
 // are cell layers bounding every sample of the lane (za > zb: none).  Each segment is walked with
 // tube_slabs' CellWalker steps, so its cells, their order and their values are those of a
-// tube_walk of that segment alone (kFlat: the walk without the y axis, as tube_walk<true>).  Must
+// tube_walk of that segment alone.  Must
 // be called by all 256 threads of the block.
-template <bool kFlat, bool kRows, typename T, class Seg, class F>
+template <bool kRows, typename T, class Seg, class F>
 __device__ __forceinline__ void tube_walk_segments(const VolG& v, const T* __restrict__ vol,
                                                    float* __restrict__ chunk, int* zr, const TubePlan& tp,
                                                    const TubeBox& tb, const TubeDir& td, int za, int zb, Seg& seg,
@@ -506,7 +486,7 @@ __device__ __forceinline__ void tube_walk_segments(const VolG& v, const T* __res
     __syncthreads();
     const int zlo = max(zr[0], -1), zhi = min(zr[1], v.nz - 1);
 
-    CellWalkerT<kFlat> w;
+    CellWalker w;
     w.init_dir(seg.q0, td.sgn, td.inv, 0);   // no segment yet: the first pass below loads one
     bool more = true;
     const int nslab = zlo <= zhi ? (zhi - zlo) / kSlabCells + 1 : 0;
@@ -558,37 +538,21 @@ __device__ __forceinline__ void tube_walk_segments(const VolG& v, const T* __res
                 int o = ((w.icell(2) - Z0) * CY + (w.icell(1) - Y0)) * CX + (w.icell(0) - X0);
                 // every step reads its cell's corners and calls f, also for a cell without
                 // samples (f adds +-0 then), so the loop body has no branch
-                if (kFlat) {
-                    // y is fixed: the box offset is one 24-bit multiply-add of the x and z indices
-                    const int K = (w.icell(1) - Y0) * CX - X0 - Z0 * CXY;
-                    while (w.active() && w.z_in(zs, kSlabCells)) {
-                        w.step_all(
-                            [&](const auto* cell, auto k, auto mi) {
-                                const int oc = flat_box_offset(cell, CXY, K);
-                                float val[8];
+                while (w.active() && w.z_in(zs, kSlabCells)) {
+                    w.step_all(
+                        [&](const int* cell, int k, int mi) {
+                            float val[8];
 #pragma unroll
-                                for (int i = 0; i < 8; i++) val[i] = chunk[oc + off[i]];
-                                f(val, cell, k, mi);
-                            },
-                            [](int) {});
-                    }
-                } else {
-                    while (w.active() && w.z_in(zs, kSlabCells)) {
-                        w.step_all(
-                            [&](const auto* cell, auto k, auto mi) {
-                                float val[8];
-#pragma unroll
-                                for (int i = 0; i < 8; i++) val[i] = chunk[o + off[i]];
-                                f(val, cell, k, mi);
-                            },
-                            [&](int i) { o += i == 0 ? st0 : (i == 1 ? st1 : st2); });
-                    }
+                            for (int i = 0; i < 8; i++) val[i] = chunk[o + off[i]];
+                            f(val, cell, k, mi);
+                        },
+                        [&](int i) { o += i == 0 ? st0 : (i == 1 ? st1 : st2); });
                 }
             } else {
                 while (w.active() && (tail || (tp.zdir > 0 ? w.icell(2) <= ze : w.icell(2) >= zs))) {
-                    w.step([&](const auto* cell, auto k, auto mi) {
+                    w.step([&](const int* cell, int k, int mi) {
                         float val[8];
-                        const int ic[3] = {(int)cell[0], (int)cell[1], (int)cell[2]};
+                        const int ic[3] = {cell[0], cell[1], cell[2]};
                         chunk_corners(v, vol, chunk, staged, X0, Y0, Z0, CX, CY, CZ, ic, val);
                         f(val, cell, k, mi);
                     });
@@ -598,13 +562,12 @@ __device__ __forceinline__ void tube_walk_segments(const VolG& v, const T* __res
     }
 }
 
-// The gather walk (see tube_slabs); kFlat: the rays have no y component (td.dq[1] == 0); kRows:
-// the boxes staged by stage_box_rows.
-template <bool kFlat = false, bool kRows = false, typename T, class F>
+// The gather walk (see tube_slabs); kRows: the boxes staged by stage_box_rows.
+template <bool kRows = false, typename T, class F>
 __device__ __forceinline__ void tube_walk(const VolG& v, const T* __restrict__ vol, float* __restrict__ chunk,
                                           int* zr, const TubePlan& tp, const TubeBox& tb, const TubeDir& td,
                                           const float q0[3], int count, F&& f) {
-    tube_slabs<false, kFlat, kRows>(v, vol, nullptr, chunk, zr, tp, tb, td, q0, count, f);
+    tube_slabs<false, kRows>(v, vol, nullptr, chunk, zr, tp, tb, td, q0, count, f);
 }
 
 // The scatter walk (see tube_slabs): grad += the weights f returns.
@@ -612,7 +575,7 @@ template <class F>
 __device__ __forceinline__ void tube_scatter(const VolG& v, float* __restrict__ grad, float* __restrict__ chunk,
                                              int* zr, const TubePlan& tp, const TubeBox& tb, const TubeDir& td,
                                              const float q0[3], int count, F&& f) {
-    tube_slabs<true, false, false>(v, static_cast<const float*>(nullptr), grad, chunk, zr, tp, tb, td, q0, count, f);
+    tube_slabs<true, false>(v, static_cast<const float*>(nullptr), grad, chunk, zr, tp, tb, td, q0, count, f);
 }
 
 }  // namespace artia
