@@ -198,69 +198,46 @@ __device__ __forceinline__ FlatBox flat_box(const VolG& v, const TubePlan& tp, c
     q.CX = wave_uniform(q.X1 - q.X0 + 1);
     q.CY = wave_uniform(q.Y1 - q.Y0 + 1);
     q.CZ = q.Z1 - q.Z0 + 1;
-    const bool some = q.CX > 1 && q.CX <= 256 && q.CY > 1 && q.CZ > 1;   // (a thread keeps one column)
+    const bool some = q.CX > 1 && q.CX <= 256 && q.CY > 1 && q.CZ > 1;
     q.SY = some && q.CX * (q.CY | 1) * q.CZ <= kChunkFloats ? (q.CY | 1) : q.CY;
     q.staged = some && q.CX * q.SY * q.CZ <= kChunkFloats;
     return q;
 }
 
-// Stages the box: thread t keeps column t mod CX and takes every (256 / CX)-th (z, y) row, as
-// stage_box_rows does.
+// a / b for 0 <= a < 2^12 and 1 <= b <= 2^12: (a + 1/2) / b lies at least 1 / 2^13 from an integer, far more
+// than the rounding of one reciprocal.
+__device__ __forceinline__ int small_div(int a, int b) {
+    return (int)(((float)a + 0.5f) * __builtin_amdgcn_rcpf((float)b));
+}
+
+// Stages the box by columns along z: a thread keeps (x, y) columns t, t + 256, .. (one for most tilts) and
+// loads their layers, whose base addresses are uniform: a lane offset that stays fixed and one LDS
+// address step per voxel, with the clamps once per column (x, y) or in scalar registers (z).
 template <typename T>
 __device__ __forceinline__ void stage_flat_box(const VolG& v, const T* __restrict__ vol, float* __restrict__ chunk,
                                                const FlatBox& q) {
-    const int rows = q.CY * q.CZ, t = (int)threadIdx.x;
-    const int P = 256 / q.CX;   // rows per pass
-    const int r0 = t / q.CX, x = t - r0 * q.CX;
-    if (r0 >= P || r0 >= rows) return;
-    const int dz = P / q.CY, dy = P - dz * q.CY;
-    int zz = r0 / q.CY, yy = r0 - zz * q.CY;
-    const int plane = q.CX * q.SY;
-    float* __restrict__ o = chunk + (zz * plane + x * q.SY + yy);
-    const int oN = dz * plane + dy, oC = oN - q.CY + plane;   // LDS step of a row step, without and with a carry
-    if (q.X0 >= 0 && q.X1 < v.nx && q.Y0 >= 0 && q.Y1 < v.ny && q.Z0 >= 0 && q.Z1 < v.nz) {
-        const long long nx = v.nx, nxy = nx * (long long)v.ny;
-        const T* __restrict__ p = vol + ((long long)(q.Z0 + zz) * nxy + (long long)(q.Y0 + yy) * nx + (q.X0 + x));
-        const long long stepN = (long long)dy * nx + (long long)dz * nxy, stepC = stepN - (long long)q.CY * nx + nxy;
-        int r = r0;
-        for (; r + 3 * P < rows; r += 4 * P) {
-            float val[4];
-            int at[4];
+    const int cols = q.CX * q.CY, plane = q.CX * q.SY;
+    const size_t nxy = (size_t)v.nx * (size_t)v.ny;
+    for (int t = (int)threadIdx.x; t < cols; t += 256) {
+        const int y = small_div(t, q.CX), x = t - y * q.CX;
+        // (nx ny < 2^30: tube_plan)
+        const uint32_t off = ((uint32_t)clampi(q.Y0 + y, 0, v.ny - 1) * (uint32_t)v.nx +
+                              (uint32_t)clampi(q.X0 + x, 0, v.nx - 1)) * (uint32_t)sizeof(T);
+        float* __restrict__ o = chunk + (x * q.SY + y);
+        auto layer = [&](int z) {
+            const char* p = reinterpret_cast<const char*>(vol + (size_t)clampi(q.Z0 + z, 0, v.nz - 1) * nxy);
+            return vox(reinterpret_cast<const T*>(p + off), 0);
+        };
+        int z = 0;
+        for (; z + 4 < q.CZ; z += 5) {
+            float val[5];
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                val[k] = vox(p, 0);
-                yy += dy;
-                const bool c = yy >= q.CY;
-                yy = c ? yy - q.CY : yy;
-                p += c ? stepC : stepN;
-                at[k] = c ? oC : oN;
-            }
+            for (int k = 0; k < 5; k++) val[k] = layer(z + k);
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                *o = val[k];
-                o += at[k];
-            }
+            for (int k = 0; k < 5; k++) o[k * plane] = val[k];
+            o += 5 * plane;
         }
-        for (; r < rows; r += P) {
-            *o = vox(p, 0);
-            yy += dy;
-            const bool c = yy >= q.CY;
-            yy = c ? yy - q.CY : yy;
-            p += c ? stepC : stepN;
-            o += c ? oC : oN;
-        }
-        return;
-    }
-    const size_t gx = (size_t)clampi(q.X0 + x, 0, v.nx - 1);
-    for (int r = r0; r < rows; r += P) {
-        const int gy = clampi(q.Y0 + yy, 0, v.ny - 1), gz = clampi(q.Z0 + zz, 0, v.nz - 1);
-        *o = vox(vol, (size_t)(unsigned)(__mul24(gz, v.ny) + gy) * (size_t)(unsigned)v.nx + gx);
-        yy += dy;
-        zz += dz;
-        const bool c = yy >= q.CY;
-        yy = c ? yy - q.CY : yy;
-        zz += c ? 1 : 0;
-        o += c ? oC : oN;
+        for (; z < q.CZ; z++, o += plane) *o = layer(z);
     }
 }
 
@@ -297,7 +274,8 @@ __device__ __forceinline__ void flat_walk_slab(const VolG& v, const T* __restric
     const float b = q0[1] - floorf(q0[1]);
     const float rstop = (w.r[1] - (float)(zlast - zn)) - 0.5f;   // r_z below it: past the last layer
     // byte offsets: the far-far edge of the current cell, and its steps along the oriented axes
-    const int sx = 4 * d.sgn[0] * q.SY, sz = 4 * d.sgn[1] * q.CX * q.SY;
+    int sx = 4 * d.sgn[0] * q.SY, sz = 4 * d.sgn[1] * q.CX * q.SY;
+    __asm__("" : "+v"(sx), "+v"(sz));   // (selects of scalar operands would copy them every step)
     int o = 4 * (((d.sgn[1] * (zn + 1) - q.Z0) * q.CX + (d.sgn[0] * (xn + 1) - q.X0)) * q.SY + (yc - q.Y0));
     const char* __restrict__ base = reinterpret_cast<const char*>(chunk);
     auto edge = [&](int at, float& dy) {
@@ -560,12 +538,13 @@ __device__ __forceinline__ void flat_tube_scatter(const VolG& v, float* __restri
         if (w.active()) flat_scatter_slab(v, grad, chunk, q, d, q0, dq, rd, w, zs, ze);
         if (q.staged) {
             __syncthreads();   // the box is complete
-            // thread t takes column t mod CX of every (256 / CX)-th (z, y) row
-            const int P = 256 / q.CX, t = (int)threadIdx.x, r0 = t / q.CX, x = t - r0 * q.CX, rows = q.CY * q.CZ;
+            // by rows along x (coalesced atomics), thread t on column t mod CX
+            const int P = small_div(256, q.CX), t = (int)threadIdx.x, r0 = small_div(t, q.CX), x = t - r0 * q.CX;
+            const int rows = q.CY * q.CZ;
             if (r0 < P) {
                 const size_t gx = (size_t)clampi(q.X0 + x, 0, v.nx - 1);
                 for (int r = r0; r < rows; r += P) {
-                    const int zz = r / q.CY, yy = r - zz * q.CY;
+                    const int zz = small_div(r, q.CY), yy = r - zz * q.CY;
                     const float add = chunk[(zz * q.CX + x) * q.SY + yy];
                     const size_t row = (size_t)clampi(q.Z0 + zz, 0, v.nz - 1) * (size_t)v.ny +
                                        (size_t)clampi(q.Y0 + yy, 0, v.ny - 1);

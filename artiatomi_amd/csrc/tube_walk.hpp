@@ -41,6 +41,7 @@ inline bool tube_plan(const VolG& v, const TiltG& g, TubePlan& tp, double span =
     // (nz bounded so that the walk's float box offsets stay exact: |cell z * CXY| < 2^24, CXY being
     // at most kChunkFloats / 2)
     if (v.nx < 2 || v.ny < 2 || v.nz < 2 || (long long)(v.nz + 2) * (kChunkFloats / 2) >= (1LL << 24)) return false;
+    if ((long long)v.nx * v.ny >= (1LL << 30)) return false;   // 32-bit byte offsets within a layer
     double sc[3], N[3], dpx[3], dpy[3];
     for (int i = 0; i < 3; i++) {
         sc[i] = (double)v.rcp[i] * (double)v.dim[i];
