@@ -503,7 +503,7 @@ __global__ void __launch_bounds__(256, 6) march_lds_kernel(VolG v, TiltG g, cons
         float dq[3];
         tube_step(v, g, step, dq);
         const float K = flat_dir(dq).K;
-        flat_tube_walk<false>(v, vol, chunk, zr, tp, tb, dq, L.q0, L.count,
+        flat_tube_walk<false, true>(v, vol, chunk, zr, tp, tb, dq, L.q0, L.count,
                               [&](float A, float B, float C, float D, float, float, float, float, float a, float c,
                                   float m) { total += (double)flat_cell_sum(A, B, C, D, a, c, m, K); });
     } else {

@@ -146,7 +146,7 @@ __global__ void __launch_bounds__(256, 5) pair_march_kernel(PairArgs a) {
             };
             if (P.staged) {   // uniform: the whole block walks the tile's tube through LDS
                 const TubeBox tb = tube_box(v, g, P.tp, pi0 + 0.25, pi0 + 7.75, pj0 + 0.25, pj0 + 7.75, sx, sy);
-                flat_tube_walk<kMode != kProject>(v, a.vols + P.vol_offset, chunk, zr, P.tp, tb, dq, s.q0, s.count,
+                flat_tube_walk<kMode != kProject, kMode != kProject>(v, a.vols + P.vol_offset, chunk, zr, P.tp, tb, dq, s.q0, s.count,
                                                   flat_fn);
             } else if (ok) {
                 FlatWalker fw;
