@@ -30,6 +30,7 @@ SOURCES = [
     "rotate.hip",
     "sart.hip",
     "prep.hip",
+    "fft2d.hip",
 ]
 
 # -ffp-contract=off: the reference-numerics kernels keep the reference's float operation order;

@@ -40,6 +40,18 @@ struct FftBatch {
     artia_status ensure(artia_ctx* ctx, int n);
     void release();
 };
+
+// The three-kernel filters' state (fft2d.hpp): twiddles exp(-2 pi i k / N), cap + 1 half spectra, an N x N
+// image of crop weights and cap slab images that wait to be summed, rebuilt when N changes.
+struct FftOwn {
+    int N = 0, cap = 0;
+    float2* tw = nullptr;
+    float2* spec = nullptr;
+    float* weight = nullptr;
+    float* images = nullptr;
+    artia_status ensure(artia_ctx* ctx, int n);
+    void release();
+};
 }  // namespace artia
 
 struct artia_ctx {
@@ -61,6 +73,7 @@ struct artia_ctx {
     long long prof_launches[ARTIA_PROF_COUNT] = {};
     artia::FftPlans fft;
     artia::FftBatch fftb;
+    artia::FftOwn ffto;
 };
 
 namespace artia {
@@ -173,7 +186,8 @@ void launch_make_square(artia_ctx* ctx, int W, int H, size_t pitch, const float*
 float ctf_wavelength(float voltage_kV);
 artia_status run_ctf(artia_ctx* ctx, float2* spec, int N, size_t pitch, const artia_ctf_params& p, float dmin_nm,
                      float dmax_nm, float angle_deg, int forFP);
-artia_status run_wbp_weight(artia_ctx* ctx, float2* spec, int N, size_t pitch, float psi_deg, int method);
+// n spectra, stride N * pitch, each with its own angle
+artia_status run_wbp_weight(artia_ctx* ctx, float2* spec, int N, size_t pitch, const float* psi_deg, int n, int method);
 // cropBorder(img) -> makeSquare -> R2C -> ctf -> C2R -> out (+)= cropBorder(square / N^2)
 artia_status ctf_slab_filter(artia_ctx* ctx, float* img, int W, int H, size_t pitch, float* out, size_t out_pitch,
                              int accumulate, const int corners[8], const float cut[2], const float dim[2],

@@ -1,8 +1,9 @@
 // Projection preparation on gfx950: PrepareProjection (Reconstructor.cpp:1158-1383) over a stack of
 // projections.  The reference prepares one projection at a time with NPP statistics copied to the
-// host between steps; here a chunk of projections goes through every step together (batched hipFFT
-// plans, one launch per step and chunk), and the per-projection statistics stay on the device
-// until the end of the call.
+// host between steps; here a chunk of projections goes through every step together, and the per-projection
+// statistics stay on the device until the end of the call.  For squares of 128 .. 4096 (a power of two)
+// the steps between the raw pixels and the filtered image are the three filter kernels' own loads,
+// factors and stores (fft2d.hpp); other sizes take batched hipFFT plans with one launch per step.
 //
 // Steps per projection (see artia_prepare_projections in artia.h):
 //   convert + mirror square -> mean of the square -> bad pixels -> [WBP: crop, statistics,
@@ -10,27 +11,20 @@
 //   -> crop / n^2 -> [SART: statistics, normalise].
 // Sums are in double, in a fixed order (block partials, then one block per projection), so a
 // projection's statistics do not depend on the chunk it is in.
+#include <algorithm>
 #include <cmath>
 #include <vector>
 
 #include "artia_internal.hpp"
 #include "device_common.hpp"
+#include "fft2d.hpp"
 #include "image_ops.hpp"
+#include "spectral_factors.hpp"
 
 namespace artia {
 namespace {
 
 constexpr int kRedBlocks = 256;   // partial sums per image and reduction
-
-// Per-projection state, on the device for the whole call.
-struct PrepStat {
-    double sq_mean;          // mean of the converted square (the bad-pixel reference)
-    double mean, std;        // statistics of the normalisation region
-    float mean_hf, std_hf;   // the normalisation's subtrahend and divisor magnitude
-    float dose, cos_tilt;    // AccumulatedDose; cosf(|tilt| in radians) for DownWeightTiltsForWBP
-    int bad;                 // bad pixels replaced
-    int pad;
-};
 
 dim3 grid2(int w, int h, int z) { return dim3((unsigned)((w + 63) / 64), (unsigned)((h + 3) / 4), (unsigned)z); }
 
@@ -159,52 +153,91 @@ __global__ void __launch_bounds__(256) normalise_kernel(float* __restrict__ img,
     *p = v;
 }
 
-// fourierFilter (wbpWeighting.cu:146-212) and doseWeighting (:214-240), each a float factor applied
-// in the reference's order, on the half spectra of the chunk
-__global__ void __launch_bounds__(256) prep_spectrum_kernel(float2* __restrict__ spec, size_t pitch, int N, int band,
-                                                            float lp, float hp, float lps, float hps, int dose_on,
-                                                            float pixA, const PrepStat* __restrict__ st) {
+// The filters' factors (prep_factor) on the half spectra of the chunk
+__global__ void __launch_bounds__(256) prep_spectrum_kernel(float2* __restrict__ spec, size_t pitch, int N,
+                                                            PrepFilter f) {
     const int x = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     const int y = (int)(blockIdx.y * blockDim.y + threadIdx.y);
     if (x >= N / 2 + 1 || y >= N) return;
-    float mx = (float)x, my = (float)y;
-    if (my > N * 0.5f) my = (N - my) * -1.0f;
-    const float dist = sqrtf(mx * mx + my * my);
     float2* p = spec + (size_t)blockIdx.z * pitch * (size_t)N + (size_t)y * pitch + x;
-    float2 e = *p;
-    if (band) {
-        float fil = 0;
-        lp = lp - lps;
-        hp = hp + hps;
-        if (lp > 0) {
-            if (dist <= lp) fil = 1;
-        } else {
-            if (dist <= N / 2 - 1) fil = 1;
-        }
-        if (lps > 0) {
-            const float fil2 = (-fil + 1.0f) * expf(-((dist - lp) * (dist - lp) / (2 * lps * lps)));
-            if (fil2 > 0.001f) fil = fil2;
-        }
-        if (lps > 0 && lp == 0 && hp == 0 && hps == 0) fil = expf(-((dist - lp) * (dist - lp) / (2 * lps * lps)));
-        if (hp > 0) {
-            float fil2 = 0;
-            if (dist >= hp) fil2 = 1;
-            fil *= fil2;
-            if (hps > 0) {
-                const float fil3 = (-fil2 + 1) * expf(-((dist - hp) * (dist - hp) / (2 * hps * hps)));
-                if (fil3 > 0.001f) fil = fil3;
+    *p = prep_factor(*p, x, y, N, f, (int)blockIdx.z);
+}
+
+// The square's or the image's sums over raw pixels of type T, in the order of region_sums_kernel: pass 0
+// over the mirrored N x N square (its mean, the bad-pixel reference), pass 1 and 2 over the W x H image
+// with its bad pixels replaced (mean, squared deviations).
+template <class T>
+__global__ void __launch_bounds__(256) raw_sums_kernel(const T* __restrict__ in, size_t pitch, size_t istride, int W,
+                                                       int H, int N, int bx, int by, int mirror_y, int correct,
+                                                       float bad_value, const PrepStat* __restrict__ st, int pass,
+                                                       double* __restrict__ partial) {
+    __shared__ double sh[256];
+    const int z = (int)blockIdx.y, w = pass ? W : N, h = pass ? H : N;
+    const T* base = in + (size_t)z * istride;
+    const double m = pass == 2 ? st[z].mean : 0.0;
+    const float mean = pass && correct ? (float)st[z].sq_mean : 0.0f;
+    double acc = 0.0;
+    for (int r = (int)blockIdx.x; r < h; r += kRedBlocks) {
+        int x0 = 0, yi = r;
+        if (!pass) mirror_source(bx, r, W, H, bx, by, 0, x0, yi);
+        const T* row = base + (size_t)(mirror_y ? H - yi - 1 : yi) * pitch;
+        // eight loads in flight (one at a time read 0.5 TB/s)
+        for (int c = (int)threadIdx.x; c < w; c += 8 * 256) {
+            float f[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                int xi = min(c + 256 * j, w - 1), y2;
+                if (!pass) mirror_source(xi, by, W, H, bx, by, 0, xi, y2);
+                f[j] = (float)row[xi];
+            }
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                if (pass && correct && f[j] > bad_value * mean) f[j] = mean;
+                const double v = (double)f[j];
+                if (c + 256 * j < w) acc += pass == 2 ? (v - m) * (v - m) : v;
             }
         }
-        e.x *= fil;
-        e.y *= fil;
     }
-    if (dose_on) {
-        const float d = dist / (N / 2 / pixA);
-        const float fil = expf(-st[blockIdx.z].dose * d);
-        e.x *= fil;
-        e.y *= fil;
+    const double s = block_sum(acc, sh);
+    if (threadIdx.x == 0) partial[(size_t)z * kRedBlocks + blockIdx.x] = s;
+}
+
+// The statistics of a filtered image from its row blocks' sums of v - c and (v - c)^2
+__global__ void __launch_bounds__(256) row_stats_finish_kernel(const double* __restrict__ partial, int blocks, double count,
+                                                               const float* __restrict__ dc, float scale,
+                                                               PrepStat* __restrict__ st) {
+    __shared__ double sh[256];
+    const int z = (int)blockIdx.x;
+    double a1 = 0.0, a2 = 0.0;
+    for (int b = (int)threadIdx.x; b < blocks; b += 256) {
+        a1 += partial[2 * ((size_t)z * blocks + b)];
+        a2 += partial[2 * ((size_t)z * blocks + b) + 1];
     }
-    *p = e;
+    const double s1 = block_sum(a1, sh), s2 = block_sum(a2, sh);
+    if (threadIdx.x == 0) {
+        const double d = s1 / count, var = s2 / count - d * d;
+        st[z].mean = (double)(dc[z] * scale) + d;
+        st[z].std = sqrt(var < 0.0 ? 0.0 : var);
+    }
+}
+
+template <class T>
+void launch_raw_sums(artia_ctx* ctx, const RowSrc& s, int N, int pass, double* partial, int b) {
+    hipLaunchKernelGGL(raw_sums_kernel<T>, dim3(kRedBlocks, (unsigned)b), dim3(256), 0, ctx->stream,
+                       static_cast<const T*>(s.raw), s.pitch, s.stride, s.W, s.H, N, s.bx, s.by, s.mirror_y, s.correct,
+                       s.bad_value, s.st, pass, partial);
+}
+// pass 0 -> sq_mean, 1 -> mean, 2 -> std
+void raw_stat(artia_ctx* ctx, const RowSrc& s, int N, int pass, double* partial, int b) {
+    switch (s.dtype) {
+        case ARTIA_DT_SHORT: launch_raw_sums<short>(ctx, s, N, pass, partial, b); break;
+        case ARTIA_DT_USHORT: launch_raw_sums<unsigned short>(ctx, s, N, pass, partial, b); break;
+        case ARTIA_DT_INT: launch_raw_sums<int>(ctx, s, N, pass, partial, b); break;
+        case ARTIA_DT_UINT: launch_raw_sums<unsigned>(ctx, s, N, pass, partial, b); break;
+        default: launch_raw_sums<float>(ctx, s, N, pass, partial, b); break;
+    }
+    const double count = pass ? (double)s.W * (double)s.H : (double)N * (double)N;
+    hipLaunchKernelGGL(region_finish_kernel, dim3((unsigned)b), dim3(256), 0, ctx->stream, partial, count, pass, s.st);
 }
 
 template <class T>
@@ -266,15 +299,21 @@ artia_status artia_prepare_projections(artia_ctx* ctx, const artia_prep_params* 
                     "artia_prepare_projections: dose weighting needs doses and a pixel size");
     const int N = width > height ? width : height;
     const bool fft = !pp->skip_filter || pp->wbp;
+    // the three-kernel filter (fft2d.hpp), or library transforms of the chunk's squares
+    const bool own = fft && fft2d_supports(N) && fft2d_fits(height, pitch) && fft2d_fits(height, out_pitch) &&
+                     ctx->numerics == ARTIA_NUMERICS_EXACT;
     FftBatch& fb = ctx->fftb;
-    artia_status st = fb.ensure(ctx, N);
+    FftOwn& fo = ctx->ffto;
+    artia_status st = own ? fo.ensure(ctx, N) : fb.ensure(ctx, N);
     if (st != ARTIA_OK) return st;
-    // workspace: partial sums of a chunk, then the per-projection state
-    const size_t partFloats = (size_t)fb.cap * kRedBlocks * 2;
+    const int cap = own ? fo.cap : fb.cap, rowBlocks = own ? fft2d_row_blocks(N) : 0;
+    // workspace: partial sums of a chunk, then the per-projection state and, behind it, the squares' means
+    const size_t partFloats = (size_t)cap * (size_t)std::max(kRedBlocks, 2 * rowBlocks) * 2;
     const size_t statFloats = ((size_t)n * sizeof(PrepStat) + sizeof(float) - 1) / sizeof(float);
-    if ((st = ensure_workspace(ctx, partFloats + statFloats + 2)) != ARTIA_OK) return st;
+    if ((st = ensure_workspace(ctx, partFloats + statFloats + 2 + kFftBatchMax)) != ARTIA_OK) return st;
     double* partial = reinterpret_cast<double*>(ctx->ws);
     PrepStat* d_stat = reinterpret_cast<PrepStat*>(ctx->ws + partFloats);
+    float* d_dc = ctx->ws + partFloats + statFloats + 2;
     std::vector<PrepStat> hs((size_t)n);
     for (int i = 0; i < n; i++) {
         PrepStat& s = hs[(size_t)i];
@@ -294,14 +333,90 @@ artia_status artia_prepare_projections(artia_ctx* ctx, const artia_prep_params* 
     const size_t istride = (size_t)height * pitch, ostride = (size_t)height * out_pitch;
     const int bx = (N - width) / 2, by = (N - height) / 2;
     const float pixA = pp->pixelsize_nm * 10.0f;
+    const bool centre = !pp->wbp && pp->normalization == ARTIA_NORM_NONE;
+    const int rx0 = centre ? width / 4 : 0, ry0 = centre ? height / 4 : 0;
+    const int rw = centre ? width / 2 : width, rh = centre ? height / 2 : height;
     for (int k0 = 0; k0 < n;) {
-        int b = fb.cap, pi = 0;
+        int b = cap, pi = 0;
+        if (own) b = std::min(b, n - k0);
         while (b > n - k0) b /= 2;
         for (int q = b; q > 1; q /= 2) pi++;
         PrepStat* s = d_stat + k0;
         float* o = out + (size_t)k0 * ostride;
-        square_of(ctx, pp->dtype, static_cast<const char*>(images) + (size_t)k0 * istride * dtype_size(pp->dtype),
-                  pitch, istride, width, height, N, pp->mirror_y, fb.square, b);
+        const void* raw = static_cast<const char*>(images) + (size_t)k0 * istride * dtype_size(pp->dtype);
+        PrepFilter f{};
+        f.band = pp->skip_filter ? 0 : 1;
+        f.lp = pp->lp;
+        f.hp = pp->hp;
+        f.lps = pp->lps;
+        f.hps = pp->hps;
+        f.dose_on = pp->dose_weighting;
+        f.pixA = pixA;
+        f.st = s;
+        if (own) {
+            RowSrc r{};
+            r.W = width;
+            r.H = height;
+            r.bx = bx;
+            r.by = by;
+            r.raw = raw;
+            r.pitch = pitch;
+            r.stride = istride;
+            r.dtype = pp->dtype;
+            r.mirror_y = pp->mirror_y;
+            r.correct = pp->correct_bad_pixels;
+            r.bad_value = pp->bad_pixel_value;
+            r.st = s;
+            if (r.correct) raw_stat(ctx, r, N, 0, partial, b);
+            if (pp->wbp) {
+                // the raw image's statistics; its pixels are normalised as they are loaded
+                raw_stat(ctx, r, N, 1, partial, b);
+                raw_stat(ctx, r, N, 2, partial, b);
+                hipLaunchKernelGGL(norm_params_kernel, dim3((unsigned)((b + 63) / 64)), dim3(64), 0, ctx->stream, s, b, 1,
+                                   pp->normalization, pp->down_weight_tilts);
+                r.norm = 1;
+                f.wbp = 1;
+                f.method = pp->wbp_method;
+                for (int i = 0; i < b; i++) {
+                    const float ang = -psi_deg[k0 + i] / 180.0f * 3.14159265358979323846f;
+                    f.sn[i] = sin((double)ang);
+                    f.cs[i] = cos((double)ang);
+                }
+            }
+            f.dc = d_dc;
+            fft2d_rows_prep(ctx, N, fo.tw, r, fo.spec, b);
+            fft2d_cols_prep(ctx, N, fo.tw, fo.spec, f, b);
+            RowDst d{};
+            d.W = width;
+            d.H = height;
+            d.bx = bx;
+            d.by = by;
+            d.scale = 1.0f / ((float)N * (float)N);
+            d.out = o;
+            d.pitch = out_pitch;
+            d.stride = ostride;
+            if (pp->wbp) {
+                fft2d_rows_store(ctx, N, fo.tw, fo.spec, d, b);
+            } else {
+                d.rx0 = rx0;
+                d.ry0 = ry0;
+                d.rw = rw;
+                d.rh = rh;
+                d.dc = d_dc;
+                d.partial = partial;
+                fft2d_rows_prep_store(ctx, N, fo.tw, fo.spec, d, b);
+                hipLaunchKernelGGL(row_stats_finish_kernel, dim3((unsigned)b), dim3(256), 0, ctx->stream, partial,
+                                   rowBlocks, (double)rw * (double)rh, d_dc, d.scale, s);
+                hipLaunchKernelGGL(norm_params_kernel, dim3((unsigned)((b + 63) / 64)), dim3(64), 0, ctx->stream, s, b, 0,
+                                   pp->normalization, 0);
+                hipLaunchKernelGGL(normalise_kernel, grid2(width, height, b), dim3(64, 4), 0, ctx->stream, o, width,
+                                   height, out_pitch, ostride, s);
+            }
+            if ((st = check_hip(ctx, hipGetLastError(), "projection preparation launch")) != ARTIA_OK) return st;
+            k0 += b;
+            continue;
+        }
+        square_of(ctx, pp->dtype, raw, pitch, istride, width, height, N, pp->mirror_y, fb.square, b);
         region_stat(ctx, fb.square, plane, (size_t)N, 0, 0, N, N, s, 0, partial, b);
         if (pp->correct_bad_pixels)
             hipLaunchKernelGGL(bad_pixel_kernel, dim3(512, (unsigned)b), dim3(256), 0, ctx->stream, fb.square, N,
@@ -324,15 +439,12 @@ artia_status artia_prepare_projections(artia_ctx* ctx, const artia_prep_params* 
                 return fail(ctx, ARTIA_ERR_FFT, "hipfftSetStream failed");
             if (hipfftExecR2C(fb.r2c[pi], fb.square, (hipfftComplex*)fb.spec) != HIPFFT_SUCCESS)
                 return fail(ctx, ARTIA_ERR_FFT, "hipfftExecR2C (batch %d) failed", b);
-            if (!pp->skip_filter || pp->dose_weighting)
+            if (f.band || f.dose_on)
                 hipLaunchKernelGGL(prep_spectrum_kernel, grid2(N / 2 + 1, N, b), dim3(64, 4), 0, ctx->stream, fb.spec,
-                                   half, N, pp->skip_filter ? 0 : 1, pp->lp, pp->hp, pp->lps, pp->hps,
-                                   pp->dose_weighting, pixA, s);
-            if (pp->wbp)
-                for (int i = 0; i < b; i++)
-                    if ((st = run_wbp_weight(ctx, fb.spec + (size_t)i * half * N, N, half, psi_deg[k0 + i],
-                                             pp->wbp_method)) != ARTIA_OK)
-                        return st;
+                                   half, N, f);
+            if (pp->wbp &&
+                (st = run_wbp_weight(ctx, fb.spec, N, half, psi_deg + k0, b, pp->wbp_method)) != ARTIA_OK)
+                return st;
             if (hipfftExecC2R(fb.c2r[pi], (hipfftComplex*)fb.spec, fb.square) != HIPFFT_SUCCESS)
                 return fail(ctx, ARTIA_ERR_FFT, "hipfftExecC2R (batch %d) failed", b);
         }
@@ -340,11 +452,8 @@ artia_status artia_prepare_projections(artia_ctx* ctx, const artia_prep_params* 
                            width, height, fft ? (float)N * (float)N : 1.0f, o, out_pitch, ostride);
         if (!pp->wbp) {
             // SART: statistics of the filtered image (its centre for IMOD-aligned stacks), normalised
-            const bool centre = pp->normalization == ARTIA_NORM_NONE;
-            const int x0 = centre ? width / 4 : 0, y0 = centre ? height / 4 : 0;
-            const int w = centre ? width / 2 : width, h = centre ? height / 2 : height;
-            region_stat(ctx, o, ostride, out_pitch, x0, y0, w, h, s, 1, partial, b);
-            region_stat(ctx, o, ostride, out_pitch, x0, y0, w, h, s, 2, partial, b);
+            region_stat(ctx, o, ostride, out_pitch, rx0, ry0, rw, rh, s, 1, partial, b);
+            region_stat(ctx, o, ostride, out_pitch, rx0, ry0, rw, rh, s, 2, partial, b);
             hipLaunchKernelGGL(norm_params_kernel, dim3((unsigned)((b + 63) / 64)), dim3(64), 0, ctx->stream, s, b, 0,
                                pp->normalization, 0);
             hipLaunchKernelGGL(normalise_kernel, grid2(width, height, b), dim3(64, 4), 0, ctx->stream, o, width, height,

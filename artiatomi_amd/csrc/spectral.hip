@@ -4,30 +4,21 @@
 //   slab filter : cropBorder (in place) -> makeSquare (zero fill) -> R2C -> ctf -> C2R ->
 //                 / N^2 with crop to W x H -> cropBorder -> store or accumulate
 //   WBP filter  : makeSquare (reflect) -> R2C -> wbpWeighting -> C2R -> / N^2 with crop
-// The FFTs are hipFFT single-precision plans cached per size in the context; the spectrum is the
+// For N = 128 .. 4096 a power of two and exact numerics the filters run in three kernels (fft2d.hpp);
+// otherwise the FFTs are hipFFT single-precision plans cached per size in the context, on the
 // (N/2+1) x N half spectrum, rows of N/2+1 complex values.
 #include <algorithm>
 #include <cmath>
 
 #include "device_common.hpp"
+#include "fft2d.hpp"
 #include "image_ops.hpp"
+#include "spectral_factors.hpp"
 
 namespace artia {
 namespace {
 
 constexpr float kPiF = 3.14159265358979323846f;
-
-struct CtfK {
-    float cs_m;         // Cs * 0.001 (mm -> m)
-    float lambda;       // electron wavelength (m), the reference's float constants
-    float freq_step;    // (1 / (2 * pixelsize)) / (N / 2)
-    float pc, ac;       // phase and amplitude contrast
-    float halfN;        // c_pixelcount * 0.5
-    float def0, def1, angle;   // metres, metres, radians
-    float wiener;
-    float beta[4];
-    int forFP, phaseFlip, N;
-};
 
 // Reference numerics: the kernel body's float operation order.
 __global__ void __launch_bounds__(256) ctf_ref_kernel(float2* __restrict__ spec, size_t pitch, CtfK k) {
@@ -70,70 +61,7 @@ __global__ void __launch_bounds__(256) ctf_ref_kernel(float2* __restrict__ spec,
     spec[(size_t)y * pitch + x] = r;
 }
 
-// Exact numerics: the CTF factor in double (the phase reaches hundreds of radians at Nyquist, where
-// a float phase carries ~1e-5 absolute error), applied to the float spectrum.
-// The exact CTF factor of one spectrum point in two parts: what does not depend on the defocus
-// (ctf_point), and the factor and its application for one defocus pair (ctf_apply_at); together the
-// double arithmetic of the kernel body, in its order.
-struct CtfPoint {
-    double c2b;      // cos(2 beta)
-    double len;      // spatial frequency
-    double lam4;     // Cs lam^3 len^4, the defocus-free term of the phase
-    double env;      // the envelope, clamped as the direction requires (used when damped)
-    bool damped;     // outside the untouched low-frequency disk, and not phase flipping
-};
-
-__device__ __forceinline__ CtfPoint ctf_point(int x, int y, const CtfK& k) {
-    CtfPoint p;
-    double xpos = (double)x, ypos = (double)y;
-    if (ypos > (double)k.N * 0.5) ypos = ((double)k.N - ypos) * -1.0;
-    const double alpha = (xpos == 0) ? (double)(kPiF * 0.5f) : atan2(ypos, xpos);
-    const double beta = alpha - (double)k.angle;
-    p.c2b = cos(2 * beta);
-    double len = sqrt(xpos * xpos + ypos * ypos);
-    len *= (double)k.freq_step;
-    p.len = len;
-    const double lam = k.lambda, Cs = k.cs_m;
-    p.lam4 = Cs * lam * lam * lam * len * len * len * len;
-    const double radius = sqrt(xpos * xpos + ypos * ypos);
-    p.damped = !k.phaseFlip && radius > (double)k.beta[0];
-    p.env = 0.0;
-    if (p.damped) {
-        const double l = len / 100000000.0;
-        const double e = exp((-(double)k.beta[1] * l - (double)k.beta[2] * l * l) - (double)k.beta[3] * l * l * l);
-        p.env = k.forFP ? fmax(e, (double)0.01f) : fmax(e, (double)k.wiener);
-    }
-    return p;
-}
-
-__device__ __forceinline__ float2 ctf_apply_at(float2 r, const CtfPoint& p, const CtfK& k, float def0f, float def1f) {
-    const double def0 = def0f, def1 = def1f;
-    const double defocus = def0 + (1 - p.c2b) * (def1 - def0);
-    const double lam = k.lambda, len = p.len;
-    const double m = (double)(kPiF / 2.0f) * (p.lam4 - 2 * defocus * lam * len * len);
-    // sin and cos from one argument reduction (the same values as the two calls)
-    double sm, cm;
-    sincos(m, &sm, &cm);
-    const double n = (double)k.pc * sm + (double)k.ac * cm;
-    double f = 1.0;
-    if (p.damped) {
-        if (k.forFP) {
-            double val = n * p.env;
-            if (fabs(val) < (double)0.0001f && val >= 0) val = (double)0.0001f;
-            if (fabs(val) < (double)0.0001f && val < 0) val = -(double)0.0001f;
-            f = -val;
-        } else {
-            const double W = k.wiener;
-            const double val = n * p.env;
-            f = -val / (val * val + W);
-        }
-    }
-    if (k.phaseFlip && n >= 0) f = -f;
-    r.x = (float)((double)r.x * f);
-    r.y = (float)((double)r.y * f);
-    return r;
-}
-
+// Exact numerics: the CTF factor in double (spectral_factors.hpp), applied to the float spectrum.
 __device__ __forceinline__ void ctf_exact_at(float2* __restrict__ spec, size_t pitch, int x, int y, const CtfK& k) {
     const CtfPoint p = ctf_point(x, y, k);
     float2* q = spec + (size_t)y * pitch + x;
@@ -147,12 +75,7 @@ __global__ void __launch_bounds__(256) ctf_exact_kernel(float2* __restrict__ spe
     ctf_exact_at(spec, pitch, x, y, k);
 }
 
-// The same over a stack of half spectra (stride N * (N/2+1)), slab blockIdx.z with its own defocus.
-struct CtfStack {
-    CtfK k;
-    float def0[kFftBatchMax], def1[kFftBatchMax];
-};
-
+// The same over a stack of half spectra (stride N * (N/2+1)), each slab with its own defocus.
 __global__ void __launch_bounds__(256) ctf_exact_stack_kernel(float2* __restrict__ spec, size_t pitch, CtfStack b,
                                                               int ns) {
     const int x = (int)(blockIdx.x * blockDim.x + threadIdx.x);
@@ -185,43 +108,27 @@ __global__ void __launch_bounds__(256) ctf_exact_fan_kernel(const float2* __rest
     }
 }
 
-// wbpWeighting.cu:48-144 (sin/cos of the angle as IEEE functions rather than __sinf/__cosf)
-__global__ void __launch_bounds__(256) wbp_weight_kernel(float2* __restrict__ spec, size_t pitch, int N, float ang,
+// wbpWeighting.cu:48-144 over a stack of spectra (sin/cos of the angles as IEEE functions rather than
+// __sinf/__cosf)
+struct WbpStack {
+    float ang[kFftBatchMax];
+    double sn[kFftBatchMax], cs[kFftBatchMax];
+};
+
+__global__ void __launch_bounds__(256) wbp_weight_kernel(float2* __restrict__ spec, size_t pitch, int N, WbpStack a,
                                                          int method, int exact) {
     const int x = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     const int y = (int)(blockIdx.y * blockDim.y + threadIdx.y);
     if (x >= N / 2 + 1 || y >= N) return;
-    const unsigned pc = (unsigned)N;
-    float w = 1.0f;
+    spec += (size_t)blockIdx.z * pitch * (size_t)N;
     if (exact) {
-        double xpos = (double)x, ypos = (double)y;
-        if (ypos > (double)pc * 0.5) ypos = ((double)pc - ypos) * -1.0;
-        const double sn = sin((double)ang), cs = cos((double)ang);
-        const double yr = sn * xpos + cs * ypos;
-        const double len = yr / (double)pc / 2.0;
-        double wd = 1.0;
-        if (method == 0) {
-            wd = fmin(fabs(len), 1.0);
-        } else if (method >= 2 && method <= 4) {
-            const double P[3][4] = {{1.000654227857550f, 0.006008581017124f, 0.004159659493151f, 0.000975903396538f},
-                                    {1.003784816598589f, 0.029016377161629f, 0.019582940715148f, 0.004559409669984f},
-                                    {0.999884616010943f, 0.000307646262566f, 0.004742915272196f, 0.004806551368900f}};
-            const double* q = P[method - 2];
-            if (len == 0) {
-                wd = 0;
-            } else {
-                const double L = log(fabs(len));
-                wd = ((q[0] + q[1] * L) + q[2] * L * L) + q[3] * L * L * L;
-            }
-            wd = fmax(0.0, fmin(wd, 1.0));
-        }
-        w = (float)wd;
-        float2 r = spec[(size_t)y * pitch + x];
-        r.x = (float)((double)r.x * wd);
-        r.y = (float)((double)r.y * wd);
-        spec[(size_t)y * pitch + x] = r;
+        spec[(size_t)y * pitch + x] =
+            wbp_weighted(spec[(size_t)y * pitch + x], x, y, N, a.sn[blockIdx.z], a.cs[blockIdx.z], method);
         return;
     }
+    const unsigned pc = (unsigned)N;
+    const float ang = a.ang[blockIdx.z];
+    float w = 1.0f;
     float xpos = (float)x, ypos = (float)y;
     if (ypos > (float)pc * 0.5f) ypos = ((float)pc - ypos) * -1.0f;
     const float temp = xpos;
@@ -345,7 +252,128 @@ CtfK make_ctf(int N, const artia_ctf_params& p, float dmin_nm, float dmax_nm, fl
     k.forFP = forFP;
     k.phaseFlip = p.phase_flip_only;
     k.N = N;
+    k.cos2a = cos(2.0 * (double)k.angle);
+    k.sin2a = sin(2.0 * (double)k.angle);
     return k;
+}
+
+// Defocus pairs of slabs 0 .. b - 1.
+CtfStack make_ctf_stack(int N, const artia_ctf_params& p, const float* dmin_nm, const float* dmax_nm, float angle_deg,
+                        int forFP, int b) {
+    CtfStack cs{};
+    cs.k = make_ctf(N, p, dmin_nm[0], dmax_nm[0], angle_deg, forFP);
+    for (int s = 0; s < b; s++) {
+        const CtfK ks = make_ctf(N, p, dmin_nm[s], dmax_nm[s], angle_deg, forFP);
+        cs.def0[s] = ks.def0;
+        cs.def1[s] = ks.def1;
+    }
+    return cs;
+}
+
+// cropBorder's weights at the places of the image in its square, 0 around them
+__global__ void __launch_bounds__(256) square_weight_kernel(float* __restrict__ out, int N, int W, int H, int bx, int by,
+                                                            CropParams cp) {
+    const int x = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    const int y = (int)(blockIdx.y * blockDim.y + threadIdx.y);
+    if (x >= N || y >= N) return;
+    const int xi = x - bx, yi = y - by;
+    out[(size_t)y * N + x] = xi >= 0 && xi < W && yi >= 0 && yi < H ? crop_weight(xi, yi, W, H, cp) : 0.0f;
+}
+
+// out += img_s for s = 0 .. ns - 1 in turn, rounded after every image
+__global__ void __launch_bounds__(256) sum_images_kernel(const float* __restrict__ img, size_t stride, int ns, int W, int H,
+                                                         float* __restrict__ out, size_t pitch) {
+    const int x = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    const int y = (int)(blockIdx.y * blockDim.y + threadIdx.y);
+    if (x >= W || y >= H) return;
+    const float* p = img + ((size_t)y * W + x);
+    float* o = out + ((size_t)y * pitch + x);
+    float acc = *o;
+    for (int s0 = 0; s0 < ns; s0 += 8) {
+        float v[8];
+#pragma unroll
+        for (int s = 0; s < 8; s++) v[s] = p[(size_t)min(s0 + s, ns - 1) * stride];
+#pragma unroll
+        for (int s = 0; s < 8; s++)
+            if (s0 + s < ns) acc = acc + v[s];
+    }
+    *o = acc;
+}
+
+RowSrc square_source(const float* src, size_t stride, int W, int H, size_t pitch, int N) {
+    RowSrc s{};
+    s.W = W;
+    s.H = H;
+    s.bx = (N - W) / 2;
+    s.by = (N - H) / 2;
+    s.src = src;
+    s.pitch = pitch;
+    s.stride = stride;
+    return s;
+}
+RowDst square_target(float* out, size_t stride, int W, int H, size_t pitch, int N, const float* weight, int accumulate) {
+    RowDst d{};
+    d.W = W;
+    d.H = H;
+    d.bx = (N - W) / 2;
+    d.by = (N - H) / 2;
+    d.scale = 1.0f / ((float)N * (float)N);
+    d.out = out;
+    d.pitch = pitch;
+    d.stride = stride;
+    d.weight = weight;
+    d.accumulate = accumulate;
+    return d;
+}
+
+// ctf_filter_slabs over the three-kernel filter (fft2d.hpp)
+artia_status ctf_filter_slabs_own(artia_ctx* ctx, const float* src, size_t src_stride, int n, int W, int H, size_t pitch,
+                                  float* out, size_t out_stride, const int corners[8], const float cut[2],
+                                  const float dim[2], const artia_ctf_params& p, const float* dmin_nm,
+                                  const float* dmax_nm, float angle_deg, int forFP) {
+    const int N = W > H ? W : H;
+    FftOwn& f = ctx->ffto;
+    artia_status st = f.ensure(ctx, N);
+    if (st != ARTIA_OK) return st;
+    const float* weight = nullptr;
+    if (corners) {
+        weight = f.weight;
+        hipLaunchKernelGGL(square_weight_kernel, grid2d(N, N), dim3(64, 4), 0, ctx->stream, f.weight, N, W, H, (N - W) / 2,
+                           (N - H) / 2, make_crop_params(cut, dim, corners));
+    }
+    // every slab filtering the same uncropped image (the sub-volume WBP): one forward transform, kept in
+    // the spare slot, serves all slabs
+    const bool shared = src_stride == 0 && !corners;
+    float2* base = f.spec + (size_t)f.cap * fft2d_spec_size(N);
+    RowSrc s = square_source(src, src_stride, W, H, pitch, N);
+    if (shared) {
+        fft2d_rows_square(ctx, N, f.tw, s, base, 1);
+        fft2d_cols_forward(ctx, N, f.tw, base, 1);
+    }
+    for (int k0 = 0; k0 < n; k0 += f.cap) {
+        const int b = std::min(f.cap, n - k0);
+        const CtfStack cs = make_ctf_stack(N, p, dmin_nm + k0, dmax_nm + k0, angle_deg, forFP, b);
+        if (shared) {
+            fft2d_cols_fan(ctx, N, f.tw, base, f.spec, cs, b);
+        } else {
+            s.src = src + (size_t)k0 * src_stride;
+            s.weight = weight;
+            s.rep0 = !corners ? 0 : (forFP ? 1 : k0 + 1);
+            s.rep_step = corners && !forFP ? 1 : 0;
+            fft2d_rows_square(ctx, N, f.tw, s, f.spec, b);
+            fft2d_cols_ctf(ctx, N, f.tw, f.spec, cs, b);
+        }
+        if (forFP) {
+            const size_t plane = (size_t)W * (size_t)H;
+            fft2d_rows_store(ctx, N, f.tw, f.spec, square_target(f.images, plane, W, H, (size_t)W, N, weight, 0), b);
+            hipLaunchKernelGGL(sum_images_kernel, grid2d(W, H), dim3(64, 4), 0, ctx->stream, f.images, plane, b, W, H, out,
+                               pitch);
+        } else
+            fft2d_rows_store(ctx, N, f.tw, f.spec,
+                             square_target(out + (size_t)k0 * out_stride, out_stride, W, H, pitch, N, weight, 0), b);
+        if ((st = check_hip(ctx, hipGetLastError(), "stacked slab filter")) != ARTIA_OK) return st;
+    }
+    return ARTIA_OK;
 }
 
 }  // namespace
@@ -449,6 +477,46 @@ void FftBatch::release() {
     N = cap = 0;
 }
 
+artia_status FftOwn::ensure(artia_ctx* ctx, int n) {
+    if (N == n && cap > 0) return ARTIA_OK;
+    release();
+    // up to eight spectra of 4096 (540 MB) at a time: a 4096 x 4096 image takes 95.5 us of column and row kernels
+    // alone, 86 us in pairs or fours and 81.5 us among eight (fewer nearly empty last waves of blocks)
+    const size_t one = fft2d_spec_size(n) * sizeof(float2);
+    const int c = (int)std::min<size_t>((size_t)kFftBatchMax, std::max<size_t>(1, ((size_t)544 << 20) / one));
+    std::vector<float2> t((size_t)n);
+    for (int k = 0; k < n; k++) {
+        const double a = -2.0 * 3.14159265358979323846 * (double)k / (double)n;
+        t[(size_t)k] = make_float2((float)std::cos(a), (float)std::sin(a));
+    }
+    artia_status st = check_hip(ctx, hipMalloc(&tw, (size_t)n * sizeof(float2)), "hipMalloc(twiddles)");
+    if (st == ARTIA_OK)
+        st = check_hip(ctx, hipMemcpy(tw, t.data(), (size_t)n * sizeof(float2), hipMemcpyHostToDevice),
+                       "hipMemcpy(twiddles)");
+    if (st == ARTIA_OK) st = check_hip(ctx, hipMalloc(&spec, (size_t)(c + 1) * one), "hipMalloc(spectra)");
+    if (st == ARTIA_OK)
+        st = check_hip(ctx, hipMalloc(&weight, (size_t)n * n * sizeof(float)), "hipMalloc(crop weights)");
+    if (st == ARTIA_OK)
+        st = check_hip(ctx, hipMalloc(&images, (size_t)c * n * n * sizeof(float)), "hipMalloc(slab images)");
+    if (st != ARTIA_OK) {
+        release();
+        return st;
+    }
+    N = n;
+    cap = c;
+    return ARTIA_OK;
+}
+
+void FftOwn::release() {
+    if (tw) (void)hipFree(tw);
+    if (spec) (void)hipFree(spec);
+    if (weight) (void)hipFree(weight);
+    if (images) (void)hipFree(images);
+    tw = spec = nullptr;
+    weight = images = nullptr;
+    N = cap = 0;
+}
+
 artia_status run_ctf(artia_ctx* ctx, float2* spec, int N, size_t pitch, const artia_ctf_params& p, float dmin_nm,
                      float dmax_nm, float angle_deg, int forFP) {
     const CtfK k = make_ctf(N, p, dmin_nm, dmax_nm, angle_deg, forFP);
@@ -459,10 +527,20 @@ artia_status run_ctf(artia_ctx* ctx, float2* spec, int N, size_t pitch, const ar
     return check_hip(ctx, hipGetLastError(), "ctf launch");
 }
 
-artia_status run_wbp_weight(artia_ctx* ctx, float2* spec, int N, size_t pitch, float psi_deg, int method) {
-    const float ang = -psi_deg / 180.0f * kPiF;
-    hipLaunchKernelGGL(wbp_weight_kernel, grid2d(N / 2 + 1, N), dim3(64, 4), 0, ctx->stream, spec, pitch, N, ang,
-                       method, ctx->numerics == ARTIA_NUMERICS_EXACT ? 1 : 0);
+artia_status run_wbp_weight(artia_ctx* ctx, float2* spec, int N, size_t pitch, const float* psi_deg, int n, int method) {
+    for (int k0 = 0; k0 < n; k0 += kFftBatchMax) {
+        const int b = std::min(kFftBatchMax, n - k0);
+        WbpStack a{};
+        for (int i = 0; i < b; i++) {
+            a.ang[i] = -psi_deg[k0 + i] / 180.0f * kPiF;
+            a.sn[i] = sin((double)a.ang[i]);
+            a.cs[i] = cos((double)a.ang[i]);
+        }
+        dim3 g = grid2d(N / 2 + 1, N);
+        g.z = (unsigned)b;
+        hipLaunchKernelGGL(wbp_weight_kernel, g, dim3(64, 4), 0, ctx->stream, spec + (size_t)k0 * pitch * (size_t)N, pitch,
+                           N, a, method, ctx->numerics == ARTIA_NUMERICS_EXACT ? 1 : 0);
+    }
     return check_hip(ctx, hipGetLastError(), "wbpWeighting launch");
 }
 
@@ -470,6 +548,21 @@ artia_status ctf_slab_filter(artia_ctx* ctx, float* img, int W, int H, size_t pi
                              int accumulate, const int corners[8], const float cut[2], const float dim[2],
                              const artia_ctf_params& p, float dmin_nm, float dmax_nm, float angle_deg, int forFP) {
     const int N = W > H ? W : H;
+    if (fft2d_supports(N) && fft2d_fits(H, pitch) && fft2d_fits(H, out_pitch) && ctx->numerics == ARTIA_NUMERICS_EXACT) {
+        FftOwn& f = ctx->ffto;
+        const artia_status so = f.ensure(ctx, N);
+        if (so != ARTIA_OK) return so;
+        if (corners) {
+            launch_crop_border(ctx, W, H, pitch, img, cut, dim, corners);
+            hipLaunchKernelGGL(square_weight_kernel, grid2d(N, N), dim3(64, 4), 0, ctx->stream, f.weight, N, W, H,
+                               (N - W) / 2, (N - H) / 2, make_crop_params(cut, dim, corners));
+        }
+        fft2d_rows_square(ctx, N, f.tw, square_source(img, 0, W, H, pitch, N), f.spec, 1);
+        fft2d_cols_ctf(ctx, N, f.tw, f.spec, make_ctf_stack(N, p, &dmin_nm, &dmax_nm, angle_deg, forFP, 1), 1);
+        fft2d_rows_store(ctx, N, f.tw, f.spec,
+                         square_target(out, 0, W, H, out_pitch, N, corners ? f.weight : nullptr, accumulate), 1);
+        return check_hip(ctx, hipGetLastError(), "slab filter");
+    }
     artia_status st = ctx->fft.ensure(ctx, N);
     if (st != ARTIA_OK) return st;
     if (corners) launch_crop_border(ctx, W, H, pitch, img, cut, dim, corners);
@@ -495,6 +588,9 @@ artia_status ctf_filter_slabs(artia_ctx* ctx, const float* src, size_t src_strid
                               const float* dmax_nm, float angle_deg, int forFP) {
     if (n <= 0) return ARTIA_OK;
     const int N = W > H ? W : H;
+    if (fft2d_supports(N) && fft2d_fits(H, pitch))
+        return ctf_filter_slabs_own(ctx, src, src_stride, n, W, H, pitch, out, out_stride, corners, cut, dim, p, dmin_nm,
+                                    dmax_nm, angle_deg, forFP);
     FftBatch& fb = ctx->fftb;
     artia_status st = fb.ensure(ctx, N);
     if (st != ARTIA_OK) return st;
@@ -533,13 +629,7 @@ artia_status ctf_filter_slabs(artia_ctx* ctx, const float* src, size_t src_strid
             if (hipfftExecR2C(fb.r2c[pi], fb.square, (hipfftComplex*)fb.spec) != HIPFFT_SUCCESS)
                 return fail(ctx, ARTIA_ERR_FFT, "hipfftExecR2C (batch %d) failed", b);
         }
-        CtfStack cs;
-        cs.k = make_ctf(N, p, dmin_nm[k0], dmax_nm[k0], angle_deg, forFP);
-        for (int s = 0; s < b; s++) {
-            const CtfK ks = make_ctf(N, p, dmin_nm[k0 + s], dmax_nm[k0 + s], angle_deg, forFP);
-            cs.def0[s] = ks.def0;
-            cs.def1[s] = ks.def1;
-        }
+        const CtfStack cs = make_ctf_stack(N, p, dmin_nm + k0, dmax_nm + k0, angle_deg, forFP, b);
         const dim3 sgrid((unsigned)((N / 2 + 1 + 63) / 64), (unsigned)((N + 3) / 4));
         if (shared)
             hipLaunchKernelGGL(ctf_exact_fan_kernel, sgrid, dim3(64, 4), 0, ctx->stream, base, fb.spec, half, cs, b,
@@ -567,6 +657,24 @@ artia_status ctf_filter_slabs(artia_ctx* ctx, const float* src, size_t src_strid
 artia_status wbp_filter(artia_ctx* ctx, const float* img, int W, int H, size_t pitch, float* out, size_t out_pitch,
                         float psi_deg, int method) {
     const int N = W > H ? W : H;
+    if (fft2d_supports(N) && fft2d_fits(H, pitch) && fft2d_fits(H, out_pitch) && ctx->numerics == ARTIA_NUMERICS_EXACT) {
+        FftOwn& f = ctx->ffto;
+        const artia_status so = f.ensure(ctx, N);
+        if (so != ARTIA_OK) return so;
+        RowSrc s = square_source(nullptr, 0, W, H, pitch, N);
+        s.raw = img;
+        s.dtype = ARTIA_DT_FLOAT;
+        PrepFilter pf{};
+        pf.wbp = 1;
+        pf.method = method;
+        const float ang = -psi_deg / 180.0f * kPiF;
+        pf.sn[0] = sin((double)ang);
+        pf.cs[0] = cos((double)ang);
+        fft2d_rows_prep(ctx, N, f.tw, s, f.spec, 1);
+        fft2d_cols_prep(ctx, N, f.tw, f.spec, pf, 1);
+        fft2d_rows_store(ctx, N, f.tw, f.spec, square_target(out, 0, W, H, out_pitch, N, nullptr, 0), 1);
+        return check_hip(ctx, hipGetLastError(), "wbp filter");
+    }
     artia_status st = ctx->fft.ensure(ctx, N);
     if (st != ARTIA_OK) return st;
     launch_make_square(ctx, W, H, pitch, img, N, ctx->fft.square, (N - W) / 2, (N - H) / 2, 0, 0);
@@ -575,7 +683,7 @@ artia_status wbp_filter(artia_ctx* ctx, const float* img, int W, int H, size_t p
         return fail(ctx, ARTIA_ERR_FFT, "hipfftSetStream failed");
     if (hipfftExecR2C(ctx->fft.r2c, ctx->fft.square, (hipfftComplex*)ctx->fft.spec) != HIPFFT_SUCCESS)
         return fail(ctx, ARTIA_ERR_FFT, "hipfftExecR2C failed");
-    st = run_wbp_weight(ctx, ctx->fft.spec, N, (size_t)(N / 2 + 1), psi_deg, method);
+    st = run_wbp_weight(ctx, ctx->fft.spec, N, (size_t)(N / 2 + 1), &psi_deg, 1, method);
     if (st != ARTIA_OK) return st;
     if (hipfftExecC2R(ctx->fft.c2r, (hipfftComplex*)ctx->fft.spec, ctx->fft.square) != HIPFFT_SUCCESS)
         return fail(ctx, ARTIA_ERR_FFT, "hipfftExecC2R failed");
@@ -614,7 +722,7 @@ artia_status artia_wbp_weight(artia_ctx* ctx, void* spectrum, int n, size_t pitc
     if (!spectrum || n <= 1 || pitch < (size_t)(n / 2 + 1) || method < 0 || method > 4)
         return fail(ctx, ARTIA_ERR_INVALID_ARGUMENT, "artia_wbp_weight: invalid arguments");
     Timing t(ctx, ms);
-    artia_status st = run_wbp_weight(ctx, (float2*)spectrum, n, pitch, psi_deg, method);
+    artia_status st = run_wbp_weight(ctx, (float2*)spectrum, n, pitch, &psi_deg, 1, method);
     if (st != ARTIA_OK) return st;
     return t.finish();
 }

@@ -1,0 +1,129 @@
+"""The three-kernel Fourier filters at each supported square (N = 128 .. 4096, a power of two) and at
+images that fill it, leave ragged borders or are much narrower, against the FP64 compositions.
+
+Tolerance: a transform's rounding errors are independent over its log2 N^2 <= 24 radix-2 levels, about
+0.6 u each (u = 2^-24) with as much again from the rounded twiddles, so one direction carries
+0.6 u sqrt(2 * 24) = 2.5e-7 and forward and back 3.5e-7 relative L2 for white images; gate 1e-6.
+"""
+import numpy as np
+import pytest
+import torch
+
+import artiatomi_amd as A
+import ctf_compose as CC
+import oracle_lib as O
+import prep_compose as P
+from conftest import rel_l2
+from test_gpu_ctf import per_slab_sart_ctf
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [(128, 128), (127, 128), (128, 5), (256, 201), (512, 512), (333, 512), (1024, 1022), (2048, 1111), (4096, 64),
+         (2047, 4096)]
+
+
+@pytest.fixture(scope="module")
+def ctx(gpu):
+    c = A.ArtiaContext(0)
+    yield c
+    c.close()
+
+
+def white(H, W, seed):
+    return np.random.default_rng(seed).standard_normal((H, W)).astype(np.float32)
+
+
+def mirror_square(img, N):
+    """Mirror padding, clamped where a pad is wider than the image (the oracle's is not defined there)."""
+    def index(n):
+        i = np.arange(N) - (N - n) // 2
+        i = np.where(i < 0, -i - 1, i)
+        return np.clip(np.where(i >= n, 2 * n - i - 1, i), 0, n - 1)
+
+    return img[np.ix_(index(img.shape[0]), index(img.shape[1]))]
+
+
+@pytest.mark.parametrize("W,H", SIZES)
+def test_slab_and_wbp_filters(ctx, W, H):
+    print(f"filters {W} x {H}", flush=True)
+    img, base = white(H, W, W + H), white(H, W, 1)
+    N = max(W, H)
+    corners = [0, H - 1, W - 1, H - 1, 0, 0, W - 1, 0]
+    p = A.ctf_params(pixelsize_nm=0.5, beta_fac=(2.0, 0.0, 0.008, 0.0), amp_contrast=0.07)
+    k = O.ctf_consts(2.7, 300.0, 0.5, N, 0.07)
+    for for_fp, cut, dim in ((True, (0.0, 0.0), (2.0, 2.0)), (False, (1.0, 0.0), (1.0, 1.0))):
+        d_img, d_out = torch.from_numpy(img).cuda(), torch.from_numpy(base).cuda()
+        ctx.ctf_slab_filter(d_img, d_out, corners, p, 3000.0, 3150.0, 20.0, for_fp=for_fp, accumulate=for_fp,
+                            cut_length=cut, dim_length=dim)
+        _, f = CC.slab_filter(img.astype(np.float64), corners, k, 3000.0, 3150.0, 20.0, for_fp, cut, dim,
+                              beta=tuple(p.beta_fac))
+        expect = base.astype(np.float64) + f if for_fp else f
+        assert float(np.abs(f).max()) > 0
+        assert rel_l2(d_out.cpu().numpy(), expect) <= 1e-6
+    out = torch.zeros((H, W), device="cuda")
+    for method in ("ramp", "contrast10"):
+        ctx.wbp_filter(torch.from_numpy(img).cuda(), out, -3.5, method)
+        X = O.wbp_weight(np.fft.rfft2(mirror_square(img.astype(np.float64), N)), -3.5, A._abi.WBP_METHODS[method],
+                         dtype=np.float64)
+        expect = np.fft.irfft2(X, s=(N, N))[(N - H) // 2:(N - H) // 2 + H, (N - W) // 2:(N - W) // 2 + W]
+        assert rel_l2(out.cpu().numpy(), expect) <= 1e-6, method
+
+
+@pytest.mark.parametrize("W,H", [(128, 127), (256, 50), (512, 512), (1024, 700)])
+def test_slab_stacks_equal_single_slabs(ctx, W, H):
+    """The driver's batched slabs (summed forward, fanned backward) against one filter call per slab."""
+    print(f"slab stack {W} x {H}", flush=True)
+    dims = (40, 40, 12)
+    vg = A.volume_geometry(*dims)
+    acq = A.Acquisition.build(vg, W, H, [-20.0, 35.0], psis_deg=[2.0, -1.0], shifts=[(0.5, 1.0), (-1.5, 0.0)])
+    tdef = [A.TiltDefocus(3000.0, 3150.0, 20.0, -20.0), A.TiltDefocus(2700.0, 2800.0, -50.0, 35.0)]
+    ctf = A.ctf_params(pixelsize_nm=0.5, slice_thickness_nm=3.1, beta_fac=(2.0, 0.0, 0.008, 0.0), amp_contrast=0.07)
+    sp = A.sart_params(lambda_=0.3, oversampling=2, cut_length=(1, 1), dim_length=(2, 2))
+    projs = torch.from_numpy(np.stack([white(H, W, 3), white(H, W, 4)])).cuda()
+    vol = torch.zeros(dims[::-1], device="cuda")
+    ctx.sart_ctf_run(vg, acq, tdef, projs, vol, sp, ctf, iterations=2)
+    ref = torch.zeros_like(vol)
+    per_slab_sart_ctf(ctx, vg, acq, tdef, projs, ref, sp, ctf, iterations=2)
+    assert float(ref.abs().max()) > 0
+    assert torch.equal(vol, ref)
+
+
+PREP = {
+    "uint16_none": dict(dtype="uint16", normalization="none", lp=30.0, lps=6.0),
+    "float_std_hp": dict(dtype="float32", normalization="std", lp=0.0, lps=0.0, hp=4.0, hps=2.0),
+    "int16_mean_flip_dose": dict(dtype="int16", normalization="mean", mirror_y=True, lp=25.0, lps=5.0,
+                                 dose_weighting=True, pixelsize_nm=0.25),
+    "int32_wbp_std": dict(dtype="int32", normalization="std", wbp=True, wbp_method="exact", mirror_y=True, lp=35.0,
+                          lps=5.0),
+    "uint32_wbp_none_raw": dict(dtype="uint32", normalization="none", wbp=True, wbp_method="ramp", skip_filter=True,
+                                correct_bad_pixels=False),
+}
+
+
+@pytest.mark.parametrize("W,H", [(128, 90), (101, 256), (512, 512)])
+@pytest.mark.parametrize("name", list(PREP))
+def test_prepare(ctx, name, W, H):
+    """Gates as tests/test_gpu_prep.py's: images and statistics within 1e-5, equal bad-pixel counts; more
+    images than one chunk takes leave each image as it is alone."""
+    print(f"prepare {name} {W} x {H}", flush=True)
+    kw, n = PREP[name], 34
+    rng = np.random.default_rng(5)
+    yy, xx = np.mgrid[0:H, 0:W]
+    imgs = np.rint(800.0 + 100.0 * np.sin(xx / 9.0) - 60.0 * np.cos(yy / 7.0) + rng.normal(0.0, 25.0, (n, H, W)))
+    imgs[:, H // 3, 1] = 30000.0
+    imgs = imgs.astype(kw["dtype"])
+    doses = np.linspace(0.05, 2.0, n).astype(np.float32)
+    psis = np.linspace(-4.0, 3.0, n).astype(np.float32)
+    pp = A.prep_params(**kw)
+    d_in, out = torch.from_numpy(imgs).cuda(), torch.zeros((n, H, W), device="cuda")
+    mean, std, bad = ctx.prepare_projections(pp, d_in, out, psi_deg=psis, dose=doses)
+    for i in (0, 31, 33):
+        ref, m, s, b = P.prepare(imgs[i], psi=float(psis[i]), dose=float(doses[i]),
+                                 **{k: v for k, v in kw.items() if k != "dtype"})
+        assert b == bad[i]
+        assert mean[i] == pytest.approx(m, rel=1e-5, abs=1e-6) and std[i] == pytest.approx(s, rel=1e-5, abs=1e-6)
+        assert rel_l2(out[i].cpu().numpy(), ref) < 1e-5
+        one = torch.zeros((1, H, W), device="cuda")
+        m1, s1, b1 = ctx.prepare_projections(pp, d_in[i:i + 1].contiguous(), one, psi_deg=psis[i:i + 1],
+                                             dose=doses[i:i + 1])
+        assert torch.equal(one[0], out[i]) and (m1[0], s1[0], b1[0]) == (mean[i], std[i], bad[i])
