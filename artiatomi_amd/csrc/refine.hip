@@ -13,6 +13,7 @@
 // because a detector shift translates all samples of a sub-ray alike: dq0/ds = scale * (-u +
 // (u_a / n_a) n) with a the axis whose face sets the entry point (likewise v).
 #include <algorithm>
+#include <climits>
 #include <numeric>
 #include <vector>
 
@@ -548,26 +549,77 @@ constexpr int kMaxCcShift = 32;
 // GetDisplacement per pair (Reconstructor.cpp:1746-1959) as a direct sum over the window: the
 // raw correlation C(r) = sum_y B(y) A(y - r) for every integer r in the disk, then the square's
 // mean and energy terms, the maxShift disk (wbpWeighting.cu:265-294) and nppiMaxIndx's first
-// maximum in the square's row-major order.  Wave w takes candidates w, w + 4, ...; lanes run
-// along window rows.
+// maximum in the square's row-major order.
+//
+// The sum is bound by double multiply-adds (the products of floats are exact in double), so the work is
+// tiled for registers: a thread owns one row shift ry, every S-th window row and kCcR column shifts in
+// double accumulators, and for each 8 window columns takes 8 values of B and 16 of A from LDS for 72
+// multiply-adds.  Neighbouring lanes have neighbouring ry: odd row pitches keep their reads of A apart.
+// Windows are staged in tiles of at most kCcTile columns and as many rows as fit, zero outside the image.
+// 4100 windows of about 76 x 76 with shifts to 12: 22.3 ms with one wave per candidate and two loads per
+// multiply-add, 1.4 ms so.
 // multi != 0: MultiPeakDetection (Reconstructor.cpp:1887-1935): among the peaks of the float map
 // (findPeak, wbpWeighting.cu:329-386: above the 8 neighbours, the two upper diagonal ones or equal,
 // and at least 0.9f of the maximum) the one nearest to zero shift (maxShiftWeighted,
 // wbpWeighting.cu:295-327: weight 1 / (dist + 0.0001f)), first in row-major order; the CC value and
 // the failure test keep the first search's maximum.  Candidates outside the disk are 0 in the map.
+constexpr int kCcR = 9, kCcTile = 80;
+constexpr int kCcStageBytes = 35 << 10;   // four blocks per compute unit at small max_shift
+
+__host__ __device__ inline int cc_side(int M) { return 2 * M + 1; }
+// window rows taken side by side: 256 threads over the row shifts
+__host__ __device__ inline int cc_slices(int M) { return 256 / cc_side(M) < 32 ? 256 / cc_side(M) : 32; }
+// bytes of the staged tiles: less where the candidates' sums leave less of 60 KB, always enough for one
+// row per slice and 256 * kCcR doubles (cc_slices * (pa + pb) + 2 M pa floats: 24.9 KB at M = 32, where
+// 27.6 KB are left)
+__host__ __device__ inline int cc_stage_bytes(int M) {
+    const int rest = (60 << 10) - cc_side(M) * cc_side(M) * 8;
+    return rest < kCcStageBytes ? rest : kCcStageBytes;
+}
+__device__ __forceinline__ bool cc_in_disk(int rx, int ry, int M) {
+    return sqrtf((float)(rx * rx + ry * ry)) <= (float)M;
+}
+
+// The first maximum of val over the block's order keys k (each thread's own first): its key in *key on
+// all threads, and its value.
+__device__ __forceinline__ double block_first_max(double val, int k, int* key) {
+    __shared__ double bv[256];
+    __shared__ int bk[256];
+    bv[threadIdx.x] = val;
+    bk[threadIdx.x] = k;
+    __syncthreads();
+    for (int o = 128; o > 0; o >>= 1) {
+        if ((int)threadIdx.x < o) {
+            const double v = bv[threadIdx.x + o];
+            const int q = bk[threadIdx.x + o];
+            // a thread without candidates has key INT_MAX
+            if (q != INT_MAX && (bk[threadIdx.x] == INT_MAX || v > bv[threadIdx.x] ||
+                                 (v == bv[threadIdx.x] && q < bk[threadIdx.x]))) {
+                bv[threadIdx.x] = v;
+                bk[threadIdx.x] = q;
+            }
+        }
+        __syncthreads();
+    }
+    const double r = bv[0];
+    *key = bk[0];
+    __syncthreads();
+    return r;
+}
+
 __global__ void __launch_bounds__(256) pair_cc_kernel(const PairDev* __restrict__ pairs, int npairs,
                                                       const float* __restrict__ models,
                                                       const float* __restrict__ targets, int N, int M,
                                                       int multi, int* __restrict__ peak, float* __restrict__ ccv,
                                                       float* __restrict__ ccmap) {
-    __shared__ double craw[(2 * kMaxCcShift + 1) * (2 * kMaxCcShift + 1)];
+    extern __shared__ double cc_lds[];   // the candidates' sums, then the staged tiles
     const int p = (int)blockIdx.x;
     if (p >= npairs) return;
     const PairDev& P = pairs[p];
     const int w = P.w, h = P.h;
     const float* __restrict__ A = targets + P.img_offset;
     const float* __restrict__ B = models + P.img_offset;
-    const int lane = (int)(threadIdx.x & 63), wave = (int)(threadIdx.x >> 6);
+    const int lane = (int)(threadIdx.x & 63), wave = (int)(threadIdx.x >> 6), tid = (int)threadIdx.x;
     // window sums of A, A^2, B, B^2 (the square is zero outside the window)
     double sa = 0.0, saa = 0.0, sb = 0.0;
     double sbb = 0.0;
@@ -588,54 +640,98 @@ __global__ void __launch_bounds__(256) pair_cc_kernel(const PairDev* __restrict_
     double d = 0.0, e = 0.0;
     block_sum3(sbb, d, e);
     if (threadIdx.x == 0) tot[3] = sbb;
-    const int side = 2 * M + 1, ncand = side * side;
-    for (int c = wave; c < ncand; c += 4) {
-        const int rx = c % side - M, ry = c / side - M;
-        double acc = 0.0;
-        if (sqrtf((float)(rx * rx + ry * ry)) <= (float)M) {
-            const int ylo = max(0, ry), yhi = min(h, h + ry);   // rows with 0 <= y - ry < h
-            const int xlo = max(0, rx), xhi = min(w, w + rx);
-            for (int y = ylo; y < yhi; y++) {
-                const float* __restrict__ brow = B + (long long)y * w;
-                const float* __restrict__ arow = A + (long long)(y - ry) * w - rx;
-                for (int x = xlo + lane; x < xhi; x += 64) acc += (double)brow[x] * (double)arow[x];
+    const int side = cc_side(M), ncand = side * side, S = cc_slices(M);
+    double* const craw = cc_lds;
+    float* const stage = reinterpret_cast<float*>(cc_lds + ncand);
+    const int ry = tid % side - M, slice = tid / side;
+    const int ntx = (w + kCcTile - 1) / kCcTile, xt = ((w + ntx - 1) / ntx + 7) / 8 * 8;
+    const int pa = (xt + 8) | 1, pb = xt | 1;   // row pitches of the tiles of A and B
+    const int fit = (cc_stage_bytes(M) / 4 - 2 * M * pa) / (S * (pa + pb));
+    const int nty = (h + fit * S - 1) / (fit * S);
+    const int nb = S * ((h + S * nty - 1) / (S * nty));   // window rows per tile
+    float* const At = stage;
+    float* const Bt = stage + (nb + 2 * M) * pa;
+    for (int rx0 = -M; rx0 <= M; rx0 += kCcR) {
+        double acc[kCcR];
+#pragma unroll
+        for (int r = 0; r < kCcR; r++) acc[r] = 0.0;
+        for (int y0 = 0; y0 < h; y0 += nb) {
+            for (int x0 = 0; x0 < w; x0 += xt) {
+                __syncthreads();
+                for (int r = wave; r < nb + 2 * M; r += 4) {
+                    const int y = y0 - M + r;
+                    for (int c = lane; c < xt + 8; c += 64) {
+                        const int x = x0 - rx0 - 8 + c;
+                        At[r * pa + c] = y >= 0 && y < h && x >= 0 && x < w ? A[(long long)y * w + x] : 0.0f;
+                    }
+                }
+                for (int r = wave; r < nb; r += 4) {
+                    const int y = y0 + r;
+                    for (int c = lane; c < xt; c += 64) {
+                        const int x = x0 + c;
+                        Bt[r * pb + c] = y < h && x < w ? B[(long long)y * w + x] : 0.0f;
+                    }
+                }
+                __syncthreads();
+                if (slice < S) {
+                    for (int y = slice; y < nb && y0 + y < h; y += S) {
+                        const float* arow = At + (y - ry + M) * pa;
+                        const float* brow = Bt + y * pb;
+                        for (int x = 0; x < xt; x += 8) {
+                            double a[16], b[8];
+#pragma unroll
+                            for (int q = 0; q < 16; q++) a[q] = (double)arow[x + q];
+#pragma unroll
+                            for (int q = 0; q < 8; q++) b[q] = (double)brow[x + q];
+#pragma unroll
+                            for (int q = 0; q < 8; q++)
+#pragma unroll
+                                for (int r = 0; r < kCcR; r++) acc[r] = __builtin_fma(b[q], a[q - r + 8], acc[r]);
+                        }
+                    }
+                }
             }
-            for (int o = 32; o > 0; o >>= 1) acc += __shfl_down(acc, o);
         }
-        if (lane == 0) craw[c] = acc;
+        __syncthreads();
+        double* const part = reinterpret_cast<double*>(stage);
+#pragma unroll
+        for (int r = 0; r < kCcR; r++) part[r * 256 + tid] = acc[r];
+        __syncthreads();
+        for (int q = tid; q < kCcR * side; q += 256) {
+            const int r = q / side, row = q % side;
+            double sum = 0.0;
+            for (int k = 0; k < S; k++) sum += part[r * 256 + k * side + row];
+            if (rx0 + r <= M) craw[row * side + rx0 + r + M] = sum;
+        }
     }
     __syncthreads();
-    if (threadIdx.x != 0) return;
     const double SA = tot[0], SB = tot[2], n2 = (double)N * (double)N;
     const double sumA = tot[1] - SA * SA / n2, sumB = tot[3] - SB * SB / n2;
     const double den = sqrt(sumA * sumB), off = SA * SB / n2;
     const bool ok = sumA * sumB > 0.0;
-    // candidates in the square's row-major order: rows ry = 0..M, then -M..-1; likewise columns
+    // candidates in the square's row-major order k: rows ry = 0..M, then -M..-1; likewise columns
+    const auto shift_of = [&](int k, int& rx, int& ry) {
+        const int yy = k / side, xx = k % side;
+        ry = yy <= M ? yy : yy - side;
+        rx = xx <= M ? xx : xx - side;
+    };
     double best = 0.0;
-    int bx = 0, by = 0;
-    bool found = false;
-    for (int yy = 0; yy < side; yy++) {
-        const int ry = yy <= M ? yy : yy - side;
-        for (int xx = 0; xx < side; xx++) {
-            const int rx = xx <= M ? xx : xx - side;
-            if (!(sqrtf((float)(rx * rx + ry * ry)) <= (float)M)) continue;
-            const int c = (ry + M) * side + (rx + M);
-            const double cc = ok ? (craw[c] - off) / den : 0.0;
-            if (ccmap) ccmap[(long long)p * ncand + c] = (float)cc;
-            if (!found || cc > best) {
-                best = cc;
-                bx = rx;
-                by = ry;
-                found = true;
-            }
+    int bestk = INT_MAX;
+    for (int k = tid; k < ncand; k += 256) {
+        int rx, ry;
+        shift_of(k, rx, ry);
+        const int c = (ry + M) * side + (rx + M);
+        const bool in = cc_in_disk(rx, ry, M);
+        const double cc = in && ok ? (craw[c] - off) / den : 0.0;
+        craw[c] = cc;
+        if (ccmap) ccmap[(long long)p * ncand + c] = (float)cc;
+        if (in && (bestk == INT_MAX || cc > best)) {
+            best = cc;
+            bestk = k;
         }
     }
-    if (ccmap) {
-        for (int c = 0; c < ncand; c++) {
-            const int rx = c % side - M, ry = c / side - M;
-            if (!(sqrtf((float)(rx * rx + ry * ry)) <= (float)M)) ccmap[(long long)p * ncand + c] = 0.0f;
-        }
-    }
+    best = block_first_max(best, bestk, &bestk);
+    int bx, by;
     if (multi) {
         // the float map value at shift (rx, ry), wrapped around the N x N square as findPeak's
         // neighbours are: 0 outside the disk (maxShift)
@@ -644,38 +740,33 @@ __global__ void __launch_bounds__(256) pair_cc_kernel(const PairDev* __restrict_
             ry = ((ry % N) + N) % N;
             rx = rx > N / 2 ? rx - N : rx;
             ry = ry > N / 2 ? ry - N : ry;
-            if (rx < -M || rx > M || ry < -M || ry > M || !(sqrtf((float)(rx * rx + ry * ry)) <= (float)M))
-                return 0.0f;
-            return ok ? (float)((craw[(ry + M) * side + (rx + M)] - off) / den) : 0.0f;
+            if (rx < -M || rx > M || ry < -M || ry > M) return 0.0f;
+            return (float)craw[(ry + M) * side + (rx + M)];
         };
         const float thr = (float)best * 0.9f;
         float bestw = 0.0f;
-        int mx = 0, my = 0;
-        bool seen = false;
-        for (int yy = 0; yy < side; yy++) {
-            const int ry = yy <= M ? yy : yy - side;
-            for (int xx = 0; xx < side; xx++) {
-                const int rx = xx <= M ? xx : xx - side;
-                const float d = sqrtf((float)(rx * rx + ry * ry));
-                float wv = 0.0f;
-                if (d <= (float)M) {
-                    const float val = map(rx, ry);
-                    const bool pk = map(rx - 1, ry) < val && map(rx + 1, ry) < val && map(rx, ry - 1) < val &&
-                                    map(rx, ry + 1) < val && map(rx - 1, ry - 1) <= val && map(rx - 1, ry + 1) < val &&
-                                    map(rx + 1, ry - 1) <= val && map(rx + 1, ry + 1) < val && val >= thr;
-                    wv = pk ? 1.0f / (d + 0.0001f) : 0.0f;
-                }
-                if (!seen || wv > bestw) {
-                    bestw = wv;
-                    mx = rx;
-                    my = ry;
-                    seen = true;
-                }
+        bestk = INT_MAX;
+        for (int k = tid; k < ncand; k += 256) {
+            int rx, ry;
+            shift_of(k, rx, ry);
+            const float d = sqrtf((float)(rx * rx + ry * ry));
+            float wv = 0.0f;
+            if (d <= (float)M) {
+                const float val = map(rx, ry);
+                const bool pk = map(rx - 1, ry) < val && map(rx + 1, ry) < val && map(rx, ry - 1) < val &&
+                                map(rx, ry + 1) < val && map(rx - 1, ry - 1) <= val && map(rx - 1, ry + 1) < val &&
+                                map(rx + 1, ry - 1) <= val && map(rx + 1, ry + 1) < val && val >= thr;
+                wv = pk ? 1.0f / (d + 0.0001f) : 0.0f;
+            }
+            if (bestk == INT_MAX || wv > bestw) {
+                bestw = wv;
+                bestk = k;
             }
         }
-        bx = mx;
-        by = my;
+        (void)block_first_max((double)bestw, bestk, &bestk);
     }
+    if (tid != 0) return;
+    shift_of(bestk, bx, by);
     const bool fail = !ok || !(best > 0.0);
     peak[2 * p] = fail ? -1000 : bx;
     peak[2 * p + 1] = fail ? -1000 : by;
@@ -948,7 +1039,8 @@ artia_status artia_pairs_cc_search(artia_pairs* ps, const float* models, const f
                     max_shift, kMaxCcShift, square);
     artia_ctx* ctx = ps->ctx;
     Timing t(ctx, ms);
-    hipLaunchKernelGGL(pair_cc_kernel, dim3((unsigned)ps->npairs), dim3(256), 0, ctx->stream, ps->pairs, ps->npairs,
+    const size_t lds = (size_t)cc_side(max_shift) * cc_side(max_shift) * sizeof(double) + (size_t)cc_stage_bytes(max_shift);
+    hipLaunchKernelGGL(pair_cc_kernel, dim3((unsigned)ps->npairs), dim3(256), lds, ctx->stream, ps->pairs, ps->npairs,
                        models, targets, square, max_shift, multi_peak ? 1 : 0, peak, cc_value,
                        cc_map);
     artia_status st = check_hip(ctx, hipGetLastError(), "artia_pairs_cc_search launch");
