@@ -62,14 +62,16 @@ __global__ void __launch_bounds__(256) fp_adjoint_kernel(VolG v, TiltG g, const 
 
 // The same transpose with each tile's rays walked through LDS-staged slabs (tube_walk.hpp): the
 // weights are summed per slab in a box of shared memory and added to grad with one atomic per box
-// voxel, not eight per cell.  Tiles are dealt to the XCDs in groups, as in the forward projector.  A wave
+// voxel, not eight per cell.  The box is in double: its float additions in LDS took 3.5 of 3.9 ms per
+// 512x512x128 tilt, a wave's ds_add_f32 194 cycles of a compute unit against 9 of a ds_add_f64; 0.51 ms so, where
+// 0.36 ms are the walk and the weights.  tp.box values of LDS: the tilt's largest slab box.  Tiles are dealt to the XCDs in groups, as in the forward projector.  A wave
 // takes one sub-ray of every pixel of the tile, so that its lanes are a pixel apart and rarely add to the
 // same voxel at once.
 template <bool kFlat>
 __global__ void __launch_bounds__(256) fp_adjoint_lds_kernel(VolG v, TiltG g, const float* __restrict__ resid,
                                                              size_t pitch, Roi roi, float scale,
                                                              float* __restrict__ grad, TubePlan tp) {
-    __shared__ float chunk[kChunkFloats];
+    extern __shared__ double chunk[];   // tp.box values
     __shared__ int zr[2];
     const int pix = (int)(threadIdx.x & 63), sub = (int)(threadIdx.x >> 6);
     const int xcd = (int)(blockIdx.x & 7u), slot = (int)(blockIdx.x >> 3);
@@ -101,11 +103,11 @@ __global__ void __launch_bounds__(256) fp_adjoint_lds_kernel(VolG v, TiltG g, co
         return;
     }
     const TubeDir td = tube_dir(v, g, step);
-    tube_scatter(v, grad, chunk, zr, tp, tb, td, s.q0, s.count, [&](float wgt[8], const int cell[3], int k, int mi) {
+    tube_scatter(v, grad, chunk, zr, tp, tb, td, s.q0, s.count, [&](double wgt[8], const int cell[3], int k, int mi) {
         double W[8];
         cell_weights(cell_moments(s.q0, td.dq, cell, k, mi), W);
 #pragma unroll
-        for (int i = 0; i < 8; i++) wgt[i] = (float)(r * W[i]);
+        for (int i = 0; i < 8; i++) wgt[i] = r * W[i];
     });
 }
 
@@ -304,10 +306,10 @@ artia_status artia_fp_adjoint(artia_ctx* ctx, const artia_vol_geom* vg, const ar
     if (r.x1 > r.x0 && r.y1 > r.y0 && ctx->march_lds && tube_plan(vd, gd, tp)) {
         const dim3 grid1 = tile_grid(r, tp);
         if (gd.n[1] == 0.0f)
-            hipLaunchKernelGGL(fp_adjoint_lds_kernel<true>, grid1, dim3(256), 0, ctx->stream, vd, gd, resid, pitch, r,
+            hipLaunchKernelGGL(fp_adjoint_lds_kernel<true>, grid1, dim3(256), tp.box * sizeof(double), ctx->stream, vd, gd, resid, pitch, r,
                                scale, vol_grad, tp);
         else
-            hipLaunchKernelGGL(fp_adjoint_lds_kernel<false>, grid1, dim3(256), 0, ctx->stream, vd, gd, resid, pitch, r,
+            hipLaunchKernelGGL(fp_adjoint_lds_kernel<false>, grid1, dim3(256), tp.box * sizeof(double), ctx->stream, vd, gd, resid, pitch, r,
                                scale, vol_grad, tp);
     } else if (r.x1 > r.x0 && r.y1 > r.y0)
     {

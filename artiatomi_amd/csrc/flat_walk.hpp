@@ -186,7 +186,8 @@ struct FlatBox {
 // The box of cell layers [zs, ze] for the rays of a tile (see tube_slabs); x is padded by two
 // clamp-addressed columns, so that a lane at the volume's faces keeps a column of margin.  SY is odd
 // where that fits (lanes of neighbouring columns in different banks).
-__device__ __forceinline__ FlatBox flat_box(const VolG& v, const TubePlan& tp, const TubeBox& tb, int zs, int ze) {
+__device__ __forceinline__ FlatBox flat_box(const VolG& v, const TubePlan& tp, const TubeBox& tb, int zs, int ze,
+                                            int cap = kChunkFloats) {
     FlatBox q;
     const float z0 = (float)zs, z1 = (float)(ze + 1);
     q.X0 = wave_uniform(max((int)floorf(tb.axl + fminf(tp.bx * z0, tp.bx * z1)) - 1, -2));
@@ -199,8 +200,8 @@ __device__ __forceinline__ FlatBox flat_box(const VolG& v, const TubePlan& tp, c
     q.CY = wave_uniform(q.Y1 - q.Y0 + 1);
     q.CZ = q.Z1 - q.Z0 + 1;
     const bool some = q.CX > 1 && q.CX <= 256 && q.CY > 1 && q.CZ > 1;
-    q.SY = some && q.CX * (q.CY | 1) * q.CZ <= kChunkFloats ? (q.CY | 1) : q.CY;
-    q.staged = some && q.CX * q.SY * q.CZ <= kChunkFloats;
+    q.SY = some && q.CX * (q.CY | 1) * q.CZ <= cap ? (q.CY | 1) : q.CY;
+    q.staged = some && q.CX * q.SY * q.CZ <= cap;
     return q;
 }
 
@@ -522,7 +523,7 @@ __device__ __forceinline__ void flat_scatter_direct(const VolG& v, float* __rest
 
 // The lane's samples in cell layers [zs, ze] of a slab, into the slab's box (zeroed before, added to
 // the volume after) where its cells provably lie in it, otherwise straight into the volume.
-__device__ __forceinline__ void flat_scatter_slab(const VolG& v, float* __restrict__ grad, float* __restrict__ chunk,
+__device__ __forceinline__ void flat_scatter_slab(const VolG& v, float* __restrict__ grad, double* __restrict__ chunk,
                                                   const FlatBox& q, const FlatDir& d, const float q0[3],
                                                   const float dq[3], double rd, FlatWalker& w, int zs, int ze) {
     const int zlast = d.sgn[1] > 0 ? ze : -(zs + 1);
@@ -548,8 +549,8 @@ __device__ __forceinline__ void flat_scatter_slab(const VolG& v, float* __restri
         auto put = [&](int dx, int dz, double s) {
             const int at = o + (dx ? sx : 0) + (dz ? sz : 0);
             const double s1 = s * b;
-            atomicAdd(chunk + at, (float)(s - s1));
-            atomicAdd(chunk + at + 1, (float)s1);
+            unsafeAtomicAdd(chunk + at, s - s1);
+            unsafeAtomicAdd(chunk + at + 1, s1);
         };
         if (!(w.r[1] > rstop && w.k < w.count)) {
             e.flush(put);
@@ -561,7 +562,7 @@ __device__ __forceinline__ void flat_scatter_slab(const VolG& v, float* __restri
 }
 
 // grad += rd times the transpose of flat_tube_walk's sum over the lane's samples.
-__device__ __forceinline__ void flat_tube_scatter(const VolG& v, float* __restrict__ grad, float* __restrict__ chunk,
+__device__ __forceinline__ void flat_tube_scatter(const VolG& v, float* __restrict__ grad, double* __restrict__ chunk,
                                                   int* zr, const TubePlan& tp, const TubeBox& tb, const float dq[3],
                                                   const float q0[3], int count, double rd) {
     const FlatDir d = flat_dir(dq);
@@ -577,11 +578,11 @@ __device__ __forceinline__ void flat_tube_scatter(const VolG& v, float* __restri
     const int nslab = zlo <= zhi ? (zhi - zlo) / kSlabCells + 1 : 0;
     for (int j = 0; j < nslab; j++) {
         const int zs = tp.zdir > 0 ? zlo + j * kSlabCells : zhi - (j + 1) * kSlabCells + 1, ze = zs + kSlabCells - 1;
-        const FlatBox q = flat_box(v, tp, tb, zs, ze);
+        const FlatBox q = flat_box(v, tp, tb, zs, ze, tp.box);
         const int n = q.CX * q.SY * q.CZ;
         __syncthreads();   // the previous slab's box is in the volume
         if (q.staged)
-            for (int e = (int)threadIdx.x; e < n; e += 256) chunk[e] = 0.0f;
+            for (int e = (int)threadIdx.x; e < n; e += 256) chunk[e] = 0.0;
         __syncthreads();
         if (w.active()) flat_scatter_slab(v, grad, chunk, q, d, q0, dq, rd, w, zs, ze);
         if (q.staged) {
@@ -593,7 +594,7 @@ __device__ __forceinline__ void flat_tube_scatter(const VolG& v, float* __restri
                 const size_t gx = (size_t)clampi(q.X0 + x, 0, v.nx - 1);
                 for (int r = r0; r < rows; r += P) {
                     const int zz = small_div(r, q.CY), yy = r - zz * q.CY;
-                    const float add = chunk[(zz * q.CX + x) * q.SY + yy];
+                    const float add = (float)chunk[(zz * q.CX + x) * q.SY + yy];
                     const size_t row = (size_t)clampi(q.Z0 + zz, 0, v.nz - 1) * (size_t)v.ny +
                                        (size_t)clampi(q.Y0 + yy, 0, v.ny - 1);
                     if (add != 0.0f) unsafeAtomicAdd(grad + row * (size_t)v.nx + gx, add);

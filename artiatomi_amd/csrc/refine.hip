@@ -474,7 +474,7 @@ __global__ void __launch_bounds__(kAdjFlatThreads) pair_adjoint_flat_kernel(Pair
 // vol_grads += scale * P_s^T in: the transpose of the per-cell closed form, one set of eight
 // atomics per cell a sub-ray crosses (as fp_adjoint_kernel).
 __global__ void __launch_bounds__(256) pair_adjoint_kernel(PairArgs a, float scale, float* __restrict__ grads) {
-    __shared__ float chunk[kChunkFloats];
+    __shared__ double chunk[kChunkFloats];
     __shared__ int zr[2];
     const int slot = slot_of_block(a.per_xcd);
     if (slot >= a.npairs) return;
@@ -506,11 +506,11 @@ __global__ void __launch_bounds__(256) pair_adjoint_kernel(PairArgs a, float sca
             const double py = (double)(y0 + j) + ((sub & 1) ? 0.75 : 0.25);
             if (r == 0.0 || !subray_samples(v, g, px, py, step, s, sx, sy)) s.count = 0;
         }
-        auto weights = [&](float wgt[8], const int cell[3], int k, int mi) {
+        auto weights = [&](double wgt[8], const int cell[3], int k, int mi) {
             double W[8];
             cell_weights(cell_moments(s.q0, s.dq, cell, k, mi), W);
 #pragma unroll
-            for (int c = 0; c < 8; c++) wgt[c] = (float)(r * W[c]);
+            for (int c = 0; c < 8; c++) wgt[c] = r * W[c];
         };
         if (g.n[1] == 0.0f) {   // uniform: flat rays (flat_walk.hpp)
             float dq[3];
@@ -534,11 +534,11 @@ __global__ void __launch_bounds__(256) pair_adjoint_kernel(PairArgs a, float sca
             for_each_cell(s.q0, s.dq, s.count, [&](const int cell[3], int k, int mi) {
                 uint32_t o[8];
                 cell_corners_bytes(v, cell, o);
-                float wgt[8];
+                double wgt[8];
                 weights(wgt, cell, k, mi);
 #pragma unroll
                 for (int c = 0; c < 8; c++)
-                    if (wgt[c] != 0.0f) unsafeAtomicAdd(gv + (o[c] >> 2), wgt[c]);
+                    if (wgt[c] != 0.0) unsafeAtomicAdd(gv + (o[c] >> 2), (float)wgt[c]);
             });
         }
     }

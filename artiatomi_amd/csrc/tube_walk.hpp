@@ -12,6 +12,7 @@
 // order as an unstaged walk, so sums are bit-identical to it.
 #pragma once
 
+#include <algorithm>
 #include <climits>
 #include <cmath>
 
@@ -29,6 +30,7 @@ struct TubePlan {
     float bx, by;   // dq_x / dq_z and dq_y / dq_z (texel units; equal for all sub-rays)
     int zdir;       // sign of dq_z (nonzero)
     int tiles_x, tiles_y, groups_x;   // launch layout of the forward projector (8x8-pixel tiles)
+    int box;        // values a slab's box needs, rows of odd length (at most kChunkFloats): the scatter walk's LDS
 };
 
 // The plan of one tilt geometry, or false when the staged walk does not apply: volumes below 2
@@ -59,6 +61,7 @@ inline bool tube_plan(const VolG& v, const TiltG& g, TubePlan& tp, double span =
     tp.by = (float)by;
     tp.zdir = N[2] > 0.0 ? 1 : -1;
     tp.tiles_x = tp.tiles_y = tp.groups_x = 0;
+    tp.box = std::min((int)(cx + 1.0) * ((int)(cy + 1.0) | 1) * (slab + 2), kChunkFloats);
     return true;
 }
 
@@ -298,10 +301,11 @@ __device__ __forceinline__ void stage_box_rows(const VolG& v, const T* __restric
 //     cells with m = 0, to which it must add nothing but +-0;
 //   scatter (kScatter true): f(float wgt[8], cell, k, m) returns eight corner weights, which are
 //     added to the slab's box in LDS (shared-memory atomics) and then to grad with one global
-//     atomic per box voxel, instead of eight global atomics per cell.
-template <bool kScatter, bool kRows, typename T, class F>
+//     atomic per box voxel, instead of eight global atomics per cell.  The box is in double: a wave's
+//     ds_add_f64 takes 9 cycles of a compute unit without conflicts, its ds_add_f32 194 (measured).
+template <bool kScatter, bool kRows, typename T, typename C, class F>
 __device__ __forceinline__ void tube_slabs(const VolG& v, const T* __restrict__ vol, float* __restrict__ grad,
-                                           float* __restrict__ chunk, int* zr, const TubePlan& tp, const TubeBox& tb,
+                                           C* __restrict__ chunk, int* zr, const TubePlan& tp, const TubeBox& tb,
                                            const TubeDir& td, const float q0[3], int count, F&& f) {
     // cell layers the block's sub-rays cross
     __syncthreads();   // a previous walk's readers are done with zr and chunk
@@ -320,12 +324,12 @@ __device__ __forceinline__ void tube_slabs(const VolG& v, const T* __restrict__ 
     const int zlo = max(zr[0], -1), zhi = min(zr[1], v.nz - 1);
 
     // corner weights into the box (LDS) or, outside it, straight to grad
-    auto scatter_global = [&](const int cell[3], const float wgt[8]) {
+    auto scatter_global = [&](const int cell[3], const double wgt[8]) {
         size_t o[8];
         cell_corners<true>(v, cell, o);
 #pragma unroll
         for (int i = 0; i < 8; i++)
-            if (wgt[i] != 0.0f) unsafeAtomicAdd(grad + o[i], wgt[i]);
+            if (wgt[i] != 0.0) unsafeAtomicAdd(grad + o[i], (float)wgt[i]);
     };
     CellWalker w;
     w.init_dir(q0, td.sgn, td.inv, count);
@@ -343,15 +347,15 @@ __device__ __forceinline__ void tube_slabs(const VolG& v, const T* __restrict__ 
         const int Y1 = min((int)floorf(tb.ayh + fmaxf(tp.by * z0, tp.by * z1)) + 2, v.ny);
         const int Z0 = max(zs, -1), Z1 = min(ze + 1, v.nz);
         const int CX = wave_uniform(X1 - X0 + 1), CY = wave_uniform(Y1 - Y0 + 1), CZ = Z1 - Z0 + 1;
-        const bool staged = CX > 1 && CY > 1 && CZ > 1 && CX * CY * CZ <= kChunkFloats;
+        const bool staged = CX > 1 && CY > 1 && CZ > 1 && CX * CY * CZ <= (kScatter ? tp.box : kChunkFloats);
         const int n = CX * CY * CZ;
         __syncthreads();   // the previous slab's reads (or flush) are done
         if (staged) {
             if (kScatter)
-                for (int e = (int)threadIdx.x; e < n; e += 256) chunk[e] = 0.0f;
-            else if (kRows)
+                for (int e = (int)threadIdx.x; e < n; e += 256) chunk[e] = 0;
+            else if constexpr (kRows)
                 stage_box_rows(v, vol, chunk, X0, Y0, Z0, CX, CY, n);
-            else
+            else if constexpr (!kScatter)
                 stage_box(v, vol, chunk, X0, Y0, Z0, CX, CY, n);
         }
         __syncthreads();
@@ -376,15 +380,15 @@ __device__ __forceinline__ void tube_slabs(const VolG& v, const T* __restrict__ 
             int o = ((w.icell(2) - Z0) * CY + (w.icell(1) - Y0)) * CX + (w.icell(0) - X0);
             // a fast lane enters with its cell in [zs, ze] and moves monotonically in z, so staying
             // in the slab is one range test
-            if (kScatter) {
+            if constexpr (kScatter) {
                 while (w.active() && w.z_in(zs, kSlabCells)) {
                     w.step(
                         [&](const int* cell, int k, int mi) {
-                            float val[8];
+                            double val[8];
                             f(val, cell, k, mi);
 #pragma unroll
                             for (int i = 0; i < 8; i++)
-                                if (val[i] != 0.0f) atomicAdd(chunk + o + off[i], val[i]);
+                                if (val[i] != 0.0) unsafeAtomicAdd(chunk + o + off[i], val[i]);
                         },
                         [&](int i) { o += i == 0 ? st0 : (i == 1 ? st1 : st2); });
                 }
@@ -406,8 +410,8 @@ __device__ __forceinline__ void tube_slabs(const VolG& v, const T* __restrict__ 
         } else {
             while (w.active() && (tp.zdir > 0 ? w.icell(2) <= ze : w.icell(2) >= zs)) {
                 w.step([&](const int* cell, int k, int mi) {
-                    float val[8];
-                    if (kScatter) {
+                    if constexpr (kScatter) {
+                        double val[8];
                         f(val, cell, k, mi);
                         const int ic[3] = {cell[0], cell[1], cell[2]};
                         const int cx = ic[0] - X0, cy = ic[1] - Y0, cz = ic[2] - Z0;
@@ -417,11 +421,12 @@ __device__ __forceinline__ void tube_slabs(const VolG& v, const T* __restrict__ 
                             const int off[8] = {0, 1, CX, CX + 1, CXY, CXY + 1, CXY + CX, CXY + CX + 1};
 #pragma unroll
                             for (int i = 0; i < 8; i++)
-                                if (val[i] != 0.0f) atomicAdd(chunk + o + off[i], val[i]);
+                                if (val[i] != 0.0) unsafeAtomicAdd(chunk + o + off[i], val[i]);
                         } else {
                             scatter_global(ic, val);
                         }
                     } else {
+                        float val[8];
                         const int ic[3] = {cell[0], cell[1], cell[2]};
                         chunk_corners(v, vol, chunk, staged, X0, Y0, Z0, CX, CY, CZ, ic, val);
                         f(val, cell, k, mi);
@@ -434,7 +439,7 @@ __device__ __forceinline__ void tube_slabs(const VolG& v, const T* __restrict__ 
             if ((int)threadIdx.x < n) {
                 BoxCursor c((int)threadIdx.x, CX, CY);
                 for (int e = (int)threadIdx.x; e < n; e += 256) {
-                    const float a = chunk[e];
+                    const float a = (float)chunk[e];
                     if (a != 0.0f) unsafeAtomicAdd(grad + c.voxel(v, X0, Y0, Z0), a);
                     c.next();
                 }
@@ -444,12 +449,13 @@ __device__ __forceinline__ void tube_slabs(const VolG& v, const T* __restrict__ 
     // cells beyond the slabs (not expected): global memory
     while (w.active()) {
         w.step([&](const int* cell, int k, int mi) {
-            float val[8];
             const int ic[3] = {cell[0], cell[1], cell[2]};
-            if (kScatter) {
+            if constexpr (kScatter) {
+                double val[8];
                 f(val, cell, k, mi);
                 scatter_global(ic, val);
             } else {
+                float val[8];
                 size_t o[8];
                 cell_corners<true>(v, ic, o);
 #pragma unroll
@@ -573,7 +579,7 @@ __device__ __forceinline__ void tube_walk(const VolG& v, const T* __restrict__ v
 
 // The scatter walk (see tube_slabs): grad += the weights f returns.
 template <class F>
-__device__ __forceinline__ void tube_scatter(const VolG& v, float* __restrict__ grad, float* __restrict__ chunk,
+__device__ __forceinline__ void tube_scatter(const VolG& v, float* __restrict__ grad, double* __restrict__ chunk,
                                              int* zr, const TubePlan& tp, const TubeBox& tb, const TubeDir& td,
                                              const float q0[3], int count, F&& f) {
     tube_slabs<true, false>(v, static_cast<const float*>(nullptr), grad, chunk, zr, tp, tb, td, q0, count, f);
