@@ -190,7 +190,7 @@ __global__ void __launch_bounds__(256) bp_exact_kernel(VolG v, TiltG g, BPExact 
         tw = max(0, tx1 - tx0 + 1);
         const int th = max(0, ty1 - ty0 + 1);
         for (int idx = tid; idx < tw * th; idx += 256) {
-            const int r = idx / tw, c = idx - r * tw;
+            const int r = small_div(idx, tw), c = idx - r * tw;
             tile[idx] = img[(size_t)(ty0 + r) * pitch + (size_t)(tx0 + c)];
         }
         __syncthreads();
@@ -301,20 +301,9 @@ __global__ void __launch_bounds__(256) bp_win_kernel(VolG v, BPWinSet S, T* __re
         // consecutive tile rows at the same columns, fall in different banks
         const int ts = (tw | 1) * th <= kTileFloats ? (tw | 1) : tw;
         if (t > 0) __syncthreads();   // the previous tilt's readers are done
-        // tile entry idx = r * tw + c, strided by 256 over the block: one division per thread,
-        // then the row and column are stepped (tiles are often a few columns wide and tall)
-        if (tid < tw * th) {
-            int r = tid / tw, c = tid - r * tw;
-            const int dr = 256 / tw, dc = 256 - dr * tw;
-            for (int idx = tid; idx < tw * th; idx += 256) {
-                tile[r * ts + c] = img[(size_t)(ty0 + r) * pitch + (size_t)(tx0 + c)];
-                r += dr;
-                c += dc;
-                if (c >= tw) {
-                    c -= tw;
-                    r++;
-                }
-            }
+        for (int idx = tid; idx < tw * th; idx += 256) {
+            const int r = small_div(idx, tw), c = idx - r * tw;
+            tile[r * ts + c] = img[(size_t)(ty0 + r) * pitch + (size_t)(tx0 + c)];
         }
         __syncthreads();
 #pragma unroll
@@ -383,8 +372,8 @@ __global__ void __launch_bounds__(256, 8) bp_stack_kernel(VolG v, TiltG g, BPExa
         if (tiled) {
             const int n = plane * (k1 - k0 + 1);
             for (int idx = tid; idx < n; idx += 256) {
-                const int s = idx / plane, rem = idx - s * plane;
-                const int r = rem / tw, c = rem - r * tw;
+                const int s = small_div(idx, plane), rem = idx - s * plane;
+                const int r = small_div(rem, tw), c = rem - r * tw;
                 tile[idx] = stack[(size_t)(k0 + s) * stride + (size_t)(ty0 + r) * pitch + (size_t)(tx0 + c)];
             }
             __syncthreads();
@@ -490,8 +479,8 @@ __global__ void __launch_bounds__(256, 8) bp_stack_lat_kernel(VolG v, TiltG g, B
             // in float, the per-box loop's px0 + (i + 0.5) / OS of the same point)
             const int per = lw * lh, n = per * (k1 - k0 + 1);
             for (int idx = tid; idx < n; idx += 256) {
-                const int s = idx / per, rem = idx - s * per;
-                const int r = rem / lw, c = rem - r * lw;
+                const int s = small_div(idx, per), rem = idx - s * per;
+                const int r = small_div(rem, lw), c = rem - r * lw;
                 const float px = (float)tx0 + ((float)c + 0.5f) * kDelta, py = (float)ty0 + ((float)r + 0.5f) * kDelta;
                 tile[s * planeL + r * ls + c] =
                     tile_linear(stack + (size_t)(k0 + s) * stride, (int)pitch, 0, 0, W, H, px, py);

@@ -9,8 +9,9 @@
 // nothing, as in the per-box loop.  With the sub-ray offset (a, b) from the projection of the
 // voxel's min corner (detector pixels along u and v), the chord through the voxel is
 //     chord = max(0, min(m, P, SP - P, Y, SY - Y))
-// with P and Y affine in (a, b).  Evaluated as med3(min(SP/2 - |P - SP/2|, SY/2 - |Y - SY/2|), 0, m),
-// which is the same clamp (m > 0), in 8 operations per lattice point:
+// with P and Y affine in (a, b).  Only the ratio of two chord-weighted sums is used, so chords are taken in
+// units of m, as the product of clamp01(min(P, SP - P) / m) = clamp01(SP/2 - |P - SP/2|) in those units and
+// the y slab's inside test, itself the clamp of a huge coordinate:
 //   - n_x != 0: the x and z slabs' entries e_x, e_z are affine in (a, b) and the chord
 //     min(e_x + S_x, e_z + S_z) - max(e_x, e_z) equals min(min(S_x, S_z), S_x - d, S_z + d) for
 //     d = e_z - e_x; P = S_x - d, SP = S_x + S_z, m = min(S_x, S_z);
@@ -24,6 +25,7 @@
 #pragma once
 
 #include <cmath>
+#include <type_traits>
 
 #include "bp_common.hpp"
 #include "device_common.hpp"
@@ -37,10 +39,10 @@ constexpr float kWinFar = 1e36f;
 
 // Per-tilt constants of the window form, prepared on the host in double.
 struct BPWin {
-    float PU, PV, PC;        // Pc = P - SP/2 = a PU + b PV + PC
+    float PU, PV, PC;        // Pc = (P - SP/2) / m = a PU + b PV + PC
     float YU, YV, YC;        // Yc = Y - SY/2 = a YU + b YV + YC
     float PUd, PVd, YUd, YVd;   // the same per lattice step (times 1/OS)
-    float SPh, SYh, m;       // SP/2, SY/2, m
+    float SPh, SYh;          // SP/2 / m, SY/2
     float uMin, vMin;        // the voxel's projected box starts (with guard) relative to its corner
     double pu0, pui, puj, puk, pv0, pvi, pvj, pvk;   // corner projection (detector pixels)
     double G[2][3], lo[2], hi[2], tlo[2], thi[2];     // quad and block footprints (see BPExact)
@@ -78,22 +80,28 @@ inline bool prepare_window(const VolG& v, const TiltG& g, const BPExact& e, int 
     };
     double Uz, Vz, Sminz, Sabsz;
     slab(2, Uz, Vz, Sminz, Sabsz);
+    double PU, PV, PC, SP, m;
     if (std::fabs(n[0]) > 1e-6) {
         double Ux, Vx, Sminx, Sabsx;
         slab(0, Ux, Vx, Sminx, Sabsx);
         // P = S_x - d, d = e_z - e_x
-        w.PU = (float)(-(Uz - Ux));
-        w.PV = (float)(-(Vz - Vx));
-        w.PC = (float)((Sabsx - (Sminz - Sminx)) - 0.5 * (Sabsx + Sabsz));
-        w.SPh = (float)(0.5 * (Sabsx + Sabsz));
-        w.m = (float)std::fmin(Sabsx, Sabsz);
+        PU = -(Uz - Ux);
+        PV = -(Vz - Vx);
+        PC = (Sabsx - (Sminz - Sminx)) - 0.5 * (Sabsx + Sabsz);
+        SP = 0.5 * (Sabsx + Sabsz);
+        m = std::fmin(Sabsx, Sabsz);
     } else {
-        w.PU = (float)(B * u[0]);
-        w.PV = (float)(B * wv[0]);
-        w.PC = (float)(-0.5 * B * vs[0]);
-        w.SPh = (float)(0.5 * B * vs[0]);
-        w.m = (float)Sabsz;
+        PU = B * u[0];
+        PV = B * wv[0];
+        PC = -0.5 * B * vs[0];
+        SP = 0.5 * B * vs[0];
+        m = 1.0;   // (the clamp gives 0 or 1 whatever the unit)
     }
+    if (!(m > 0.0)) return false;
+    w.PU = (float)(PU / m);
+    w.PV = (float)(PV / m);
+    w.PC = (float)(PC / m);
+    w.SPh = (float)(SP / m);
     w.YU = (float)(B * u[1]);
     w.YV = (float)(B * wv[1]);
     w.YC = (float)(-0.5 * B * vs[1]);
@@ -167,12 +175,31 @@ inline bool gate_passes_all(const VolG& v, const BPWin& w, double distMin, doubl
     return true;
 }
 
+// The constants of a window in vector registers: a scalar operand halves the rate of an add or a multiply-add.
+struct WinRegs {
+    float SPh, SYh, PUd, PVd, YUd, YVd, PUd2, YUd2;
+    __device__ __forceinline__ explicit WinRegs(const BPWin& w)
+        : SPh(w.SPh), SYh(w.SYh), PUd(w.PUd), PVd(w.PVd), YUd(w.YUd), YVd(w.YVd), PUd2(2.0f * w.PUd), YUd2(2.0f * w.YUd) {
+        __asm__("" : "+v"(SPh), "+v"(SYh), "+v"(PUd), "+v"(PVd), "+v"(YUd), "+v"(YVd), "+v"(PUd2), "+v"(YUd2));
+    }
+    // x + d step, rounded once (step2: twice the step, which is exact)
+    __device__ __forceinline__ static float at(float x, int d, float step, float step2) {
+        return d == 0 ? x : (d == 1 ? x + step : (d == 2 ? x + step2 : __builtin_fmaf((float)d, step, x)));
+    }
+    __device__ __forceinline__ float px(float x, int d) const { return at(x, d, PUd, PUd2); }
+    __device__ __forceinline__ float yx(float x, int d) const { return at(x, d, YUd, YUd2); }
+    __device__ __forceinline__ float py(float x, int d) const { return d == 2 ? __builtin_fmaf(2.0f, PVd, x) : at(x, d, PVd, 0.0f); }
+    __device__ __forceinline__ float yy(float x, int d) const { return d == 2 ? __builtin_fmaf(2.0f, YVd, x) : at(x, d, YVd, 0.0f); }
+};
+
+__device__ __forceinline__ float clamp01(float x) { return __builtin_amdgcn_fmed3f(x, 0.0f, 1.0f); }
+
 // The chord-weighted sums of one voxel over its kNI x kNJ window, read from the block's LDS tile
-// of image pixels (row pitch tw).  (i0, j0): the window's first lattice point, global; (a0, b0):
-// its offset from the voxel's min-corner projection; tile origin pixel (tx0, ty0).  Only lattice
-// points in the quad footprint [li0, li1) x [lj0, lj1) count, which kMode applies as:
+// of image pixels (row pitch tw).  P0, Y0: Pc and Yc at the window's first lattice point, which lies in
+// tile pixel `base`, in its ph-th column and qh-th row of lattice points.  Only lattice points in the quad
+// footprint count: columns di with il + di < iw (unsigned), rows dj with jl + dj < jh, which kMode applies as:
 //   kWinOpen:   not at all (the footprint covers every voxel box: w.covers);
-//   kWinMasked: as a chord cap of 0 outside it (every window pixel lies in the tile);
+//   kWinMasked: by moving the point out of its slabs (every window pixel lies in the tile);
 //   kWinClamp:  by skipping the point and its read (blocks at the image edges).
 // The three give the same sums for finite images: a point outside adds fma(val, 0, n) = n.
 // kYCol: the y slab term does not change down a window column (YVd == 0: every tilt about y whose
@@ -181,61 +208,45 @@ inline bool gate_passes_all(const VolG& v, const BPWin& w, double distMin, doubl
 // or outside the footprint's columns) or a whole row (outside the footprint's rows) are skipped
 // with their reads.  The sums start at -0, the additive identity, so that the first point taken
 // adds what the window's first point would.
+//
+// VALU issue bounds the sums: a lattice point takes seven instructions of full rate (two coordinates,
+// two clamped differences, their product, the two sums) and its read; min and med3 in their place run at half.
+// 1024x1024x256 from 1024^2 pixels, 3 x 3 points: 0.96 -> 0.82 ms per tilt, 300 sub-volumes by 41 tilts 20.4 ->
+// 17.8 ms (with the four voxels of a quad in one branch and the tile's rows without integer division).
 constexpr int kWinOpen = 0, kWinMasked = 1, kWinClamp = 2;
 template <int kOS, int kNI, int kNJ, int kMode, bool kYCol = false>
-__device__ __forceinline__ void window_sums(const BPWin& w, const float* __restrict__ tile, int tw, int tx0, int ty0,
-                                            int i0, int j0, float a0, float b0, int li0, int li1, int lj0, int lj1,
+__device__ __forceinline__ void window_sums(const WinRegs& w, const float* __restrict__ tile, int tw, int base,
+                                            int ph, int qh, float P0, float Y0, int il, unsigned iw, int jl, unsigned jh,
                                             float& num, float& den) {
-    const float P0 = __builtin_fmaf(a0, w.PU, __builtin_fmaf(b0, w.PV, w.PC));
-    const float Y0 = __builtin_fmaf(a0, w.YU, __builtin_fmaf(b0, w.YV, w.YC));
-    // pixel of lattice point i: (i0 + di) / kOS = c0 + (ph + di) / kOS
-    const int c0 = kOS == 1 ? i0 : (i0 >> 1), ph = kOS == 1 ? 0 : (i0 & 1);
-    const int r0 = kOS == 1 ? j0 : (j0 >> 1), qh = kOS == 1 ? 0 : (j0 & 1);
-    // tile rows are small: 24-bit multiplies (full rate; the 32-bit one is a quarter)
-    const int base = __mul24(r0 - ty0, tw) + (c0 - tx0);
     const int qtw = qh ? tw : 0;
-    // masked: the chord cap of each window column (m inside the footprint's columns, else 0)
-    float cap[kNI];
-#pragma unroll
-    for (int di = 0; di < kNI; di++)
-        cap[di] = (kMode == kWinMasked && !((unsigned)(i0 + di - li0) < (unsigned)(li1 - li0))) ? 0.0f : w.m;
-    // kYCol: Yc = (Y0 + dj * 0) + di * YUd has the absolute value of Y0 + di * YUd at every point of
-    // column di; a chord is positive only where min(A, Bq) > 0 and the cap is positive
-    float Bcol[kNI];
+    // the window's columns: whether they count (in the footprint, and for kYCol in the y slab)
     bool live[kNI];
 #pragma unroll
-    for (int di = 0; di < kNI; di++) {
-        const float Yc = di == 0 ? Y0 : (di == 1 ? Y0 + w.YUd : __builtin_fmaf((float)di, w.YUd, Y0));
-        Bcol[di] = w.SYh - fabsf(Yc);
-        live[di] = Bcol[di] > 0.0f;
-        if (kMode != kWinOpen) live[di] = live[di] && (unsigned)(i0 + di - li0) < (unsigned)(li1 - li0);
-    }
+    for (int di = 0; di < kNI; di++)
+        live[di] = (kMode == kWinOpen || (unsigned)(il + di) < iw) && (!kYCol || w.SYh - fabsf(w.yx(Y0, di)) > 0.0f);
+    // masked: SP/2 of a column outside the footprint is below every |Pc|
+    float SPcol[kNI];
+#pragma unroll
+    for (int di = 0; di < kNI; di++) SPcol[di] = kMode == kWinMasked && !live[di] ? -1.0f : w.SPh;
     float n = kYCol ? -0.0f : 0.0f, d = kYCol ? -0.0f : 0.0f;
 #pragma unroll
     for (int dj = 0; dj < kNJ; dj++) {
-        const float Pr = dj == 0 ? P0 : (dj == 1 ? P0 + w.PVd : __builtin_fmaf((float)dj, w.PVd, P0));
-        float Yr = dj == 0 ? Y0 : (dj == 1 ? Y0 + w.YVd : __builtin_fmaf((float)dj, w.YVd, Y0));
-        const int rowOff = kOS == 1 ? dj * tw : (dj >> 1) * tw + ((dj & 1) ? qtw : 0);
-        const int rowBase = base + rowOff;
-        const int rowOdd = rowBase + ph;   // odd di of the 2x lattice: pixel c0 + ph + (di - 1) / 2
-        bool rowOk = true;
-        if (kMode != kWinOpen) rowOk = (unsigned)(j0 + dj - lj0) < (unsigned)(lj1 - lj0);
-        // masked: a row outside the footprint moves beyond every y slab, so its chords are 0 (the
-        // med3 of a negative value, 0 and the column cap), as a cap of 0 would make them
-        if (kMode == kWinMasked) Yr = rowOk ? Yr : kWinFar;
+        const bool rowOk = kMode == kWinOpen || (unsigned)(jl + dj) < jh;
         if (kYCol && !rowOk) continue;
+        const float Pr = w.py(P0, dj);
+        float Yr = w.yy(Y0, dj);
+        // masked: a row outside the footprint moves beyond every y slab
+        if (kMode == kWinMasked && !kYCol) Yr = rowOk ? Yr : kWinFar;
+        const int rowBase = base + (kOS == 1 ? dj * tw : (dj >> 1) * tw + ((dj & 1) ? qtw : 0));
+        const int rowOdd = rowBase + ph;   // odd di of the 2x lattice: pixel c0 + ph + (di - 1) / 2
 #pragma unroll
         for (int di = 0; di < kNI; di++) {
             if (kYCol && !live[di]) continue;
-            const float Pc = di == 0 ? Pr : (di == 1 ? Pr + w.PUd : __builtin_fmaf((float)di, w.PUd, Pr));
-            const float Yc = di == 0 ? Yr : (di == 1 ? Yr + w.YUd : __builtin_fmaf((float)di, w.YUd, Yr));
-            // min(m, P, SP - P, Y, SY - Y) clamped at 0 (cap 0: exactly 0)
-            const float A = w.SPh - fabsf(Pc), Bq = kYCol ? Bcol[di] : w.SYh - fabsf(Yc);
-            const float mcap = (kMode == kWinMasked && !kYCol) ? cap[di] : w.m;
-            float chord = __builtin_amdgcn_fmed3f(fminf(A, Bq), 0.0f, mcap);
+            const float A = clamp01((kMode == kWinMasked && !kYCol ? SPcol[di] : w.SPh) - fabsf(w.px(Pr, di)));
+            float chord = kYCol ? A : A * clamp01(w.SYh - fabsf(w.yx(Yr, di)));
             int addr = kOS == 1 ? rowBase + di : ((di & 1) ? rowOdd + (di >> 1) : rowBase + (di >> 1));
             if (kMode == kWinClamp && !kYCol) {
-                const bool ok = rowOk && (unsigned)(i0 + di - li0) < (unsigned)(li1 - li0);
+                const bool ok = rowOk && live[di];
                 chord = ok ? chord : 0.0f;
                 addr = ok ? addr : 0;
             }
@@ -303,35 +314,42 @@ __device__ __forceinline__ bool window_quad(const BPWin& w, const float* __restr
     const double Uq = fma(w.pui, qx, fma(w.puj, qy, fma(w.puk, qz, w.pu0)));
     const double Vq = fma(w.pvi, qx, fma(w.pvj, qy, fma(w.pvk, qz, w.pv0)));
     const double fUq = floor(Uq), fVq = floor(Vq);
-    const int iq = (int)fUq * kOS, jq = (int)fVq * kOS;
+    const int iq = (int)fUq, jq = (int)fVq;
     const float fu = (float)(Uq - fUq), fv = (float)(Vq - fVq);
     const float dui = (float)w.pui, dvi = (float)w.pvi;
+    const WinRegs r(w);
+    // tile rows are small: 24-bit multiplies (full rate; the 32-bit one is a quarter)
+    const int baseq = __mul24(jq - ty0, tw) + (iq - tx0);
+    const int ilq = iq * kOS - li0, jlq = jq * kOS - lj0;
     bool any = false;
+    const auto voxels = [&](auto mode_c) {
+        constexpr int kMode = decltype(mode_c)::value;
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-        const float du = __builtin_fmaf((float)k, dui, fu);
-        const float dv = __builtin_fmaf((float)k, dvi, fv);
-        // the window's first lattice point, as a float (an integer) and an int
-        const float fi0 = ceilf((du + w.uMin) * (float)kOS - 0.5f);
-        const float fj0 = ceilf((dv + w.vMin) * (float)kOS - 0.5f);
-        const int i0 = (int)fi0, j0 = (int)fj0;
-        const float a0 = __builtin_fmaf(fi0 + 0.5f, kDelta, -du);
-        const float b0 = __builtin_fmaf(fj0 + 0.5f, kDelta, -dv);
-        float num, den;
-        if (mode == kWinOpen)
-            window_sums<kOS, kNI, kNJ, kWinOpen, kYCol>(w, tile, tw, tx0, ty0, iq + i0, jq + j0, a0, b0, 0, 0, 0, 0, num,
-                                                 den);
-        else if (mode == kWinMasked)
-            window_sums<kOS, kNI, kNJ, kWinMasked, kYCol>(w, tile, tw, tx0, ty0, iq + i0, jq + j0, a0, b0, li0, li1, lj0,
-                                                   lj1, num, den);
-        else
-            window_sums<kOS, kNI, kNJ, kWinClamp, kYCol>(w, tile, tw, tx0, ty0, iq + i0, jq + j0, a0, b0, li0, li1, lj0,
-                                                  lj1, num, den);
-        if (den > 0.0f) {
-            out[k] += (lambda * num) * __builtin_amdgcn_rcpf(den);
-            any = true;
+        for (int k = 0; k < 4; k++) {
+            const float du = __builtin_fmaf((float)k, dui, fu);
+            const float dv = __builtin_fmaf((float)k, dvi, fv);
+            // the window's first lattice point, as a float (an integer) and an int
+            const float fi0 = ceilf((du + w.uMin) * (float)kOS - 0.5f), fj0 = ceilf((dv + w.vMin) * (float)kOS - 0.5f);
+            const int i0 = (int)fi0, j0 = (int)fj0;
+            const float a0 = __builtin_fmaf(fi0 + 0.5f, kDelta, -du), b0 = __builtin_fmaf(fj0 + 0.5f, kDelta, -dv);
+            const float P0 = __builtin_fmaf(a0, w.PU, __builtin_fmaf(b0, w.PV, w.PC));
+            const float Y0 = __builtin_fmaf(a0, w.YU, __builtin_fmaf(b0, w.YV, w.YC));
+            // pixel of lattice point i: floor(i / kOS)
+            const int base = kOS == 1 ? __mul24(j0, tw) + i0 + baseq : __mul24(j0 >> 1, tw) + (i0 >> 1) + baseq;
+            const int ph = kOS == 1 ? 0 : (i0 & 1), qh = kOS == 1 ? 0 : (j0 & 1);
+            float num, den;
+            window_sums<kOS, kNI, kNJ, kMode, kYCol>(r, tile, tw, base, ph, qh, P0, Y0, ilq + i0, (unsigned)(li1 - li0),
+                                                     jlq + j0, (unsigned)(lj1 - lj0), num, den);
+            if (den > 0.0f) {
+                out[k] += (lambda * num) * __builtin_amdgcn_rcpf(den);
+                any = true;
+            }
         }
-    }
+    };
+    // (the branch around the four voxels, so that their reads overlap)
+    if (mode == kWinOpen) voxels(std::integral_constant<int, kWinOpen>());
+    else if (mode == kWinMasked) voxels(std::integral_constant<int, kWinMasked>());
+    else voxels(std::integral_constant<int, kWinClamp>());
     return any;
 }
 

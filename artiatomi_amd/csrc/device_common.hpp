@@ -13,6 +13,11 @@ namespace artia {
 
 // clamp to [lo, hi] (lo <= hi): one v_med3_i32
 __device__ __forceinline__ int clampi(int i, int lo, int hi) { return min(max(i, lo), hi); }
+// a / b for 0 <= a < 2^20 and b >= 1 (an integer division takes some 35 instructions): (a + 1/2) / b lies at
+// least 1 / (2 b) from an integer, and the reciprocal, its product and the sum err by less than 2^-22 a / b.
+__device__ __forceinline__ int small_div(int a, int b) {
+    return (int)(((float)a + 0.5f) * __builtin_amdgcn_rcpf((float)b));
+}
 __device__ __forceinline__ float lerpf(float p, float q, float w) { return __builtin_fmaf(w, q - p, p); }
 
 // Volume element types: fp32, or IEEE binary16, the reference's FP16Volume storage (a half-float

@@ -205,12 +205,6 @@ __device__ __forceinline__ FlatBox flat_box(const VolG& v, const TubePlan& tp, c
     return q;
 }
 
-// a / b for 0 <= a < 2^12 and 1 <= b <= 2^12: (a + 1/2) / b lies at least 1 / 2^13 from an integer, far more
-// than the rounding of one reciprocal.
-__device__ __forceinline__ int small_div(int a, int b) {
-    return (int)(((float)a + 0.5f) * __builtin_amdgcn_rcpf((float)b));
-}
-
 // A box is staged by columns along z: a thread keeps (x, y) columns t, t + 256, .. (one for most tilts) and
 // loads their layers, whose base addresses are uniform: a lane offset that stays fixed and one LDS
 // address step per voxel, with the clamps once per column (x, y) or in scalar registers (z).

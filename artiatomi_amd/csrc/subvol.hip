@@ -251,8 +251,8 @@ __global__ void __launch_bounds__(256, 6) subvol_bp_kernel(const Item* __restric
                 if (tiled) {
                     const int n = plane * (k1 - k0 + 1);
                     for (int idx = tid; idx < n; idx += 256) {
-                        const int sl = idx / plane, rem = idx - sl * plane;
-                        const int r = rem / tw, c = rem - r * tw;
+                        const int sl = small_div(idx, plane), rem = idx - sl * plane;
+                        const int r = small_div(rem, tw), c = rem - r * tw;
                         tile[idx] = img[(size_t)(k0 + sl) * imgStride + (size_t)(ty0 + r) * pitch + (size_t)(tx0 + c)];
                     }
                     __syncthreads();
@@ -308,7 +308,7 @@ __global__ void __launch_bounds__(256, 6) subvol_bp_kernel(const Item* __restric
                 const int ts = (tw | 1) * th <= kTileFloats ? (tw | 1) : tw;
                 if (useTile) {
                     for (int idx = tid; idx < tw * th; idx += 256) {
-                        const int r = idx / tw, c = idx - r * tw;
+                        const int r = small_div(idx, tw), c = idx - r * tw;
                         tile[r * ts + c] = img[(size_t)(ty0 + r) * pitch + (size_t)(tx0 + c)];
                     }
                     __syncthreads();
@@ -329,7 +329,7 @@ __global__ void __launch_bounds__(256, 6) subvol_bp_kernel(const Item* __restric
             }
             if (useTile) {
                 for (int idx = tid; idx < tw * th; idx += 256) {
-                    const int r = idx / tw, c = idx - r * tw;
+                    const int r = small_div(idx, tw), c = idx - r * tw;
                     tile[idx] = img[(size_t)(ty0 + r) * pitch + (size_t)(tx0 + c)];
                 }
                 __syncthreads();
