@@ -349,9 +349,11 @@ __global__ void __launch_bounds__(256) pair_adjoint_slab_kernel(PairArgs a, AdjS
 // slab sets every sub-ray of every tilt up again for each slab, 65 times for 64 layers).  The rows'
 // voxel planes are in LDS in double, padded by the clamp border, and reach the gradient with one atomic
 // per voxel and run.  Lanes run along the detector axis on which y changes less: a wave's rays lie a
-// pixel apart in one row and rarely add to one voxel at once.  100 cubes of 64^3 by 41 tilts: 22 ms,
-// against 156 ms with z slabs and eight additions per cell.
-constexpr int kAdjFlatThreads = 512;
+// pixel apart in one row and rarely add to one voxel at once.  The planes leave room for one workgroup on a
+// compute unit, so it has sixteen waves to cover the LDS additions (a wave's ds_add_f64 takes nine cycles).
+// 100 cubes of 64^3 by 41 tilts: 19.7 ms (22.2 with eight waves), against 156 ms with z slabs and eight
+// additions per cell.
+constexpr int kAdjFlatThreads = 1024;
 constexpr int kAdjFlatBytes = 144 << 10;   // LDS for the padded planes
 constexpr int kAdjFlatPlanes = 8;          // at most
 
