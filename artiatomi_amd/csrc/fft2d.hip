@@ -346,7 +346,7 @@ template <int N, int kKind>
 __global__ void __launch_bounds__(Shape<N>::threads, 4) cols_kernel(const float2* __restrict__ tw,
                                                                const float2* __restrict__ base,
                                                                float2* __restrict__ spec, size_t zstride, CtfStack ctf,
-                                                               PrepFilter pf) {
+                                                               PrepFilter pf, const uint32_t* need) {
     constexpr int E = Shape<N>::E, T = Shape<N>::T, P = Shape<N>::pairs;
     __shared__ C2 lds[2 * P * padded(N)];
     // lanes alternate between the two columns of a pair, whose values alternate in memory
@@ -417,7 +417,13 @@ __global__ void __launch_bounds__(Shape<N>::threads, 4) cols_kernel(const float2
         uint32_t off2 = off;
         __asm__ volatile("" : "+v"(off2));
 #pragma unroll
-        for (int i = 0; i < E; i++) store_at(out, off2 + (uint32_t)(16 * T * i), make_float2(v[i].x, v[i].y));
+        for (int i = 0; i < E; i++) {
+            if (kKind == kColFan && need) {   // uniform
+                const int ky = t + T * i;
+                if (!((need[(size_t)z * (N / 32) + (ky >> 5)] >> (ky & 31)) & 1u)) continue;
+            }
+            store_at(out, off2 + (uint32_t)(16 * T * i), make_float2(v[i].x, v[i].y));
+        }
     }
 }
 
@@ -472,6 +478,13 @@ __global__ void __launch_bounds__(Shape<N>::threads, 4) rows_back_kernel(const f
     const int y0 = (int)blockIdx.x * Shape<N>::rows, y = y0 + 2 * f - d.by;
     C2 v[E];
     const int z = (int)blockIdx.y;
+    if (kKind == kDstStore && d.need) {   // uniform
+        constexpr int R = Shape<N>::rows, step = R < 32 ? R : 32;
+        uint32_t any = 0;
+        for (int r = 0; r < R; r += step)
+            any |= (d.need[(size_t)z * (N / 32) + ((y0 + r) >> 5)] >> ((y0 + r) & 31)) & (step == 32 ? ~0u : (1u << (step & 31)) - 1u);
+        if (!any) return;   // whole workgroup
+    }
     rows_back<N>(tw, spec + (size_t)z * zstride, y0, f, t, lds, v);
     float* out = d.out + (size_t)z * d.stride;
     double s1 = 0.0, s2 = 0.0;
@@ -545,11 +558,11 @@ void launch_rows_forward(artia_ctx* ctx, int N, const float2* tw, const RowSrc& 
 }
 template <int kKind>
 void launch_cols(artia_ctx* ctx, int N, const float2* tw, const float2* base, float2* spec, const CtfStack& c,
-                 const PrepFilter& f, int nz) {
+                 const PrepFilter& f, int nz, const uint32_t* need = nullptr) {
     with_length(N, [&](auto n) {
         constexpr int L = decltype(n)::value;
         hipLaunchKernelGGL((cols_kernel<L, kKind>), dim3((L / 4 + Shape<L>::pairs) / Shape<L>::pairs, (unsigned)nz),
-                           dim3(Shape<L>::threads), 0, ctx->stream, tw, base, spec, fft2d_spec_size(L), c, f);
+                           dim3(Shape<L>::threads), 0, ctx->stream, tw, base, spec, fft2d_spec_size(L), c, f, need);
     });
 }
 template <int kKind>
@@ -584,8 +597,8 @@ void fft2d_cols_ctf(artia_ctx* ctx, int N, const float2* tw, float2* spec, const
     launch_cols<kColCtf>(ctx, N, tw, nullptr, spec, c, PrepFilter{}, nz);
 }
 void fft2d_cols_fan(artia_ctx* ctx, int N, const float2* tw, const float2* base, float2* spec, const CtfStack& c,
-                    int nz) {
-    launch_cols<kColFan>(ctx, N, tw, base, spec, c, PrepFilter{}, nz);
+                    int nz, const uint32_t* need) {
+    launch_cols<kColFan>(ctx, N, tw, base, spec, c, PrepFilter{}, nz, need);
 }
 void fft2d_cols_prep(artia_ctx* ctx, int N, const float2* tw, float2* spec, const PrepFilter& f, int nz) {
     launch_cols<kColPrep>(ctx, N, tw, nullptr, spec, CtfStack{}, f, nz);

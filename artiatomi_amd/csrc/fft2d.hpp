@@ -45,8 +45,9 @@ struct RowDst {
     float* out;
     size_t pitch, stride;
     const float* weight;   // as RowSrc's
-    // kStore: out[z * stride] = w v (accumulate: += )
+    // kStore: out[z * stride] = w v (accumulate: += ), rows in need
     int accumulate;
+    const uint32_t* need;
     // kPrep: out = v, and the double sums of v - c and (v - c)^2 over the region [rx0, rx0 + rw) x
     // [ry0, ry0 + rh), c = dc[z] * scale (the square's mean), per block: partial[2 * (z * blocks + block)]
     int rx0, ry0, rw, rh;
@@ -59,13 +60,16 @@ int fft2d_row_blocks(int N);   // blocks per image of the row kernels
 // spec[z] = half spectrum rows of image z (not yet transformed along the columns)
 void fft2d_rows_square(artia_ctx* ctx, int N, const float2* tw, const RowSrc& s, float2* spec, int nz);
 void fft2d_rows_prep(artia_ctx* ctx, int N, const float2* tw, const RowSrc& s, float2* spec, int nz);
+// Rows of the stack's images that are wanted: bit y % 32 of word y / 32 of image z at need + z * N / 32, whole
+// row blocks (fft2d_row_blocks) at a time; null: all.  The others are neither written by the columns nor
+// transformed.
 // columns: forward only (in place)
 void fft2d_cols_forward(artia_ctx* ctx, int N, const float2* tw, float2* spec, int nz);
 // forward, CTF of slab z, back (in place)
 void fft2d_cols_ctf(artia_ctx* ctx, int N, const float2* tw, float2* spec, const CtfStack& c, int nz);
 // spec[z] = back(base * CTF of slab z), base transformed along the columns
 void fft2d_cols_fan(artia_ctx* ctx, int N, const float2* tw, const float2* base, float2* spec, const CtfStack& c,
-                    int nz);
+                    int nz, const uint32_t* need = nullptr);
 // forward, projection preparation's filters, back (in place)
 void fft2d_cols_prep(artia_ctx* ctx, int N, const float2* tw, float2* spec, const PrepFilter& f, int nz);
 // rows back: each image stored (or added), or the preparation's store

@@ -330,7 +330,7 @@ RowDst square_target(float* out, size_t stride, int W, int H, size_t pitch, int 
 artia_status ctf_filter_slabs_own(artia_ctx* ctx, const float* src, size_t src_stride, int n, int W, int H, size_t pitch,
                                   float* out, size_t out_stride, const int corners[8], const float cut[2],
                                   const float dim[2], const artia_ctf_params& p, const float* dmin_nm,
-                                  const float* dmax_nm, float angle_deg, int forFP) {
+                                  const float* dmax_nm, float angle_deg, int forFP, const uint32_t* need) {
     const int N = W > H ? W : H;
     FftOwn& f = ctx->ffto;
     artia_status st = f.ensure(ctx, N);
@@ -354,7 +354,7 @@ artia_status ctf_filter_slabs_own(artia_ctx* ctx, const float* src, size_t src_s
         const int b = std::min(f.cap, n - k0);
         const CtfStack cs = make_ctf_stack(N, p, dmin_nm + k0, dmax_nm + k0, angle_deg, forFP, b);
         if (shared) {
-            fft2d_cols_fan(ctx, N, f.tw, base, f.spec, cs, b);
+            fft2d_cols_fan(ctx, N, f.tw, base, f.spec, cs, b, need);
         } else {
             s.src = src + (size_t)k0 * src_stride;
             s.weight = weight;
@@ -368,9 +368,12 @@ artia_status ctf_filter_slabs_own(artia_ctx* ctx, const float* src, size_t src_s
             fft2d_rows_store(ctx, N, f.tw, f.spec, square_target(f.images, plane, W, H, (size_t)W, N, weight, 0), b);
             hipLaunchKernelGGL(sum_images_kernel, grid2d(W, H), dim3(64, 4), 0, ctx->stream, f.images, plane, b, W, H, out,
                                pitch);
-        } else
-            fft2d_rows_store(ctx, N, f.tw, f.spec,
-                             square_target(out + (size_t)k0 * out_stride, out_stride, W, H, pitch, N, weight, 0), b);
+        } else {
+            RowDst d = square_target(out + (size_t)k0 * out_stride, out_stride, W, H, pitch, N, weight, 0);
+            d.need = shared ? need : nullptr;
+            fft2d_rows_store(ctx, N, f.tw, f.spec, d, b);
+            if (need) need += (size_t)b * (size_t)(N / 32);
+        }
         if ((st = check_hip(ctx, hipGetLastError(), "stacked slab filter")) != ARTIA_OK) return st;
     }
     return ARTIA_OK;
@@ -582,15 +585,20 @@ artia_status ctf_slab_filter(artia_ctx* ctx, float* img, int W, int H, size_t pi
     return check_hip(ctx, hipGetLastError(), "slab filter");
 }
 
+int slab_row_block(int W, int H) {
+    const int N = W > H ? W : H;
+    return fft2d_supports(N) ? N / fft2d_row_blocks(N) : 0;
+}
+
 artia_status ctf_filter_slabs(artia_ctx* ctx, const float* src, size_t src_stride, int n, int W, int H, size_t pitch,
                               float* out, size_t out_stride, const int corners[8], const float cut[2],
                               const float dim[2], const artia_ctf_params& p, const float* dmin_nm,
-                              const float* dmax_nm, float angle_deg, int forFP) {
+                              const float* dmax_nm, float angle_deg, int forFP, const uint32_t* need) {
     if (n <= 0) return ARTIA_OK;
     const int N = W > H ? W : H;
     if (fft2d_supports(N) && fft2d_fits(H, pitch))
         return ctf_filter_slabs_own(ctx, src, src_stride, n, W, H, pitch, out, out_stride, corners, cut, dim, p, dmin_nm,
-                                    dmax_nm, angle_deg, forFP);
+                                    dmax_nm, angle_deg, forFP, need);
     FftBatch& fb = ctx->fftb;
     artia_status st = fb.ensure(ctx, N);
     if (st != ARTIA_OK) return st;

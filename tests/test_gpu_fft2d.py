@@ -127,3 +127,33 @@ def test_prepare(ctx, name, W, H):
         m1, s1, b1 = ctx.prepare_projections(pp, d_in[i:i + 1].contiguous(), one, psi_deg=psis[i:i + 1],
                                              dose=doses[i:i + 1])
         assert torch.equal(one[0], out[i]) and (m1[0], s1[0], b1[0]) == (mean[i], std[i], bad[i])
+
+
+@pytest.mark.parametrize("W,H", [(256, 256), (1024, 777), (600, 2048)])
+def test_subvolume_plan_filters_the_rows_it_reads(ctx, W, H):
+    """A CTF plan transforms only the rows of the slab images that its sub-volumes read: the same voxels as
+    one whole-image filter per slab, for cubes inside, across and beyond the detector's edges."""
+    print(f"sub-volume rows {W} x {H}", flush=True)
+    full = A.volume_geometry(W - W % 4, H, 96)
+    tilts, rng = [-50.0, 0.0, 33.0], np.random.default_rng(7)
+    ctf = A.ctf_params(pixelsize_nm=0.5, slice_thickness_nm=9.3, beta_fac=(2.0, 0.0, 0.008, 0.0), amp_contrast=0.07)
+    base = [A.tilt_geometry(t, W, H, psi_deg=4.0, shift=(1.0, -2.0)) for t in tilts]
+    kw = dict(ctf=ctf, slab_ranges=[A.defocus_distances(full, g) for g in base],
+              defocus=[A.TiltDefocus(3000.0, 3200.0, 15.0, t) for t in tilts])
+    geo, geoms = [], []
+    for n, x, y, z in ((16, 0.5, 0.5, 0.5), (32, 0.2, 0.9, 0.4), (24, 0.0, 0.02, 0.6), (16, 0.7, 1.0, 0.1), (8, 1.2, 1.3, 0.5)):
+        geo.append(A.subvolume_geometry(n, 1.0, (1.0, 1.0, 1.0), full, (x * W + 1.0, y * H + 1.0, z * 96 + 1.0)))
+        geoms.append([A.subvolume_tilt_geometry(t, W, H, psi_deg=4.0, shift=(1.0, -2.0),
+                                                extra_shift=rng.uniform(-2.0, 2.0, 2)) for t in tilts])
+    active = np.ones((len(geo), len(tilts)), bool)
+    active[0, 1] = False
+    images = torch.from_numpy(np.stack([white(H, W, i) for i in range(len(tilts))])).cuda()
+    sets = [[(g, torch.zeros((g.nz, g.ny, g.nx), device="cuda")) for g in geo] for _ in range(2)]
+    A.subvol_wbp_plain(ctx, sets[0], geoms, images, 2, active=active, **kw)
+    plan = A.SubvolPlan(ctx, sets[1], geoms, images, 2, active=active, tuning=A.SubvolTuning(0, 0, 1, 2), **kw)
+    plan.execute()
+    torch.cuda.synchronize()
+    plan.close()
+    assert float(sets[0][0][1].abs().max()) > 0   # (some of the others miss a narrow detector)
+    for (_, a), (_, b) in zip(*sets):
+        assert torch.equal(a, b)
