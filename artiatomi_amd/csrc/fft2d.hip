@@ -376,6 +376,7 @@ __global__ void __launch_bounds__(Shape<N>::threads, 4) cols_kernel(const float2
             for (int i = 0; i < E; i++) mine[slot<2>(t + T * i)] = v[i];
         }
         const bool steps = kKind != kColPrep && !ctf.k.phaseFlip && ctf.k.beta[1] == 0.0f && ctf.k.beta[3] == 0.0f;
+        double power = 0.0;
 #pragma unroll 1
         for (int half = 0; half < 2; half++) {   // frequencies >= 0 and < 0
             CtfEnvelopeRun env{0.0, 0.0, 0.0};
@@ -393,6 +394,7 @@ __global__ void __launch_bounds__(Shape<N>::threads, 4) cols_kernel(const float2
                 if (kKind == kColPrep) {
                     r = prep_factor(r, kx, ky, N, pf, z);
                     if (pf.dc && kx == 0 && ky == 0) pf.dc[z] = r.x;
+                    else power = __builtin_fma((double)r.x, (double)r.x, __builtin_fma((double)r.y, (double)r.y, power));
                 } else {
                     const CtfPoint pt = steps ? ctf_point(kx, ky, ctf.k, env.e) : ctf_point(kx, ky, ctf.k);
                     r = ctf_apply_at(r, pt, ctf.k, ctf.def0[z], ctf.def1[z]);
@@ -400,6 +402,14 @@ __global__ void __launch_bounds__(Shape<N>::threads, 4) cols_kernel(const float2
                 }
                 *at = C2{r.x, r.y};
             }
+        }
+        if (kKind == kColPrep && pf.power) {   // uniform
+            // columns 1 .. N / 2 - 1 stand for their mirror images too; the last pair's second is not used
+            power = own && kx <= N / 2 ? (kx == 0 || kx == N / 2 ? power : 2.0 * power) : 0.0;
+            for (int o = 32; o > 0; o >>= 1) power += __shfl_down(power, o);
+            constexpr int waves = Shape<N>::threads / 64;
+            if ((threadIdx.x & 63) == 0)
+                pf.power[((size_t)z * gridDim.x + blockIdx.x) * waves + (threadIdx.x >> 6)] = power;
         }
 #pragma unroll
         for (int i = 0; i < E; i++) v[i] = mine[slot<2>(t + T * i)];
@@ -498,6 +508,10 @@ __global__ void __launch_bounds__(Shape<N>::threads, 4) rows_back_kernel(const f
             float val = (q ? v[i].y : v[i].x) * d.scale;
             const uint32_t at = ((uint32_t)(y + q) * (uint32_t)d.pitch + (uint32_t)x) * 4u;
             if (kKind == kDstStore) {
+                if (d.st) {   // uniform
+                    val = val - d.st[z].mean_hf;
+                    val = val / -d.st[z].std_hf;
+                }
                 if (d.weight)
                     val = load_at<float>(d.weight, (uint32_t)((y0 + 2 * f + q) * N + t + T * i) * 4u) * val;
                 store_at(out, at, d.accumulate ? load_at<float>(out, at) + val : val);
@@ -581,6 +595,15 @@ bool fft2d_supports(int N) { return N >= 128 && N <= 4096 && (N & (N - 1)) == 0;
 int fft2d_row_blocks(int N) {
     int n = 0;
     with_length(N, [&](auto l) { n = decltype(l)::value / Shape<decltype(l)::value>::rows; });
+    return n;
+}
+
+int fft2d_col_waves(int N) {
+    int n = 0;
+    with_length(N, [&](auto l) {
+        constexpr int L = decltype(l)::value;
+        n = (L / 4 + Shape<L>::pairs) / Shape<L>::pairs * (Shape<L>::threads / 64);
+    });
     return n;
 }
 

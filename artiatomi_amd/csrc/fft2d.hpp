@@ -45,8 +45,9 @@ struct RowDst {
     float* out;
     size_t pitch, stride;
     const float* weight;   // as RowSrc's
-    // kStore: out[z * stride] = w v (accumulate: += ), rows in need
+    // kStore: out[z * stride] = w v (accumulate: += ), rows in need; with st the preparation's normalisation of v
     int accumulate;
+    const PrepStat* st;
     const uint32_t* need;
     // kPrep: out = v, and the double sums of v - c and (v - c)^2 over the region [rx0, rx0 + rw) x
     // [ry0, ry0 + rh), c = dc[z] * scale (the square's mean), per block: partial[2 * (z * blocks + block)]
@@ -56,6 +57,7 @@ struct RowDst {
 };
 
 int fft2d_row_blocks(int N);   // blocks per image of the row kernels
+int fft2d_col_waves(int N);    // waves per image of the column kernels
 
 // spec[z] = half spectrum rows of image z (not yet transformed along the columns)
 void fft2d_rows_square(artia_ctx* ctx, int N, const float2* tw, const RowSrc& s, float2* spec, int nz);

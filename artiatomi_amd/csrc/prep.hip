@@ -221,6 +221,22 @@ __global__ void __launch_bounds__(256) row_stats_finish_kernel(const double* __r
     }
 }
 
+// The statistics of a filtered N x N image from its spectrum: the mean from frequency 0 and the variance from
+// the other squares (Parseval).
+__global__ void __launch_bounds__(256) spectrum_stats_kernel(const double* __restrict__ power, int waves, int N,
+                                                             const float* __restrict__ dc, float scale,
+                                                             PrepStat* __restrict__ st) {
+    __shared__ double sh[256];
+    const int z = (int)blockIdx.x;
+    double a = 0.0;
+    for (int w = (int)threadIdx.x; w < waves; w += 256) a += power[(size_t)z * waves + w];
+    const double s = block_sum(a, sh);
+    if (threadIdx.x == 0) {
+        st[z].mean = (double)(dc[z] * scale);
+        st[z].std = sqrt(s) * (double)scale;
+    }
+}
+
 template <class T>
 void launch_raw_sums(artia_ctx* ctx, const RowSrc& s, int N, int pass, double* partial, int b) {
     hipLaunchKernelGGL(raw_sums_kernel<T>, dim3(kRedBlocks, (unsigned)b), dim3(256), 0, ctx->stream,
@@ -307,8 +323,15 @@ artia_status artia_prepare_projections(artia_ctx* ctx, const artia_prep_params* 
     artia_status st = own ? fo.ensure(ctx, N) : fb.ensure(ctx, N);
     if (st != ARTIA_OK) return st;
     const int cap = own ? fo.cap : fb.cap, rowBlocks = own ? fft2d_row_blocks(N) : 0;
+    // The normalisation of a whole square's mean and deviation needs no pass over the image: both come from the
+    // spectrum, and the pixels are normalised as they are stored (31 images of 4096 x 4096: 5.4 -> 4.7 ms).
+    // Not with a high pass and the mean as divisor, where a frequency 0 filtered to nothing would be divided by.
+    const bool fromSpectrum = own && !pp->wbp && width == N && height == N &&
+                              (pp->normalization == ARTIA_NORM_STD ||
+                               (pp->normalization == ARTIA_NORM_MEAN && (pp->skip_filter || !(pp->hp > 0.0f))));
+    const int waves = fromSpectrum ? fft2d_col_waves(N) : 0;
     // workspace: partial sums of a chunk, then the per-projection state and, behind it, the squares' means
-    const size_t partFloats = (size_t)cap * (size_t)std::max(kRedBlocks, 2 * rowBlocks) * 2;
+    const size_t partFloats = (size_t)cap * (size_t)std::max(kRedBlocks, std::max(2 * rowBlocks, waves)) * 2;
     const size_t statFloats = ((size_t)n * sizeof(PrepStat) + sizeof(float) - 1) / sizeof(float);
     if ((st = ensure_workspace(ctx, partFloats + statFloats + 2 + kFftBatchMax)) != ARTIA_OK) return st;
     double* partial = reinterpret_cast<double*>(ctx->ws);
@@ -384,6 +407,7 @@ artia_status artia_prepare_projections(artia_ctx* ctx, const artia_prep_params* 
                 }
             }
             f.dc = d_dc;
+            f.power = fromSpectrum ? partial : nullptr;
             fft2d_rows_prep(ctx, N, fo.tw, r, fo.spec, b);
             fft2d_cols_prep(ctx, N, fo.tw, fo.spec, f, b);
             RowDst d{};
@@ -396,6 +420,13 @@ artia_status artia_prepare_projections(artia_ctx* ctx, const artia_prep_params* 
             d.pitch = out_pitch;
             d.stride = ostride;
             if (pp->wbp) {
+                fft2d_rows_store(ctx, N, fo.tw, fo.spec, d, b);
+            } else if (fromSpectrum) {
+                hipLaunchKernelGGL(spectrum_stats_kernel, dim3((unsigned)b), dim3(256), 0, ctx->stream, partial, waves, N,
+                                   d_dc, d.scale, s);
+                hipLaunchKernelGGL(norm_params_kernel, dim3((unsigned)((b + 63) / 64)), dim3(64), 0, ctx->stream, s, b, 0,
+                                   pp->normalization, 0);
+                d.st = s;
                 fft2d_rows_store(ctx, N, fo.tw, fo.spec, d, b);
             } else {
                 d.rx0 = rx0;

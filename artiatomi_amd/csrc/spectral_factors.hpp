@@ -176,6 +176,9 @@ struct PrepFilter {
     int wbp, method;                                  // exact-numerics WBP weighting (method as artia_wbp_weight)
     double sn[kFftBatchMax], cs[kFftBatchMax];        // of each image's angle
     const PrepStat* st;
+    // out (or null): each wave's sum of the filtered spectrum's squares over both half planes, without frequency 0
+    // (fft2d_col_waves(N) an image)
+    double* power;
     float* dc;                                        // out (or null): image z's filtered value at frequency 0
 };
 
