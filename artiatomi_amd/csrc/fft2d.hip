@@ -261,22 +261,6 @@ __device__ __forceinline__ void load_raw_rows(const RowSrc& s, int t, int y, int
     }
 }
 
-// a raw pixel's bad value replaced, and its normalisation
-__device__ __forceinline__ float prep_pixel(const RowSrc& s, const PrepStat& st, float v, int& bad) {
-    if (s.correct) {
-        const float mean = (float)st.sq_mean;
-        if (v > s.bad_value * mean) {
-            v = mean;
-            bad++;
-        }
-    }
-    if (s.norm) {
-        v = v - st.mean_hf;
-        v = v / -st.std_hf;
-    }
-    return v;
-}
-
 template <int N, int kKind>
 __global__ void __launch_bounds__(Shape<N>::threads, 4) rows_forward_kernel(const float2* __restrict__ tw, RowSrc s,
                                                                        float2* __restrict__ spec, size_t zstride) {

@@ -38,6 +38,22 @@ struct RowSrc {
     PrepStat* st;
 };
 
+// a raw pixel's bad value replaced, and its normalisation
+__device__ __forceinline__ float prep_pixel(const RowSrc& s, const PrepStat& st, float v, int& bad) {
+    if (s.correct) {
+        const float mean = (float)st.sq_mean;
+        if (v > s.bad_value * mean) {
+            v = mean;
+            bad++;
+        }
+    }
+    if (s.norm) {
+        v = v - st.mean_hf;
+        v = v / -st.std_hf;
+    }
+    return v;
+}
+
 // What the backward row kernel does with image pixel (x, y) of image z: v = value * scale, then
 struct RowDst {
     int W, H, bx, by;
