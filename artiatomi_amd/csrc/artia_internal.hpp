@@ -201,12 +201,13 @@ artia_status ctf_slab_filter(artia_ctx* ctx, float* img, int W, int H, size_t pi
 // corners == nullptr: no border crop (the sub-volume WBP's slab filter)
 // need (forFP = 0; the three-kernel filter's sizes, otherwise ignored): the rows of slab s's image that the
 // caller reads, bit y % 32 of word y / 32 at need + s * N / 32 (rows of the square, whole blocks of
-// slab_row_block(W, H) rows); the rest of out is undefined
+// slab_row_block(W, H) rows); the rest of out is undefined.  wanted (host): 0 for a slab without such rows
 int slab_row_block(int W, int H);   // 0: the size's filter takes no rows
 artia_status ctf_filter_slabs(artia_ctx* ctx, const float* src, size_t src_stride, int n, int W, int H, size_t pitch,
                               float* out, size_t out_stride, const int corners[8], const float cut[2],
                               const float dim[2], const artia_ctf_params& p, const float* dmin_nm,
-                              const float* dmax_nm, float angle_deg, int forFP, const uint32_t* need = nullptr);
+                              const float* dmax_nm, float angle_deg, int forFP, const uint32_t* need = nullptr,
+                              const unsigned char* wanted = nullptr);
 // makeSquare (reflect) -> R2C -> wbpWeighting -> C2R -> out = square / N^2
 artia_status wbp_filter(artia_ctx* ctx, const float* img, int W, int H, size_t pitch, float* out, size_t out_pitch,
                         float psi_deg, int method);

@@ -330,12 +330,13 @@ template <int N, int kKind>
 __global__ void __launch_bounds__(Shape<N>::threads, 4) cols_kernel(const float2* __restrict__ tw,
                                                                const float2* __restrict__ base,
                                                                float2* __restrict__ spec, size_t zstride, CtfStack ctf,
-                                                               PrepFilter pf, const uint32_t* need) {
+                                                               PrepFilter pf, const uint32_t* need, uint32_t wanted) {
     constexpr int E = Shape<N>::E, T = Shape<N>::T, P = Shape<N>::pairs;
     __shared__ C2 lds[2 * P * padded(N)];
     // lanes alternate between the two columns of a pair, whose values alternate in memory
     const int g = (int)threadIdx.x / (2 * T), u = (int)threadIdx.x % (2 * T), h = u & 1, t = u >> 1;
     const int z = (int)blockIdx.y;
+    if (kKind == kColFan && !((wanted >> z) & 1u)) return;   // whole workgroup
     const int p = min((int)blockIdx.x * P + g, N / 4);   // (the last block repeats the last pair)
     const bool own = (int)blockIdx.x * P + g <= N / 4;
     const int kx = 2 * p + h;
@@ -556,11 +557,11 @@ void launch_rows_forward(artia_ctx* ctx, int N, const float2* tw, const RowSrc& 
 }
 template <int kKind>
 void launch_cols(artia_ctx* ctx, int N, const float2* tw, const float2* base, float2* spec, const CtfStack& c,
-                 const PrepFilter& f, int nz, const uint32_t* need = nullptr) {
+                 const PrepFilter& f, int nz, const uint32_t* need = nullptr, uint32_t wanted = ~0u) {
     with_length(N, [&](auto n) {
         constexpr int L = decltype(n)::value;
         hipLaunchKernelGGL((cols_kernel<L, kKind>), dim3((L / 4 + Shape<L>::pairs) / Shape<L>::pairs, (unsigned)nz),
-                           dim3(Shape<L>::threads), 0, ctx->stream, tw, base, spec, fft2d_spec_size(L), c, f, need);
+                           dim3(Shape<L>::threads), 0, ctx->stream, tw, base, spec, fft2d_spec_size(L), c, f, need, wanted);
     });
 }
 template <int kKind>
@@ -604,8 +605,8 @@ void fft2d_cols_ctf(artia_ctx* ctx, int N, const float2* tw, float2* spec, const
     launch_cols<kColCtf>(ctx, N, tw, nullptr, spec, c, PrepFilter{}, nz);
 }
 void fft2d_cols_fan(artia_ctx* ctx, int N, const float2* tw, const float2* base, float2* spec, const CtfStack& c,
-                    int nz, const uint32_t* need) {
-    launch_cols<kColFan>(ctx, N, tw, base, spec, c, PrepFilter{}, nz, need);
+                    int nz, const uint32_t* need, uint32_t wanted) {
+    launch_cols<kColFan>(ctx, N, tw, base, spec, c, PrepFilter{}, nz, need, wanted);
 }
 void fft2d_cols_prep(artia_ctx* ctx, int N, const float2* tw, float2* spec, const PrepFilter& f, int nz) {
     launch_cols<kColPrep>(ctx, N, tw, nullptr, spec, CtfStack{}, f, nz);

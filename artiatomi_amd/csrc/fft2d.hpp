@@ -80,14 +80,14 @@ void fft2d_rows_square(artia_ctx* ctx, int N, const float2* tw, const RowSrc& s,
 void fft2d_rows_prep(artia_ctx* ctx, int N, const float2* tw, const RowSrc& s, float2* spec, int nz);
 // Rows of the stack's images that are wanted: bit y % 32 of word y / 32 of image z at need + z * N / 32, whole
 // row blocks (fft2d_row_blocks) at a time; null: all.  The others are neither written by the columns nor
-// transformed.
+// transformed.  wanted: bit z 0 where image z has none (its columns are left out too).
 // columns: forward only (in place)
 void fft2d_cols_forward(artia_ctx* ctx, int N, const float2* tw, float2* spec, int nz);
 // forward, CTF of slab z, back (in place)
 void fft2d_cols_ctf(artia_ctx* ctx, int N, const float2* tw, float2* spec, const CtfStack& c, int nz);
 // spec[z] = back(base * CTF of slab z), base transformed along the columns
 void fft2d_cols_fan(artia_ctx* ctx, int N, const float2* tw, const float2* base, float2* spec, const CtfStack& c,
-                    int nz, const uint32_t* need = nullptr);
+                    int nz, const uint32_t* need = nullptr, uint32_t wanted = ~0u);
 // forward, projection preparation's filters, back (in place)
 void fft2d_cols_prep(artia_ctx* ctx, int N, const float2* tw, float2* spec, const PrepFilter& f, int nz);
 // rows back: each image stored (or added), or the preparation's store

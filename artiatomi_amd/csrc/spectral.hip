@@ -330,7 +330,8 @@ RowDst square_target(float* out, size_t stride, int W, int H, size_t pitch, int 
 artia_status ctf_filter_slabs_own(artia_ctx* ctx, const float* src, size_t src_stride, int n, int W, int H, size_t pitch,
                                   float* out, size_t out_stride, const int corners[8], const float cut[2],
                                   const float dim[2], const artia_ctf_params& p, const float* dmin_nm,
-                                  const float* dmax_nm, float angle_deg, int forFP, const uint32_t* need) {
+                                  const float* dmax_nm, float angle_deg, int forFP, const uint32_t* need,
+                                  const unsigned char* wanted) {
     const int N = W > H ? W : H;
     FftOwn& f = ctx->ffto;
     artia_status st = f.ensure(ctx, N);
@@ -354,7 +355,16 @@ artia_status ctf_filter_slabs_own(artia_ctx* ctx, const float* src, size_t src_s
         const int b = std::min(f.cap, n - k0);
         const CtfStack cs = make_ctf_stack(N, p, dmin_nm + k0, dmax_nm + k0, angle_deg, forFP, b);
         if (shared) {
-            fft2d_cols_fan(ctx, N, f.tw, base, f.spec, cs, b, need);
+            uint32_t use = ~0u;
+            if (need && wanted) {
+                use = 0;
+                for (int i = 0; i < b; i++) use |= wanted[k0 + i] ? 1u << i : 0u;
+                if (!use) {
+                    need += (size_t)b * (size_t)(N / 32);
+                    continue;
+                }
+            }
+            fft2d_cols_fan(ctx, N, f.tw, base, f.spec, cs, b, need, use);
         } else {
             s.src = src + (size_t)k0 * src_stride;
             s.weight = weight;
@@ -593,12 +603,13 @@ int slab_row_block(int W, int H) {
 artia_status ctf_filter_slabs(artia_ctx* ctx, const float* src, size_t src_stride, int n, int W, int H, size_t pitch,
                               float* out, size_t out_stride, const int corners[8], const float cut[2],
                               const float dim[2], const artia_ctf_params& p, const float* dmin_nm,
-                              const float* dmax_nm, float angle_deg, int forFP, const uint32_t* need) {
+                              const float* dmax_nm, float angle_deg, int forFP, const uint32_t* need,
+                              const unsigned char* wanted) {
     if (n <= 0) return ARTIA_OK;
     const int N = W > H ? W : H;
     if (fft2d_supports(N) && fft2d_fits(H, pitch))
         return ctf_filter_slabs_own(ctx, src, src_stride, n, W, H, pitch, out, out_stride, corners, cut, dim, p, dmin_nm,
-                                    dmax_nm, angle_deg, forFP, need);
+                                    dmax_nm, angle_deg, forFP, need, wanted);
     FftBatch& fb = ctx->fftb;
     artia_status st = fb.ensure(ctx, N);
     if (st != ARTIA_OK) return st;

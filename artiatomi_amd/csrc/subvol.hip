@@ -508,6 +508,8 @@ struct artia_subvol_plan {
     TiltSlab* d_tslab = nullptr;   // CTF: per tilt, its slab bounds and stack offset
     uint32_t* d_need = nullptr;    // CTF: the rows of every tilt's slab images that the sub-volumes read (or null)
     std::vector<size_t> need_off;  // per tilt, its first word
+    std::vector<unsigned char> wanted;   // per slab of every tilt, whether it has such rows
+    std::vector<int> bound_off;          // per tilt, its first slab
     std::vector<int> bound_count;
     std::vector<long long> stack_off;   // per tilt, within its chunk (in slab images)
     std::vector<int> chunks;            // tilt chunk starts, then ntilts
@@ -551,7 +553,8 @@ artia_status set_items(artia_subvol_plan* p, int policy, int qpt) {
 // ctf_filter_slabs takes them: per slab whose distances a sub-volume's quads meet, the rows of its quads'
 // footprints with the LINEAR fetch's pixel on each side and one more for rounding.  Both are affine over
 // the quads, so the corner quads bound them.  A few hundred picked particles meet each of a tilt's some
-// hundred slabs in a quarter of the rows: 400 cubes in a 4096 field by 11 tilts 195 -> 128 ms.
+// hundred slabs in a quarter of the rows: 400 cubes in a 4096 field by 11 tilts 195 -> 128 ms, 125 with the
+// columns of slabs that no cube meets left out.
 void mark_rows(const std::vector<PairDev>& pairs, int nsub, int ntilts, int t, const float* starts, int count, int W, int H,
                int rb, uint32_t* need) {
     const int N = std::max(W, H), words = N / 32, by = (N - H) / 2;
@@ -602,7 +605,8 @@ artia_status filter_tilt(artia_subvol_plan* p, int t) {
     return ctf_filter_slabs(p->ctx, in.images + (size_t)t * slabStride, 0, count, in.W, in.H, in.pitch,
                             p->d_stack + (size_t)p->stack_off[(size_t)t] * slabStride, slabStride, nullptr, nullptr, nullptr, p->ctfp, dmin.data(), dmax.data(),
                             p->defocus[(size_t)t].astig_angle_deg, 0,
-                            p->d_need ? p->d_need + p->need_off[(size_t)t] : nullptr);
+                            p->d_need ? p->d_need + p->need_off[(size_t)t] : nullptr,
+                            p->d_need ? p->wanted.data() + p->bound_off[(size_t)t] : nullptr);
 }
 
 // CTF: the persistent backprojection of tilts [t0, t1) from their filtered stacks.
@@ -912,6 +916,10 @@ artia_status artia_subvol_plan_create(artia_ctx* ctx, const artia_subvol* subs, 
                 mark_rows(pairs, nsub, ntilts, t, all.data() + boff[(size_t)t], p->bound_count[(size_t)t], width, height, rb,
                           need.data() + p->need_off.back());
             }
+            p->bound_off = boff;
+            p->wanted.assign(all.size(), 0);
+            for (size_t i = 0; i < need.size(); i++)
+                if (need[i]) p->wanted[i / words] = 1;
             if ((st = upload(ctx, (void**)&p->d_need, need.data(), need.size() * sizeof(uint32_t), "slab rows")) !=
                 ARTIA_OK) {
                 delete p;
