@@ -363,16 +363,17 @@ __global__ void __launch_bounds__(Shape<N>::threads, 4) cols_kernel(const float2
         const bool steps = kKind != kColPrep && !ctf.k.phaseFlip && ctf.k.beta[1] == 0.0f && ctf.k.beta[3] == 0.0f;
         double power = 0.0;
 #pragma unroll 1
-        for (int half = 0; half < 2; half++) {   // frequencies >= 0 and < 0
+        for (int half = 0; half < 2; half++) {   // frequencies >= 0 and < 0, each outwards (see CtfEnvelopeRun)
+            const int step = half ? -T : T;
             CtfEnvelopeRun env{0.0, 0.0, 0.0};
-            if (steps) env.start(kx, t - half * (N / 2), T, ctf.k);
+            if (steps) env.start(kx, half ? t - T : t, step, ctf.k);
+            int ky = half ? t + T * (E - 1) : t;
 #pragma unroll 1
-            for (int i = half * (E / 2); i < (half + 1) * (E / 2); i++) {
-                const int ky = t + T * i;
+            for (int i = 0; i < E / 2; i++, ky += step) {
                 C2* at = mine + slot<2>(ky);
                 float2 r;
                 if (kKind == kColFan) {
-                    r = load_at<float2>(in, off + (uint32_t)(16 * T * i));
+                    r = load_at<float2>(in, (uint32_t)(p * N * 2 + 2 * ky + h) * 8u);
                 } else {
                     r = make_float2(at->x, at->y);
                 }

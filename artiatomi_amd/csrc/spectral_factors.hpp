@@ -73,10 +73,12 @@ __device__ __forceinline__ CtfPoint ctf_point(int x, int y, const CtfK& k) {
 }
 
 // The envelopes of column x at y = y0, y0 + step, .. without an exp for each (no odd powers): exp(a len^2)
-// steps by a factor that itself steps by a constant one.
+// steps by a factor that itself steps by a constant one.  |y| grows along the run, so that with the usual a < 0 all
+// three only decay and a steep envelope that underflows stays 0 as its exp does (towards y = 0 the product
+// could not rise from 0 again, or would be 0 times infinity); with a > 0 the envelope overflows first.
 struct CtfEnvelopeRun {
     double e, r, q;
-    // yp: the signed frequency of the first point
+    // yp: the signed frequency of the first point, step: away from 0
     __device__ __forceinline__ void start(int x, int yp, int step, const CtfK& k) {
         const double fs = (double)k.freq_step, a = -(double)k.beta[2] * 1e-16 * (fs * fs);
         const double y = (double)yp, s = (double)step, xp = (double)x;

@@ -157,3 +157,38 @@ def test_subvolume_plan_filters_the_rows_it_reads(ctx, W, H):
     assert float(sets[0][0][1].abs().max()) > 0   # (some of the others miss a narrow detector)
     for (_, a), (_, b) in zip(*sets):
         assert torch.equal(a, b)
+
+
+# At a pixel of 0.5 nm the envelope's exponent is 100 beta_fac[2] at the edge of an axis: 5, and three steep ones
+# whose exp underflows before the corner (twice as much), before the edge and well within it; a negative one
+# (growing), odd powers, and phase flips (no envelope).
+ENVELOPES = {
+    "mild": dict(beta_fac=(2.0, 0.0, 0.05, 0.0)),
+    "exponent_800": dict(beta_fac=(2.0, 0.0, 8.0, 0.0)),
+    "exponent_1500": dict(beta_fac=(2.0, 0.0, 15.0, 0.0)),
+    "exponent_3000": dict(beta_fac=(0.0, 0.0, 30.0, 0.0)),
+    "growing": dict(beta_fac=(2.0, 0.0, -0.05, 0.0)),
+    "odd_powers": dict(beta_fac=(2.0, 0.3, 0.008, 0.01)),
+    "phase_flip": dict(beta_fac=(2.0, 0.0, 0.008, 0.0), phase_flip_only=True),
+}
+
+
+@pytest.mark.parametrize("W,H", [(128, 128), (256, 131), (512, 512), (1000, 1024)])
+@pytest.mark.parametrize("name", list(ENVELOPES))
+def test_slab_filter_envelopes(ctx, name, W, H):
+    """Every form of the CTF's envelope, against the FP64 composition: a factor scales a point's rounding error
+    with its value, so the gate is that of white images (above)."""
+    print(f"envelope {name} {W} x {H}", flush=True)
+    kw = ENVELOPES[name]
+    img = white(H, W, W + H)
+    corners, cut, dim = [0, H - 1, W - 1, H - 1, 0, 0, W - 1, 0], (0.0, 0.0), (2.0, 2.0)
+    p = A.ctf_params(pixelsize_nm=0.5, amp_contrast=0.07, **kw)
+    k = O.ctf_consts(2.7, 300.0, 0.5, max(W, H), 0.07)
+    for for_fp in (True, False):
+        out = torch.zeros((H, W), device="cuda")
+        ctx.ctf_slab_filter(torch.from_numpy(img).cuda(), out, corners, p, 3000.0, 3150.0, 20.0, for_fp=for_fp,
+                            accumulate=False, cut_length=cut, dim_length=dim)
+        _, f = CC.slab_filter(img.astype(np.float64), corners, k, 3000.0, 3150.0, 20.0, for_fp, cut, dim,
+                              beta=kw["beta_fac"], phase_flip=kw.get("phase_flip_only", False))
+        assert float(np.abs(f).max()) > 0
+        assert rel_l2(out.cpu().numpy(), f) <= 1e-6, for_fp
