@@ -92,16 +92,21 @@ struct CtfEnvelopeRun {
     }
 };
 
-// sin and cos of t quarter turns, by the Taylor polynomials on [-pi/4, pi/4] (remainders below 1e-11).
+// sin and cos of t quarter turns, by the Taylor polynomials on [-pi/4, pi/4]: the first terms left out are
+// x^17 / 17! = 5e-17 and x^18 / 18! = 2e-18, below the rounding of the values (1.1e-16).
 __device__ __forceinline__ void sincos_quarters(double t, double& s, double& c) {
     const double n = rint(t), x = (t - n) * 1.57079632679489661923, x2 = x * x;
     const int q = (int)(long long)n;
-    double a = __builtin_fma(x2, -1.0 / 39916800.0, 1.0 / 362880.0);
+    double a = __builtin_fma(x2, -1.0 / 1307674368000.0, 1.0 / 6227020800.0);
+    a = __builtin_fma(x2, a, -1.0 / 39916800.0);
+    a = __builtin_fma(x2, a, 1.0 / 362880.0);
     a = __builtin_fma(x2, a, -1.0 / 5040.0);
     a = __builtin_fma(x2, a, 1.0 / 120.0);
     a = __builtin_fma(x2, a, -1.0 / 6.0);
     a = __builtin_fma(x2 * x, a, x);
-    double b = __builtin_fma(x2, 1.0 / 479001600.0, -1.0 / 3628800.0);
+    double b = __builtin_fma(x2, 1.0 / 20922789888000.0, -1.0 / 87178291200.0);
+    b = __builtin_fma(x2, b, 1.0 / 479001600.0);
+    b = __builtin_fma(x2, b, -1.0 / 3628800.0);
     b = __builtin_fma(x2, b, 1.0 / 40320.0);
     b = __builtin_fma(x2, b, -1.0 / 720.0);
     b = __builtin_fma(x2, b, 1.0 / 24.0);

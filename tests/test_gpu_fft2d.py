@@ -192,3 +192,23 @@ def test_slab_filter_envelopes(ctx, name, W, H):
                               beta=kw["beta_fac"], phase_flip=kw.get("phase_flip_only", False))
         assert float(np.abs(f).max()) > 0
         assert rel_l2(out.cpu().numpy(), f) <= 1e-6, for_fp
+
+
+def test_ctf_factor_near_its_zeros(ctx):
+    """The factor itself where it is small, so that an absolute error of the phase's sine and cosine shows beside
+    the float rounding: sine and cosine of equal weight put the zeros an eighth of a turn off, where truncated
+    polynomials err most.  Phases to 40 radians carry 40 * 2^-53 * 4 operations = 2e-14 in either arithmetic, and
+    without damping the factor's slope at a zero is 1 / wiener = 10: 4e-13, gate 2e-12 beside the rounding.
+    (Column 0 is left out: there the oracle's angle is the float pi / 2.)"""
+    N = 1024
+    print(f"factor near zeros {N}", flush=True)
+    beta = (0.0, 0.0, 0.0, 0.0)
+    p = A.ctf_params(pixelsize_nm=0.5, amp_contrast=0.70710678, beta_fac=beta)
+    k = O.ctf_consts(2.7, 300.0, 0.5, N, 0.70710678)
+    ones = np.ones((N, N // 2 + 1), np.complex64)
+    spec = torch.from_numpy(ones).cuda()
+    ctx.ctf_apply(spec, p, 3000.0, 3150.0, 20.0, for_fp=False)
+    got = spec.cpu().numpy().real[:, 1:].astype(np.float64)
+    ref = O.ctf_apply(ones.astype(np.complex128), k, 3000.0, 3150.0, 20.0, for_fp=False, beta=beta).real[:, 1:]
+    assert float(np.abs(ref).min()) < 4e-5   # zeros are met (3.2e-5)
+    assert np.all(np.abs(got - ref) <= 2.0 ** -23 * np.abs(ref) + 2e-12)
