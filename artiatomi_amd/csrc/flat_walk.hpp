@@ -95,13 +95,14 @@ struct FlatWalker {
 };
 
 // Sum of a cell's m samples from its y-blended edges A (near x, near z), B (far x), C (far z), D:
-// m g(middle) + m (m^2 - 1) / 12 (D - C - B + A) |dq_x dq_z|, rounded once to float (the ray adds the
-// cells in double).  m = 0 gives +-0.
-__device__ __forceinline__ float flat_cell_sum(float A, float B, float C, float D, float a, float c, float m, float K) {
+// m g(middle) + m (m^2 - 1) / 12 (D - C - B + A) |dq_x dq_z|, the sum rounded once to float (the ray adds
+// the cells in double).  m = 0 gives +-0.
+__host__ __device__ __forceinline__ float flat_cell_sum(float A, float B, float C, float D, float a, float c, float m,
+                                                        float K) {
     const float d0 = B - A, d1 = D - C;
     const float e0 = __builtin_fmaf(a, d0, A), e1 = __builtin_fmaf(a, d1, C);
     const float g = __builtin_fmaf(c, e1 - e0, e0);
-    return m * __builtin_fmaf((d1 - d0) * K, __builtin_fmaf(m, m, -1.0f), g);
+    return __builtin_fmaf(m, g, ((d1 - d0) * K) * (m * __builtin_fmaf(m, m, -1.0f)));
 }
 
 // Gradient of the cell's interpolant summed over its samples, in oriented texel coordinates, added to
