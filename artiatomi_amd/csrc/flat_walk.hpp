@@ -49,30 +49,36 @@ __device__ __forceinline__ FlatDir flat_dir(const float dq[3]) {
     return d;
 }
 
-// Samples k .. count - 1 of one sub-ray, cell by cell.  r = (start - near edge) - hd in oriented
-// coordinates, so that the middle of samples k .. k + m - 1 lies (2 k + m) hd + r into the cell
-// (one fma), and sample index kb = (1 - hd - r) inv crosses the cell's far face.  A step takes the axis
-// that is crossed first (z on a tie; the cell in between holds no samples).
+// Samples k .. count - 1 of one sub-ray, cell by cell.  With R = (start - near edge) - hd in oriented
+// coordinates the middle of samples k .. k + m - 1 lies (2 k + m) hd + R into the cell, and sample index
+// kb = (1 - hd - R) inv crosses the cell's far face.  A step lowers R by 1 and takes the axis that is crossed
+// first (z on a tie; the cell in between holds no samples).
+//
+// R is kept as r + lo, r a multiple of 2^-8 (exact down to -65536, so that steps do not round) and lo the rest,
+// which stays.  R in one float rounds every time it passes a power of two, alike for all rays that enter through
+// one face: at 256 layers a shift of 1e-5 of a cell that no averaging takes out.
 struct FlatWalker {
-    float r[2], kb[2];
+    float r[2], lo[2], c1[2], kb[2];
     float k, count;
 
     __device__ __forceinline__ void crossings(const FlatDir& d) {
 #pragma unroll
-        for (int i = 0; i < 2; i++) kb[i] = __builtin_fmaf(-r[i], d.inv[i], d.c1[i]);
+        for (int i = 0; i < 2; i++) kb[i] = __builtin_fmaf(-r[i], d.inv[i], c1[i]);
     }
     __device__ __forceinline__ void init(const FlatDir& d, const float q0[3], int n) {
 #pragma unroll
         for (int i = 0; i < 2; i++) {
-            const float q = q0[2 * i], fl = floorf(q);
-            r[i] = (d.sgn[i] > 0 ? q - fl : (fl + 1.0f) - q) - d.hd[i];
+            const float q = q0[2 * i], fl = floorf(q), at = d.sgn[i] > 0 ? q - fl : (fl + 1.0f) - q;   // exact
+            r[i] = rintf((at - d.hd[i]) * 256.0f) * 0.00390625f;
+            lo[i] = (at - r[i]) - d.hd[i];
+            c1[i] = __builtin_fmaf(-lo[i], d.inv[i], d.c1[i]);
         }
         crossings(d);
         k = 0.0f;
         count = (float)n;
     }
     __device__ __forceinline__ bool active() const { return k < count; }
-    // near lattice index of the current cell on oriented axis i (r is near - start up to rounding)
+    // near lattice index of the current cell on oriented axis i (r is start - near - hd up to lo, below 2^-9)
     __device__ __forceinline__ int near(const FlatDir& d, const float q0[3], int i) const {
         const float X = d.sgn[i] > 0 ? q0[2 * i] : -q0[2 * i];
         return (int)rintf((X - d.hd[i]) - r[i]);
@@ -81,8 +87,8 @@ struct FlatWalker {
     __device__ __forceinline__ float samples(const FlatDir& d, float kn, float& a, float& c) {
         const float kend = __builtin_amdgcn_fmed3f(ceilf(kn), k, count);
         const float m = kend - k, s = k + kend;
-        a = __builtin_fmaf(s, d.hd[0], r[0]);
-        c = __builtin_fmaf(s, d.hd[1], r[1]);
+        a = __builtin_fmaf(s, d.hd[0], r[0]) + lo[0];
+        c = __builtin_fmaf(s, d.hd[1], r[1]) + lo[1];
         k = kend;
         return m;
     }
