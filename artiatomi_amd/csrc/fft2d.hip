@@ -379,8 +379,12 @@ __global__ void __launch_bounds__(Shape<N>::threads, 4) cols_kernel(const float2
                 }
                 if (kKind == kColPrep) {
                     r = prep_factor(r, kx, ky, N, pf, z);
-                    if (pf.dc && kx == 0 && ky == 0) pf.dc[z] = r.x;
-                    else power = __builtin_fma((double)r.x, (double)r.x, __builtin_fma((double)r.y, (double)r.y, power));
+                    if (pf.dc && kx == 0 && ky == 0) {
+                        pf.dc[z] = r.x;
+                        // with the statistics from the spectrum the mean leaves here
+                        if (pf.power) r = make_float2(0.0f, 0.0f);
+                    } else
+                        power = __builtin_fma((double)r.x, (double)r.x, __builtin_fma((double)r.y, (double)r.y, power));
                 } else {
                     const CtfPoint pt = steps ? ctf_point(kx, ky, ctf.k, env.e) : ctf_point(kx, ky, ctf.k);
                     r = ctf_apply_at(r, pt, ctf.k, ctf.def0[z], ctf.def1[z]);
@@ -494,10 +498,7 @@ __global__ void __launch_bounds__(Shape<N>::threads, 4) rows_back_kernel(const f
             float val = (q ? v[i].y : v[i].x) * d.scale;
             const uint32_t at = ((uint32_t)(y + q) * (uint32_t)d.pitch + (uint32_t)x) * 4u;
             if (kKind == kDstStore) {
-                if (d.st) {   // uniform
-                    val = val - d.st[z].mean_hf;
-                    val = val / -d.st[z].std_hf;
-                }
+                if (d.st) val = val / -d.st[z].std_hf;   // uniform
                 if (d.weight)
                     val = load_at<float>(d.weight, (uint32_t)((y0 + 2 * f + q) * N + t + T * i) * 4u) * val;
                 store_at(out, at, d.accumulate ? load_at<float>(out, at) + val : val);

@@ -61,7 +61,8 @@ struct RowDst {
     float* out;
     size_t pitch, stride;
     const float* weight;   // as RowSrc's
-    // kStore: out[z * stride] = w v (accumulate: += ), rows in need; with st the preparation's normalisation of v
+    // kStore: out[z * stride] = w v (accumulate: += ), rows in need; with st divided by the preparation's
+    // deviation (its mean has left with frequency 0)
     int accumulate;
     const PrepStat* st;
     const uint32_t* need;

@@ -184,7 +184,7 @@ struct PrepFilter {
     double sn[kFftBatchMax], cs[kFftBatchMax];        // of each image's angle
     const PrepStat* st;
     // out (or null): each wave's sum of the filtered spectrum's squares over both half planes, without frequency 0
-    // (fft2d_col_waves(N) an image)
+    // (fft2d_col_waves(N) an image), and frequency 0 taken out
     double* power;
     float* dc;                                        // out (or null): image z's filtered value at frequency 0
 };

@@ -212,3 +212,19 @@ def test_ctf_factor_near_its_zeros(ctx):
     ref = O.ctf_apply(ones.astype(np.complex128), k, 3000.0, 3150.0, 20.0, for_fp=False, beta=beta).real[:, 1:]
     assert float(np.abs(ref).min()) < 4e-5   # zeros are met (3.2e-5)
     assert np.all(np.abs(got - ref) <= 2.0 ** -23 * np.abs(ref) + 2e-12)
+
+
+@pytest.mark.parametrize("N", [128, 512, 2048])
+def test_prepared_squares_have_no_mean(ctx, N):
+    """A square whose mean is 30000 times its deviation: the normalised image has none of it left.  Without
+    frequency 0 a pixel's error is a few 2^-24 of the deviation 1, independent of the others' or a bias of that
+    size: gate 1e-6.  (The mean subtracted from float pixels left up to half a unit of its last place, 1e-3.)"""
+    print(f"mean of a prepared square {N}", flush=True)
+    img = (30000.3 + white(N, N, 11)).astype(np.float32)
+    out = torch.zeros((1, N, N), device="cuda")
+    pp = A.prep_params(dtype="float32", normalization="std", lp=0.4 * N, lps=0.05 * N)
+    mean, std, _ = ctx.prepare_projections(pp, torch.from_numpy(img[None]).cuda(), out)
+    assert mean[0] == pytest.approx(float(img.astype(np.float64).mean()), rel=1e-6)
+    got = out[0].double()
+    assert abs(float(got.mean())) <= 1e-6
+    assert float(got.std(unbiased=False)) == pytest.approx(1.0, rel=1e-5)
