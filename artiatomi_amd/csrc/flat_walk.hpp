@@ -201,8 +201,8 @@ __device__ __forceinline__ FlatBox flat_box(const VolG& v, const TubePlan& tp, c
     q.X1 = min((int)floorf(tb.axh + fmaxf(tp.bx * z0, tp.bx * z1)) + 2, v.nx + 1);
     q.Y0 = wave_uniform(max((int)floorf(tb.ayl) - 1, -1));
     q.Y1 = min((int)floorf(tb.ayh) + 2, v.ny);
-    q.Z0 = max(zs, -1);
-    q.Z1 = min(ze + 1, v.nz);
+    q.Z0 = zs;
+    q.Z1 = ze + 1;
     q.CX = wave_uniform(q.X1 - q.X0 + 1);
     q.CY = wave_uniform(q.Y1 - q.Y0 + 1);
     q.CZ = q.Z1 - q.Z0 + 1;
@@ -278,7 +278,7 @@ struct FlatAhead {
 };
 
 // Whether the cells the lane crosses in layers [zs, ze] lie in the box with a column of margin: from its
-// current cell (xn, zn) to its last sample or the slab's exit.
+// current cell (xn, zn) to its last sample or the slab's exit, whose layer the box holds.
 __device__ __forceinline__ bool flat_lane_in_box(const VolG& v, const FlatBox& q, const FlatDir& d, const float q0[3],
                                                  const float dq[3], const FlatWalker& w, int zs, int ze, int xn,
                                                  int zn) {
@@ -288,7 +288,7 @@ __device__ __forceinline__ bool flat_lane_in_box(const VolG& v, const FlatBox& q
     const int xb = (int)floorf(__builtin_fmaf(ke, dq[0], q0[0])), yc = (int)floorf(q0[1]);
     const int xa = d.sgn[0] > 0 ? xn : -(xn + 1), za = d.sgn[1] > 0 ? zn : -(zn + 1);
     return min(xa, xb) - 1 >= q.X0 && max(xa, xb) + 2 <= q.X1 && yc >= q.Y0 && yc + 1 <= q.Y1 &&
-           (d.sgn[1] > 0 ? za : max(zs, -1)) >= q.Z0 && (d.sgn[1] > 0 ? min(ze + 1, v.nz) : za + 1) <= q.Z1;
+           (d.sgn[1] > 0 ? za >= q.Z0 : za + 1 <= q.Z1);
 }
 
 // The lane's samples in cell layers [zs, ze] of a slab, from the staged box where the cells they cross
@@ -381,27 +381,30 @@ __device__ __forceinline__ void flat_tube_walk(const VolG& v, const T* __restric
     FlatWalker w;
     w.init(d, q0, count);
     const int nslab = zlo <= zhi ? (zhi - zlo) / kSlabCells + 1 : 0;
-    auto first_layer = [&](int j) { return tp.zdir > 0 ? zlo + j * kSlabCells : zhi - (j + 1) * kSlabCells + 1; };
     FlatAhead<T> ahead;
     FlatBox next{};
+    int zs, ze;
     if (kAhead && nslab > 0) {
-        next = flat_box(v, tp, tb, first_layer(0), first_layer(0) + kSlabCells - 1);
+        slab_layers(v, tp.zdir, zlo, zhi, 0, zs, ze);
+        next = flat_box(v, tp, tb, zs, ze);
         ahead.load(v, vol, next);
     }
     for (int j = 0; j < nslab; j++) {
-        const int zs = first_layer(j), ze = zs + kSlabCells - 1;
+        slab_layers(v, tp.zdir, zlo, zhi, j, zs, ze);
         const FlatBox q = kAhead ? next : flat_box(v, tp, tb, zs, ze);
         __syncthreads();   // the previous slab's reads are done
         if (kAhead) ahead.store(v, vol, chunk, q);
         else if (q.staged) stage_flat_box(v, vol, chunk, q);
         __syncthreads();
         if (kAhead && j + 1 < nslab) {
-            next = flat_box(v, tp, tb, first_layer(j + 1), first_layer(j + 1) + kSlabCells - 1);
+            int ns, ne;
+            slab_layers(v, tp.zdir, zlo, zhi, j + 1, ns, ne);
+            next = flat_box(v, tp, tb, ns, ne);
             ahead.load(v, vol, next);
         }
         if (w.active()) flat_walk_slab<kGrad>(v, vol, chunk, q, d, q0, dq, w, zs, ze, f);
     }
-    // cells beyond the slabs (not expected)
+    // cells beyond the slabs
     flat_walk_direct<true>(v, vol, d, q0, w, []() { return true; }, f);
 }
 
@@ -420,10 +423,11 @@ __device__ __forceinline__ void flat_tube_segments(const VolG& v, const T* __res
     w.init(d, seg.q0, 0);   // no segment yet: the first pass below loads one
     bool more = true;
     const int nslab = zlo <= zhi ? (zhi - zlo) / kSlabCells + 1 : 0;
-    // slabs of cell layers, then (j == nslab) the cells beyond them (not expected) from the volume
+    // slabs of cell layers, then (j == nslab) the cells beyond them from the volume
     for (int j = 0; j <= nslab; j++) {
         const bool tail = j == nslab;
-        const int zs = tp.zdir > 0 ? zlo + j * kSlabCells : zhi - (j + 1) * kSlabCells + 1, ze = zs + kSlabCells - 1;
+        int zs, ze;
+        slab_layers(v, tp.zdir, zlo, zhi, j, zs, ze);
         FlatBox q{};
         if (!tail) {
             q = flat_box(v, tp, tb, zs, ze);
@@ -578,7 +582,8 @@ __device__ __forceinline__ void flat_tube_scatter(const VolG& v, float* __restri
     w.init(d, q0, count);
     const int nslab = zlo <= zhi ? (zhi - zlo) / kSlabCells + 1 : 0;
     for (int j = 0; j < nslab; j++) {
-        const int zs = tp.zdir > 0 ? zlo + j * kSlabCells : zhi - (j + 1) * kSlabCells + 1, ze = zs + kSlabCells - 1;
+        int zs, ze;
+        slab_layers(v, tp.zdir, zlo, zhi, j, zs, ze);
         const FlatBox q = flat_box(v, tp, tb, zs, ze, tp.box);
         const int n = q.CX * q.SY * q.CZ;
         __syncthreads();   // the previous slab's box is in the volume
@@ -603,7 +608,7 @@ __device__ __forceinline__ void flat_tube_scatter(const VolG& v, float* __restri
             }
         }
     }
-    // cells beyond the slabs (not expected)
+    // cells beyond the slabs
     flat_scatter_direct(v, grad, d, q0, rd, w, []() { return true; });
 }
 

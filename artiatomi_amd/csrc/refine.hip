@@ -432,12 +432,14 @@ __global__ void __launch_bounds__(kAdjFlatThreads) pair_adjoint_flat_kernel(Pair
             const FlatDir d = flat_dir(s.dq);
             FlatWalker w;
             w.init(d, s.q0, s.count);
-            // the walk's cells, first and last sample's, in the padded planes (a volume with a z shift
-            // may be sampled beyond them)
+            // the walk's cells in the padded planes (-1 .. n): the first sample's as it is, the last with a
+            // quarter of a cell for the walk's rounding, half as far as a whole volume's last sample is from the
+            // border (a volume stored in part, with a z shift, is sampled beyond it)
             const float last = (float)(s.count - 1);
-            const int xa = (int)floorf(s.q0[0]), xb = (int)floorf(__builtin_fmaf(last, s.dq[0], s.q0[0]));
-            const int za = (int)floorf(s.q0[2]), zb = (int)floorf(__builtin_fmaf(last, s.dq[2], s.q0[2]));
-            if (min(xa, xb) < -1 || max(xa, xb) > v.nx - 1 || min(za, zb) < -1 || max(za, zb) > v.nz - 1) {
+            const int xf = (int)floorf(s.q0[0]), zf = (int)floorf(s.q0[2]);
+            const float xl = __builtin_fmaf(last, s.dq[0], s.q0[0]), zl = __builtin_fmaf(last, s.dq[2], s.q0[2]);
+            if (xf < -1 || xf > v.nx - 1 || zf < -1 || zf > v.nz - 1 ||
+                !(xl >= -0.75f && xl < (float)v.nx - 0.25f && zl >= -0.75f && zl < (float)v.nz - 0.25f)) {
                 flat_scatter_direct(v, gv, d, s.q0, r, w, []() { return true; });
                 continue;
             }

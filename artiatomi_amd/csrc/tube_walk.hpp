@@ -128,6 +128,15 @@ __device__ __forceinline__ TubeBox tube_box(const VolG& v, const TiltG& g, const
     return TubeBox{wave_uniform(axl), wave_uniform(axh), wave_uniform(ayl), wave_uniform(ayh)};
 }
 
+// Cell layers [zs, ze] of slab j, in the rays' z direction, clipped to the volume's -1 .. nz - 1: the box holds
+// layers zs .. ze + 1 of them all, and what a volume stored in part (z shift) is sampled at beyond its clamp border
+// is left to the walk from memory after the last slab.
+__device__ __forceinline__ void slab_layers(const VolG& v, int zdir, int zlo, int zhi, int j, int& zs, int& ze) {
+    const int first = zdir > 0 ? zlo + j * kSlabCells : zhi - (j + 1) * kSlabCells + 1;
+    zs = max(first, -1);
+    ze = min(first + kSlabCells - 1, v.nz - 1);
+}
+
 // Corners of a cell from the staged box when it lies inside, otherwise from global memory with
 // clamped indices.  The LDS reads are issued unconditionally (at offset 0 when outside, which stays
 // inside the box) and overwritten on the rare global path: branching between the two sources would
@@ -335,9 +344,8 @@ __device__ __forceinline__ void tube_slabs(const VolG& v, const T* __restrict__ 
     w.init_dir(q0, td.sgn, td.inv, count);
     const int nslab = zlo <= zhi ? (zhi - zlo) / kSlabCells + 1 : 0;
     for (int j = 0; j < nslab; j++) {
-        // cell layers [zs, ze] of this slab, in the rays' z direction
-        const int zs = tp.zdir > 0 ? zlo + j * kSlabCells : zhi - (j + 1) * kSlabCells + 1;
-        const int ze = zs + kSlabCells - 1;
+        int zs, ze;
+        slab_layers(v, tp.zdir, zlo, zhi, j, zs, ze);
         // box of lattice indices the slab's cells touch, in index space padded by the clamp border
         // (-1 .. n); the margins cover the float rounding of the walk
         const float z0 = (float)zs, z1 = (float)(ze + 1);
@@ -345,7 +353,7 @@ __device__ __forceinline__ void tube_slabs(const VolG& v, const T* __restrict__ 
         const int X1 = min((int)floorf(tb.axh + fmaxf(tp.bx * z0, tp.bx * z1)) + 2, v.nx);
         const int Y0 = wave_uniform(max((int)floorf(tb.ayl + fminf(tp.by * z0, tp.by * z1)) - 1, -1));
         const int Y1 = min((int)floorf(tb.ayh + fmaxf(tp.by * z0, tp.by * z1)) + 2, v.ny);
-        const int Z0 = max(zs, -1), Z1 = min(ze + 1, v.nz);
+        const int Z0 = zs, Z1 = ze + 1;
         const int CX = wave_uniform(X1 - X0 + 1), CY = wave_uniform(Y1 - Y0 + 1), CZ = Z1 - Z0 + 1;
         const bool staged = CX > 1 && CY > 1 && CZ > 1 && CX * CY * CZ <= (kScatter ? tp.box : kChunkFloats);
         const int n = CX * CY * CZ;
@@ -368,8 +376,7 @@ __device__ __forceinline__ void tube_slabs(const VolG& v, const T* __restrict__ 
             const float ke = fminf(fmaxf((zp - q0[2]) * td.inv[2], (float)w.k), (float)(w.count - 1));
             const int xb = (int)floorf(__builtin_fmaf(ke, td.dq[0], q0[0]));
             const int yb = (int)floorf(__builtin_fmaf(ke, td.dq[1], q0[1]));
-            const int zl = tp.zdir > 0 ? w.icell(2) : max(zs, -1);
-            const int zh = tp.zdir > 0 ? min(ze + 1, v.nz) : w.icell(2) + 1;
+            const int zl = tp.zdir > 0 ? w.icell(2) : zs, zh = tp.zdir > 0 ? ze + 1 : w.icell(2) + 1;
             fast = min(w.icell(0), xb) - 1 >= X0 && max(w.icell(0), xb) + 2 <= X1 && min(w.icell(1), yb) - 1 >= Y0 &&
                    max(w.icell(1), yb) + 2 <= Y1 && zl >= Z0 && zh <= Z1;
         }
@@ -381,7 +388,7 @@ __device__ __forceinline__ void tube_slabs(const VolG& v, const T* __restrict__ 
             // a fast lane enters with its cell in [zs, ze] and moves monotonically in z, so staying
             // in the slab is one range test
             if constexpr (kScatter) {
-                while (w.active() && w.z_in(zs, kSlabCells)) {
+                while (w.active() && w.z_in(zs, ze - zs + 1)) {
                     w.step(
                         [&](const int* cell, int k, int mi) {
                             double val[8];
@@ -396,7 +403,7 @@ __device__ __forceinline__ void tube_slabs(const VolG& v, const T* __restrict__ 
                 // every step reads its cell's corners and calls f, also for a cell without samples
                 // (f adds +-0 then: the gather callbacks add cell and gradient sums), so the loop
                 // body has no branch
-                while (w.active() && w.z_in(zs, kSlabCells)) {
+                while (w.active() && w.z_in(zs, ze - zs + 1)) {
                     w.step_all(
                         [&](const int* cell, int k, int mi) {
                             float val[8];
@@ -446,7 +453,7 @@ __device__ __forceinline__ void tube_slabs(const VolG& v, const T* __restrict__ 
             }
         }
     }
-    // cells beyond the slabs (not expected): global memory
+    // cells beyond the slabs: global memory
     while (w.active()) {
         w.step([&](const int* cell, int k, int mi) {
             const int ic[3] = {cell[0], cell[1], cell[2]};
@@ -497,17 +504,17 @@ __device__ __forceinline__ void tube_walk_segments(const VolG& v, const T* __res
     w.init_dir(seg.q0, td.sgn, td.inv, 0);   // no segment yet: the first pass below loads one
     bool more = true;
     const int nslab = zlo <= zhi ? (zhi - zlo) / kSlabCells + 1 : 0;
-    // slabs of cell layers, then (j == nslab) the cells beyond them (not expected) from global memory
+    // slabs of cell layers, then (j == nslab) the cells beyond them from global memory
     for (int j = 0; j <= nslab; j++) {
         const bool tail = j == nslab;
-        const int zs = tp.zdir > 0 ? zlo + j * kSlabCells : zhi - (j + 1) * kSlabCells + 1;
-        const int ze = zs + kSlabCells - 1;
+        int zs, ze;
+        slab_layers(v, tp.zdir, zlo, zhi, j, zs, ze);
         const float z0 = (float)zs, z1 = (float)(ze + 1);
         const int X0 = wave_uniform(max((int)floorf(tb.axl + fminf(tp.bx * z0, tp.bx * z1)) - 1, -1));
         const int X1 = min((int)floorf(tb.axh + fmaxf(tp.bx * z0, tp.bx * z1)) + 2, v.nx);
         const int Y0 = wave_uniform(max((int)floorf(tb.ayl + fminf(tp.by * z0, tp.by * z1)) - 1, -1));
         const int Y1 = min((int)floorf(tb.ayh + fmaxf(tp.by * z0, tp.by * z1)) + 2, v.ny);
-        const int Z0 = max(zs, -1), Z1 = min(ze + 1, v.nz);
+        const int Z0 = zs, Z1 = ze + 1;
         const int CX = wave_uniform(X1 - X0 + 1), CY = wave_uniform(Y1 - Y0 + 1), CZ = Z1 - Z0 + 1;
         const bool staged = !tail && CX > 1 && CY > 1 && CZ > 1 && CX * CY * CZ <= kChunkFloats;
         const int n = CX * CY * CZ;
@@ -533,8 +540,7 @@ __device__ __forceinline__ void tube_walk_segments(const VolG& v, const T* __res
                 const float ke = fminf(fmaxf((zp - seg.q0[2]) * td.inv[2], (float)w.k), (float)(w.count - 1));
                 const int xb = (int)floorf(__builtin_fmaf(ke, td.dq[0], seg.q0[0]));
                 const int yb = (int)floorf(__builtin_fmaf(ke, td.dq[1], seg.q0[1]));
-                const int zl = tp.zdir > 0 ? w.icell(2) : max(zs, -1);
-                const int zh = tp.zdir > 0 ? min(ze + 1, v.nz) : w.icell(2) + 1;
+                const int zl = tp.zdir > 0 ? w.icell(2) : zs, zh = tp.zdir > 0 ? ze + 1 : w.icell(2) + 1;
                 fast = min(w.icell(0), xb) - 1 >= X0 && max(w.icell(0), xb) + 2 <= X1 && min(w.icell(1), yb) - 1 >= Y0 &&
                        max(w.icell(1), yb) + 2 <= Y1 && zl >= Z0 && zh <= Z1;
             }
@@ -545,7 +551,7 @@ __device__ __forceinline__ void tube_walk_segments(const VolG& v, const T* __res
                 int o = ((w.icell(2) - Z0) * CY + (w.icell(1) - Y0)) * CX + (w.icell(0) - X0);
                 // every step reads its cell's corners and calls f, also for a cell without
                 // samples (f adds +-0 then), so the loop body has no branch
-                while (w.active() && w.z_in(zs, kSlabCells)) {
+                while (w.active() && w.z_in(zs, ze - zs + 1)) {
                     w.step_all(
                         [&](const int* cell, int k, int mi) {
                             float val[8];
