@@ -311,8 +311,10 @@ __global__ void __launch_bounds__(256) pair_adjoint_slab_kernel(PairArgs a, AdjS
             // the walker computes face crossings (CellWalker::step), clamped to the sub-ray
             const float offz = -s.q0[2] * inv[2];
             const float fin = (float)(sgn[2] > 0 ? zs : ze), fout = (float)(sgn[2] > 0 ? ze : zs);
-            const int kA = max(0, min(s.count, (int)ceilf(__builtin_fmaf(fin, inv[2], offz))));
-            const int kB = max(0, min(s.count, (int)ceilf(__builtin_fmaf(fout, inv[2], offz))));
+            // (the first and last slabs also take what a volume stored in part is sampled at beyond its layers)
+            const bool bottom = zs <= -1, top = ze >= v.nz;
+            const int kA = (sgn[2] > 0 ? bottom : top) ? 0 : max(0, min(s.count, (int)ceilf(__builtin_fmaf(fin, inv[2], offz))));
+            const int kB = (sgn[2] > 0 ? top : bottom) ? s.count : max(0, min(s.count, (int)ceilf(__builtin_fmaf(fout, inv[2], offz))));
             if (kB <= kA) continue;
             CellWalker wk;
             wk.init_from(s.q0, s.dq, sgn, inv, kA, kB);

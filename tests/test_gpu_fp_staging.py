@@ -242,7 +242,7 @@ def test_partial_volume_staged_equals_direct(ctx, part, tilt, tilt_x):
     assert torch.allclose(s1, s2, rtol=1e-9, atol=1e-9 * lhs)
 
 
-@pytest.mark.parametrize("tilt_x", [0.0])
+@pytest.mark.parametrize("tilt_x", [0.0, 3.0])
 def test_pair_adjoint_of_partial_volumes(ctx, tilt_x):
     """The pair adjoint summed per sub-volume, for volumes whose rays are sampled beyond their layers."""
     print(f"pair adjoint of partial volumes, tilt_x {tilt_x}", flush=True)
