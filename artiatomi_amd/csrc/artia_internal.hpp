@@ -41,15 +41,18 @@ struct FftBatch {
     void release();
 };
 
-// The three-kernel filters' state (fft2d.hpp): twiddles exp(-2 pi i k / N), cap + 1 half spectra, an N x N
-// image of crop weights and cap slab images that wait to be summed, rebuilt when N changes.
+// The three-kernel filters' state (fft2d.hpp), each buffer allocated when a filter first needs it and kept, where
+// it is, until N changes: twiddles exp(-2 pi i k / N), one half spectrum for single images, cap + 1 for stacks, an
+// N x N image of crop weights and cap slab images that wait to be summed.
 struct FftOwn {
+    enum { kOne = 1, kStack = 2, kWeight = 4, kImages = 8 };
     int N = 0, cap = 0;
     float2* tw = nullptr;
+    float2* one = nullptr;
     float2* spec = nullptr;
     float* weight = nullptr;
     float* images = nullptr;
-    artia_status ensure(artia_ctx* ctx, int n);
+    artia_status ensure(artia_ctx* ctx, int n, int buffers);
     void release();
 };
 }  // namespace artia

@@ -304,7 +304,7 @@ artia_status artia_prepare_projections(artia_ctx* ctx, const artia_prep_params* 
                      ctx->numerics == ARTIA_NUMERICS_EXACT;
     FftBatch& fb = ctx->fftb;
     FftOwn& fo = ctx->ffto;
-    artia_status st = own ? fo.ensure(ctx, N) : fb.ensure(ctx, N);
+    artia_status st = own ? fo.ensure(ctx, N, FftOwn::kStack) : fb.ensure(ctx, N);
     if (st != ARTIA_OK) return st;
     const int cap = own ? fo.cap : fb.cap, rowBlocks = own ? fft2d_row_blocks(N) : 0;
     // The normalisation of a whole square's mean and deviation needs no pass over the image: both come from the

@@ -334,7 +334,7 @@ artia_status ctf_filter_slabs_own(artia_ctx* ctx, const float* src, size_t src_s
                                   const unsigned char* wanted) {
     const int N = W > H ? W : H;
     FftOwn& f = ctx->ffto;
-    artia_status st = f.ensure(ctx, N);
+    artia_status st = f.ensure(ctx, N, FftOwn::kStack | (corners ? FftOwn::kWeight : 0) | (forFP ? FftOwn::kImages : 0));
     if (st != ARTIA_OK) return st;
     const float* weight = nullptr;
     if (corners) {
@@ -490,42 +490,43 @@ void FftBatch::release() {
     N = cap = 0;
 }
 
-artia_status FftOwn::ensure(artia_ctx* ctx, int n) {
-    if (N == n && cap > 0) return ARTIA_OK;
-    release();
-    // up to eight spectra of 4096 (540 MB) at a time: a 4096 x 4096 image takes 95.5 us of column and row kernels
-    // alone, 86 us in pairs or fours and 81.5 us among eight (fewer nearly empty last waves of blocks)
-    const size_t one = fft2d_spec_size(n) * sizeof(float2);
-    const int c = (int)std::min<size_t>((size_t)kFftBatchMax, std::max<size_t>(1, ((size_t)544 << 20) / one));
-    std::vector<float2> t((size_t)n);
-    for (int k = 0; k < n; k++) {
-        const double a = -2.0 * 3.14159265358979323846 * (double)k / (double)n;
-        t[(size_t)k] = make_float2((float)std::cos(a), (float)std::sin(a));
-    }
-    artia_status st = check_hip(ctx, hipMalloc(&tw, (size_t)n * sizeof(float2)), "hipMalloc(twiddles)");
-    if (st == ARTIA_OK)
-        st = check_hip(ctx, hipMemcpy(tw, t.data(), (size_t)n * sizeof(float2), hipMemcpyHostToDevice),
-                       "hipMemcpy(twiddles)");
-    if (st == ARTIA_OK) st = check_hip(ctx, hipMalloc(&spec, (size_t)(c + 1) * one), "hipMalloc(spectra)");
-    if (st == ARTIA_OK)
-        st = check_hip(ctx, hipMalloc(&weight, (size_t)n * n * sizeof(float)), "hipMalloc(crop weights)");
-    if (st == ARTIA_OK)
-        st = check_hip(ctx, hipMalloc(&images, (size_t)c * n * n * sizeof(float)), "hipMalloc(slab images)");
-    if (st != ARTIA_OK) {
+artia_status FftOwn::ensure(artia_ctx* ctx, int n, int buffers) {
+    const size_t image = (size_t)n * n * sizeof(float), spectrum = fft2d_spec_size(n) * sizeof(float2);
+    artia_status st = ARTIA_OK;
+    if (N != n) {
         release();
-        return st;
+        std::vector<float2> t((size_t)n);
+        for (int k = 0; k < n; k++) {
+            const double a = -2.0 * 3.14159265358979323846 * (double)k / (double)n;
+            t[(size_t)k] = make_float2((float)std::cos(a), (float)std::sin(a));
+        }
+        st = check_hip(ctx, hipMalloc(&tw, (size_t)n * sizeof(float2)), "hipMalloc(twiddles)");
+        if (st == ARTIA_OK)
+            st = check_hip(ctx, hipMemcpy(tw, t.data(), (size_t)n * sizeof(float2), hipMemcpyHostToDevice),
+                           "hipMemcpy(twiddles)");
+        if (st != ARTIA_OK) {
+            release();
+            return st;
+        }
+        N = n;
+        // up to eight spectra of 4096 (540 MB) at a time: a 4096 x 4096 image takes 95.5 us of column and row
+        // kernels alone, 86 us in pairs or fours and 81.5 us among eight (fewer nearly empty last waves of blocks)
+        cap = (int)std::min<size_t>((size_t)kFftBatchMax, std::max<size_t>(1, ((size_t)544 << 20) / spectrum));
     }
-    N = n;
-    cap = c;
-    return ARTIA_OK;
+    if ((buffers & kOne) && !one) st = check_hip(ctx, hipMalloc(&one, spectrum), "hipMalloc(spectrum)");
+    if (st == ARTIA_OK && (buffers & kStack) && !spec)
+        st = check_hip(ctx, hipMalloc(&spec, (size_t)(cap + 1) * spectrum), "hipMalloc(spectra)");
+    if (st == ARTIA_OK && (buffers & kWeight) && !weight)
+        st = check_hip(ctx, hipMalloc(&weight, image), "hipMalloc(crop weights)");
+    if (st == ARTIA_OK && (buffers & kImages) && !images)
+        st = check_hip(ctx, hipMalloc(&images, (size_t)cap * image), "hipMalloc(slab images)");
+    return st;
 }
 
 void FftOwn::release() {
-    if (tw) (void)hipFree(tw);
-    if (spec) (void)hipFree(spec);
-    if (weight) (void)hipFree(weight);
-    if (images) (void)hipFree(images);
-    tw = spec = nullptr;
+    for (void* p : {(void*)tw, (void*)one, (void*)spec, (void*)weight, (void*)images})
+        if (p) (void)hipFree(p);
+    tw = one = spec = nullptr;
     weight = images = nullptr;
     N = cap = 0;
 }
@@ -563,16 +564,16 @@ artia_status ctf_slab_filter(artia_ctx* ctx, float* img, int W, int H, size_t pi
     const int N = W > H ? W : H;
     if (fft2d_supports(N) && fft2d_fits(H, pitch) && fft2d_fits(H, out_pitch) && ctx->numerics == ARTIA_NUMERICS_EXACT) {
         FftOwn& f = ctx->ffto;
-        const artia_status so = f.ensure(ctx, N);
+        const artia_status so = f.ensure(ctx, N, FftOwn::kOne | (corners ? FftOwn::kWeight : 0));
         if (so != ARTIA_OK) return so;
         if (corners) {
             launch_crop_border(ctx, W, H, pitch, img, cut, dim, corners);
             hipLaunchKernelGGL(square_weight_kernel, grid2d(N, N), dim3(64, 4), 0, ctx->stream, f.weight, N, W, H,
                                (N - W) / 2, (N - H) / 2, make_crop_params(cut, dim, corners));
         }
-        fft2d_rows_square(ctx, N, f.tw, square_source(img, 0, W, H, pitch, N), f.spec, 1);
-        fft2d_cols_ctf(ctx, N, f.tw, f.spec, make_ctf_stack(N, p, &dmin_nm, &dmax_nm, angle_deg, forFP, 1), 1);
-        fft2d_rows_store(ctx, N, f.tw, f.spec,
+        fft2d_rows_square(ctx, N, f.tw, square_source(img, 0, W, H, pitch, N), f.one, 1);
+        fft2d_cols_ctf(ctx, N, f.tw, f.one, make_ctf_stack(N, p, &dmin_nm, &dmax_nm, angle_deg, forFP, 1), 1);
+        fft2d_rows_store(ctx, N, f.tw, f.one,
                          square_target(out, 0, W, H, out_pitch, N, corners ? f.weight : nullptr, accumulate), 1);
         return check_hip(ctx, hipGetLastError(), "slab filter");
     }
@@ -678,7 +679,7 @@ artia_status wbp_filter(artia_ctx* ctx, const float* img, int W, int H, size_t p
     const int N = W > H ? W : H;
     if (fft2d_supports(N) && fft2d_fits(H, pitch) && fft2d_fits(H, out_pitch) && ctx->numerics == ARTIA_NUMERICS_EXACT) {
         FftOwn& f = ctx->ffto;
-        const artia_status so = f.ensure(ctx, N);
+        const artia_status so = f.ensure(ctx, N, FftOwn::kOne);
         if (so != ARTIA_OK) return so;
         RowSrc s = square_source(nullptr, 0, W, H, pitch, N);
         s.raw = img;
@@ -689,9 +690,9 @@ artia_status wbp_filter(artia_ctx* ctx, const float* img, int W, int H, size_t p
         const float ang = -psi_deg / 180.0f * kPiF;
         pf.sn[0] = sin((double)ang);
         pf.cs[0] = cos((double)ang);
-        fft2d_rows_prep(ctx, N, f.tw, s, f.spec, 1);
-        fft2d_cols_prep(ctx, N, f.tw, f.spec, pf, 1);
-        fft2d_rows_store(ctx, N, f.tw, f.spec, square_target(out, 0, W, H, out_pitch, N, nullptr, 0), 1);
+        fft2d_rows_prep(ctx, N, f.tw, s, f.one, 1);
+        fft2d_cols_prep(ctx, N, f.tw, f.one, pf, 1);
+        fft2d_rows_store(ctx, N, f.tw, f.one, square_target(out, 0, W, H, out_pitch, N, nullptr, 0), 1);
         return check_hip(ctx, hipGetLastError(), "wbp filter");
     }
     artia_status st = ctx->fft.ensure(ctx, N);

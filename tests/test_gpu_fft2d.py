@@ -228,3 +228,33 @@ def test_prepared_squares_have_no_mean(ctx, N):
     got = out[0].double()
     assert abs(float(got.mean())) <= 1e-6
     assert float(got.std(unbiased=False)) == pytest.approx(1.0, rel=1e-5)
+
+
+def test_filters_take_the_memory_they_use(gpu):
+    """A context holds one spectrum (2048: 17 MB) and the crop weights (17 MB) for single images, and 33 spectra
+    (555 MB) for a stack that is prepared; the slab images (537 MB) are the summed slabs' alone."""
+    N = 2048
+    print(f"filter memory {N}", flush=True)
+    p = A.ctf_params(pixelsize_nm=0.5)
+    pp = A.prep_params(dtype="float32", normalization="std", lp=0.4 * N, lps=0.05 * N)
+
+    def used(c, n, what):
+        img, out = torch.ones((2, n, n), device="cuda"), torch.zeros((2, n, n), device="cuda")
+        torch.cuda.synchronize()
+        before = torch.cuda.mem_get_info()[0]
+        if what == "wbp":
+            c.wbp_filter(img[0], out[0], 1.0)
+        elif what == "slab":
+            c.ctf_slab_filter(img[0], out[0], [0, n - 1, n - 1, n - 1, 0, 0, n - 1, 0], p, 3000.0, 3100.0, 0.0,
+                              dim_length=(2.0, 2.0))
+        else:
+            c.prepare_projections(pp, img, out)
+        torch.cuda.synchronize()
+        return before - torch.cuda.mem_get_info()[0]
+
+    for what, gate in (("wbp", 48), ("slab", 64), ("prepare", 640)):
+        c = A.ArtiaContext(0)
+        used(c, 128, what)   # kernels loaded
+        took = used(c, N, what)
+        c.close()
+        assert took <= gate << 20, (what, took >> 20)
