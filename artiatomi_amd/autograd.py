@@ -106,7 +106,7 @@ def _bb_descent(grad_at, s0: torch.Tensor, steps: int, first_step_px: float, max
     g = grad_at(s)
     if callback:
         callback(1, s)
-    gn = g.norm(dim=1, keepdim=True)
+    gn = gmax = g.norm(dim=1, keepdim=True)
     alpha = torch.where(gn > 0, first_step_px / gn.clamp_min(1e-300), torch.zeros_like(gn))
     for k in range(steps - 1):
         d = alpha * g
@@ -116,10 +116,11 @@ def _bb_descent(grad_at, s0: torch.Tensor, steps: int, first_step_px: float, max
         g_new = grad_at(s_new)
         ds, dg = s_new - s, g_new - g
         den = (ds * dg).sum(1, keepdim=True)
-        # at the optimum dg is rounding alone and den may be any small number: a step length grows at
-        # most 100-fold, so that such a row stays near its optimum
-        alpha = torch.where(den > 0, torch.minimum((ds * ds).sum(1, keepdim=True) / den.clamp_min(1e-300),
-                                                   100.0 * alpha), alpha)
+        # a change of the gradient below the float rounding of the row's largest one says nothing about the
+        # curvature (den may be any small number, and the step length with it): the step length stays
+        gmax = torch.maximum(gmax, g_new.norm(dim=1, keepdim=True))
+        known = (den > 0) & (dg.norm(dim=1, keepdim=True) > 1e-7 * gmax)
+        alpha = torch.where(known, (ds * ds).sum(1, keepdim=True) / den.clamp_min(1e-300), alpha)
         s, g = s_new, g_new
         if callback:
             callback(k + 2, s)
