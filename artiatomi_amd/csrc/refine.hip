@@ -355,8 +355,8 @@ __global__ void __launch_bounds__(256) pair_adjoint_slab_kernel(PairArgs a, AdjS
 // and walks exactly the sub-rays of its tilts that lie there, each once and over its whole length (a z
 // slab sets every sub-ray of every tilt up again for each slab, 65 times for 64 layers).  The rows'
 // voxel planes are in LDS in double, padded by the clamp border, and reach the gradient with one atomic
-// per voxel and run.  Lanes run along the detector axis on which y changes less: a wave's rays lie a
-// pixel apart in one row and rarely add to one voxel at once.  The planes leave room for one workgroup on a
+// per voxel and run.  Lanes run along the detector axis on which y changes less, over the pixels of the run, and on
+// along the other: a wave's rays lie a pixel apart and rarely add to one voxel at once.  The planes leave room for one workgroup on a
 // compute unit, so it has sixteen waves to cover the LDS additions (a wave's ds_add_f64 takes nine cycles).
 // 100 cubes of 64^3 by 41 tilts: 19.7 ms (22.2 with eight waves), against 156 ms with z slabs and eight
 // additions per cell.
@@ -407,19 +407,34 @@ __global__ void __launch_bounds__(kAdjFlatThreads) pair_adjoint_flat_kernel(Pair
         const bool along_x = fabs(gx) <= fabs(gy);
         const int ni = along_x ? P.w : P.h, nj = along_x ? P.h : P.w;   // lanes along i
         const double gi = along_x ? gx : gy, gj = along_x ? gy : gx;
-        // the j whose sub-rays reach y in [ys, ys + L) for some i (the first and last rows also take what
-        // lies below and above the volume): y00 + i gi + j gj, a pixel of margin
+        // y of the run's sub-rays: [ys, ys + L), the first and last rows to the volume's faces (a ray beyond them
+        // misses it); tol is far above the rounding of texel_y and of the row's first pixel
+        constexpr double tol = 1e-2;
+        const double lo = (ys <= -1 ? -0.5 : (double)ys) - tol - y00;
+        const double hi = (ys + L >= v.ny ? ((double)v.bbMax[1] - (double)v.bbMin[1]) * ysc - 0.5 : (double)(ys + L)) + tol - y00;
+        // a sub-ray's y is i gi + j gj and its offset in the pixel, om .. oM: the j with such sub-rays for some i,
+        const double om = fmin(0.25 * gx, 0.75 * gx) + fmin(0.25 * gy, 0.75 * gy);
+        const double oM = fmax(0.25 * gx, 0.75 * gx) + fmax(0.25 * gy, 0.75 * gy);
         int j0 = 0, j1 = nj - 1;
         if (fabs(gj) > 1e-3) {
-            const double lo = (ys <= -1 ? -1e9 : (double)ys) - y00 - fmax(0.0, gi * ni),
-                         hi = (ys + L >= v.ny ? 1e9 : (double)(ys + L)) - y00 - fmin(0.0, gi * ni);
-            const double a0 = fmin(lo / gj, hi / gj), a1 = fmax(lo / gj, hi / gj);
-            j0 = (int)fmax(0.0, fmin((double)nj, floor(a0) - 2.0));
-            j1 = (int)fmin((double)(nj - 1), fmax(-1.0, ceil(a1) + 1.0));
+            const double l = lo - oM - fmax(0.0, gi * (ni - 1)), h = hi - om - fmin(0.0, gi * (ni - 1));
+            const double a0 = fmin(l / gj, h / gj), a1 = fmax(l / gj, h / gj);
+            j0 = (int)fmax(0.0, fmin((double)nj, ceil(a0)));
+            j1 = (int)fmin((double)(nj - 1), fmax(-1.0, floor(a1)));
         }
-        const int total = ni * (j1 - j0 + 1) * 4;
+        // and of each j the `row` pixels i from the first with sub-rays in the run, so that a wave's lanes are rays
+        // of the run also where the detector's axes are oblique to y (all ni pixels of a row kept a few of 64
+        // lanes busy at 45 degrees: 12 cubes of 94^3 by 21 tilts 122 ms, 11.6 so; by z slabs 59 ms)
+        const bool part = fabs(gi) > 1e-3;
+        const double inv = part ? 1.0 / gi : 0.0, edge = gi > 0.0 ? lo - oM : hi - om;
+        const int row = wave_uniform(part ? (int)fmax(0.0, fmin((double)ni, floor((hi - lo + (oM - om)) * fabs(inv)) + 1.0)) : ni);
+        const int nrow = wave_uniform(j1 - j0 + 1), total = row * nrow * 4;
+        const float start = wave_uniform((float)(edge * inv - gj * inv * j0)), slope = wave_uniform((float)(gj * inv));
+        j0 = wave_uniform(j0);
         for (int idx = (int)threadIdx.x; idx < total; idx += kAdjFlatThreads) {
-            const int rest = idx / ni, i = idx - rest * ni, sub = rest & 3, j = j0 + (rest >> 2);
+            const int rest = idx / row, sub = rest / nrow, jj = rest - sub * nrow, j = j0 + jj;
+            const int i = idx - rest * row + (int)ceilf(start - slope * (float)jj);   // (+ 0 without part)
+            if (i < 0 || i >= ni) continue;
             const int wx = along_x ? i : j, wy = along_x ? j : i;
             const double pxd = (double)(P.x0 + wx) + ((sub & 2) ? 0.75 : 0.25);
             const double pyd = (double)(P.y0 + wy) + ((sub & 1) ? 0.75 : 0.25);

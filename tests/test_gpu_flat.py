@@ -93,6 +93,14 @@ def test_pair_adjoint_is_the_transpose(ctx, n, psi):
     ps.close()
 
 
+@pytest.mark.parametrize("n", [64, 94, 95])
+@pytest.mark.parametrize("psi", [-45.0, 10.0, 135.0])
+def test_pair_adjoint_rows_oblique_to_the_detector(ctx, n, psi):
+    """Runs of y rows that cross the detector obliquely, with four planes (64), the last size with two (94) and the
+    first without (95)."""
+    test_pair_adjoint_is_the_transpose(ctx, n, psi)
+
+
 def march_given_samples(vg, g, vol, W, H):
     """Projection in float64 at the walk's own sample lattice: its float start and step of every sub-ray."""
     f = lambda a: np.array(list(a), np.float64)  # noqa: E731
