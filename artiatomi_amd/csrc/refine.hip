@@ -93,7 +93,10 @@ __device__ __forceinline__ void block_sum3(double& a, double& b, double& c) {
 // last round (4100 windows of 80 x 94: 15.3 -> 14.0 ms; two parts 14.4, eight 13.9) and a short list of
 // pairs.  The other modes sum over the pair's pixels in one workgroup.
 constexpr int kPairParts = 4;
-template <int kMode>
+// kFlat: the pairs whose rays have no y component (n_y == 0 after flat_beam), otherwise the others.  A kernel for
+// each, because one with both walks spills the registers of the longer one in the other too (500 cubes' loss
+// and gradient with a y component 36.6 ms alone, 44.2 together with the flat walk).
+template <int kMode, bool kFlat>
 __global__ void __launch_bounds__(256, 5) pair_march_kernel(PairArgs a) {
     __shared__ float chunk[kChunkFloats];
     __shared__ int zr[2];
@@ -102,6 +105,7 @@ __global__ void __launch_bounds__(256, 5) pair_march_kernel(PairArgs a) {
     if (slot >= a.npairs) return;   // whole workgroup
     const int p = a.order[slot];
     const PairDev& P = a.pairs[p];
+    if ((P.g.n[1] == 0.0f) != kFlat) return;   // whole workgroup: the other kernel's pair
     const int x0 = P.x0, y0 = P.y0, w = P.w, h = P.h;
     const long long io = P.img_offset;
     const int lane = (int)(threadIdx.x & 63), wave = (int)(threadIdx.x >> 6);
@@ -140,8 +144,7 @@ __global__ void __launch_bounds__(256, 5) pair_march_kernel(PairArgs a) {
             if (kMode != kProject) cell_grad_sum(val, cm, G);
         };
         const double pi0 = (double)(x0 + (t % ntx) * 8), pj0 = (double)(y0 + (t / ntx) * 8);
-        // rays without a y component (n_y == 0 after flat_beam; block-uniform: one pair per block)
-        if (g.n[1] == 0.0f) {
+        if constexpr (kFlat) {
             float dq[3];
             tube_step(v, g, step, dq);
             const FlatDir d = flat_dir(dq);
@@ -809,6 +812,7 @@ struct artia_pairs {
     PairDev* pairs = nullptr;
     int* order = nullptr;
     int npairs = 0, per_xcd = 0;
+    bool any_flat = false, any_other = false;   // pairs with and without n_y == 0
     // the summed adjoint (pair_adjoint_flat_kernel when every pair's rays are flat, otherwise
     // pair_adjoint_slab_kernel): work items and per-volume slot ranges, or none when a sub-volume's
     // planes do not fit or a tilt runs parallel to its z layers
@@ -836,6 +840,13 @@ PairArgs base_args(const artia_pairs* ps) {
 }
 
 dim3 pair_grid(const artia_pairs* ps, int parts = 1) { return dim3((unsigned)(8 * ps->per_xcd * parts)); }
+
+template <int kMode>
+void launch_march(const artia_pairs* ps, const PairArgs& a) {
+    const dim3 grid = pair_grid(ps, kMode == kProject ? kPairParts : 1);
+    if (ps->any_flat) hipLaunchKernelGGL((pair_march_kernel<kMode, true>), grid, dim3(256), 0, ps->ctx->stream, a);
+    if (ps->any_other) hipLaunchKernelGGL((pair_march_kernel<kMode, false>), grid, dim3(256), 0, ps->ctx->stream, a);
+}
 
 }  // namespace
 
@@ -896,8 +907,9 @@ artia_status artia_pairs_create(artia_ctx* ctx, const artia_pair_volume* volumes
     bool slab_ok = ctx->march_lds, flat = ctx->march_lds;
     for (int p = 0; p < npairs; p++) {
         slab_ok = slab_ok && std::fabs(host[(size_t)p].g.n[2]) > 1e-3f;   // rays cross the z layers
-        flat = flat && host[(size_t)p].g.n[1] == 0.0f;
+        (host[(size_t)p].g.n[1] == 0.0f ? ps->any_flat : ps->any_other) = true;
     }
+    flat = flat && !ps->any_other;
     for (int vi = 0; vi < nvol && flat; vi++)
         flat = vcount[(size_t)vi] == 0 || adj_flat_planes(volumes[vi].geom.nx, volumes[vi].geom.nz) > 0;
     slab_ok = slab_ok || flat;
@@ -983,7 +995,7 @@ artia_status artia_pairs_project(artia_pairs* ps, const float* volumes, const do
     a.shifts = shifts;
     a.out = images;
     Timing t(ctx, ms);
-    hipLaunchKernelGGL(pair_march_kernel<kProject>, pair_grid(ps, kPairParts), dim3(256), 0, ctx->stream, a);
+    launch_march<kProject>(ps, a);
     artia_status st = check_hip(ctx, hipGetLastError(), "artia_pairs_project launch");
     if (st != ARTIA_OK) return st;
     return t.finish();
@@ -1004,7 +1016,7 @@ artia_status artia_pairs_loss_grad(artia_pairs* ps, const float* volumes, const 
     a.grad = grad;
     a.normal = normal;
     Timing t(ctx, ms);
-    hipLaunchKernelGGL(pair_march_kernel<kLossGrad>, pair_grid(ps), dim3(256), 0, ctx->stream, a);
+    launch_march<kLossGrad>(ps, a);
     artia_status st = check_hip(ctx, hipGetLastError(), "artia_pairs_loss_grad launch");
     if (st != ARTIA_OK) return st;
     return t.finish();
@@ -1022,7 +1034,7 @@ artia_status artia_pairs_shift_grad(artia_pairs* ps, const float* volumes, const
     a.in = weights;
     a.grad = grad;
     Timing t(ctx, ms);
-    hipLaunchKernelGGL(pair_march_kernel<kShiftGrad>, pair_grid(ps), dim3(256), 0, ctx->stream, a);
+    launch_march<kShiftGrad>(ps, a);
     artia_status st = check_hip(ctx, hipGetLastError(), "artia_pairs_shift_grad launch");
     if (st != ARTIA_OK) return st;
     return t.finish();
