@@ -364,8 +364,8 @@ __device__ __forceinline__ void flat_layers(const VolG& v, int* zr, int za, int 
 // Called by all 256 threads of the block; chunk holds kChunkFloats floats and zr two ints of shared
 // memory.  The steps and values are flat_walk_direct's, so sums are bit-identical to it.  kGrad: f uses
 // the y differences.  kAhead: the next slab's voxels are loaded into
-// registers during the walk (the march: 1.80 -> 1.63 ms per 1024x1024x256 tilt; the segments and the pair
-// projection, short of registers, lose by it).
+// registers during the walk (the march: 1.80 -> 1.63 ms per 1024x1024x256 tilt; the segments, the pair
+// projection and the pairs' shift gradient lose by it).
 template <bool kGrad, bool kAhead, typename T, class F>
 __device__ __forceinline__ void flat_tube_walk(const VolG& v, const T* __restrict__ vol, float* __restrict__ chunk,
                                                int* zr, const TubePlan& tp, const TubeBox& tb, const float dq[3],

@@ -88,16 +88,18 @@ __device__ __forceinline__ void block_sum3(double& a, double& b, double& c) {
 }
 
 // Five waves per SIMD (96 registers, a few spilled): measured faster than the unconstrained
-// allocation (3-4 waves) for the LDS-staged walk.
+// allocation (3-4 waves) for the LDS-staged walk.  The flat walk with gradients takes four (128 registers): at five
+// it spilled 200 to 320 bytes a lane (40 cubes of 64^3 by 21 tilts, loss and gradient 7.26 -> 5.32 ms, shift gradient
+// 5.47 -> 4.61; 200 of 16^3 by 11 1.23 -> 0.80 and 0.91 -> 0.54).
 // Projections alone (kProject) split a pair's tiles over kPairParts workgroups: shorter ones fill the chip's
 // last round (4100 windows of 80 x 94: 15.3 -> 14.0 ms; two parts 14.4, eight 13.9) and a short list of
 // pairs.  The other modes sum over the pair's pixels in one workgroup.
 constexpr int kPairParts = 4;
 // kFlat: the pairs whose rays have no y component (n_y == 0 after flat_beam), otherwise the others.  A kernel for
-// each, because one with both walks spills the registers of the longer one in the other too (500 cubes' loss
-// and gradient with a y component 36.6 ms alone, 44.2 together with the flat walk).
+// each, because one with both walks spills the registers of the longer one in the other too (4 cubes of 128^3 by
+// 11 tilts with a y component, loss and gradient: 36.5 ms alone, 44.2 together with the flat walk).
 template <int kMode, bool kFlat>
-__global__ void __launch_bounds__(256, 5) pair_march_kernel(PairArgs a) {
+__global__ void __launch_bounds__(256, kMode != kProject && kFlat ? 4 : 5) pair_march_kernel(PairArgs a) {
     __shared__ float chunk[kChunkFloats];
     __shared__ int zr[2];
     constexpr int kParts = kMode == kProject ? kPairParts : 1;
@@ -155,8 +157,8 @@ __global__ void __launch_bounds__(256, 5) pair_march_kernel(PairArgs a) {
             };
             if (P.staged) {   // uniform: the whole block walks the tile's tube through LDS
                 const TubeBox tb = tube_box(v, g, P.tp, pi0 + 0.25, pi0 + 7.75, pj0 + 0.25, pj0 + 7.75, sx, sy);
-                flat_tube_walk<kMode != kProject, kMode != kProject>(v, a.vols + P.vol_offset, chunk, zr, P.tp, tb, dq, s.q0, s.count,
-                                                  flat_fn);
+                flat_tube_walk<kMode != kProject, kMode == kLossGrad>(v, a.vols + P.vol_offset, chunk, zr, P.tp, tb, dq, s.q0,
+                                                                      s.count, flat_fn);
             } else if (ok) {
                 FlatWalker fw;
                 fw.init(d, s.q0, s.count);
