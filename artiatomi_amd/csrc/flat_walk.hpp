@@ -128,58 +128,51 @@ __device__ __forceinline__ float flat_edge(float v0, float v1, float b, float& d
     return __builtin_fmaf(b, dy, v0);
 }
 
-// The walk with every edge read from the volume (clamp addressing): all steps while go(), the path of
+// The walk with its edges read from the volume (clamp addressing): all steps while go(), the path of
 // unstaged volumes and of lanes whose cells leave a staged box.  f(A, B, C, D, yA, yB, yC, yD, a, c, m).
+// A step keeps the two edges it shares with the one before and reads the other two.
 // kBig: 64-bit addresses; otherwise buffer loads at 32-bit offsets (below 2^30 voxels, z * ny + y and x
 // below 2^24).
 template <bool kBig, typename T, class Go, class F>
 __device__ __forceinline__ void flat_walk_direct(const VolG& v, const T* __restrict__ vol, const FlatDir& d,
                                                  const float q0[3], FlatWalker& w, Go&& go, F&& f) {
+    if (!(w.active() && go())) return;
     const float yf = floorf(q0[1]), b = q0[1] - yf;
     const int y0 = clampi((int)yf, 0, v.ny - 1), y1 = clampi((int)yf + 1, 0, v.ny - 1);
-    const int most = 4 * (int)w.count + 64;   // every step takes samples or advances an axis
-    for (int guard = 0; guard < most && w.active() && go(); guard++) {
-        const int xn = w.near(d, q0, 0), zn = w.near(d, q0, 1);
-        const int x0 = clampi(d.sgn[0] * xn, 0, v.nx - 1), x1 = clampi(d.sgn[0] * (xn + 1), 0, v.nx - 1);
-        const int z0 = clampi(d.sgn[1] * zn, 0, v.nz - 1), z1 = clampi(d.sgn[1] * (zn + 1), 0, v.nz - 1);
-        float val[8];   // (x0 y0 z0), (x0 y1 z0), (x1 ..), then z1
+    auto edge = [&](int xo, int zo, float& dy) {   // oriented lattice indices
+        const int x = clampi(d.sgn[0] * xo, 0, v.nx - 1), z = clampi(d.sgn[1] * zo, 0, v.nz - 1);
         if (kBig) {
-            const size_t r00 = ((size_t)z0 * (size_t)v.ny + (size_t)y0) * (size_t)v.nx;
-            const size_t r10 = ((size_t)z0 * (size_t)v.ny + (size_t)y1) * (size_t)v.nx;
-            const size_t r01 = ((size_t)z1 * (size_t)v.ny + (size_t)y0) * (size_t)v.nx;
-            const size_t r11 = ((size_t)z1 * (size_t)v.ny + (size_t)y1) * (size_t)v.nx;
-            val[0] = vox(vol, r00 + (size_t)x0);
-            val[1] = vox(vol, r10 + (size_t)x0);
-            val[2] = vox(vol, r00 + (size_t)x1);
-            val[3] = vox(vol, r10 + (size_t)x1);
-            val[4] = vox(vol, r01 + (size_t)x0);
-            val[5] = vox(vol, r11 + (size_t)x0);
-            val[6] = vox(vol, r01 + (size_t)x1);
-            val[7] = vox(vol, r11 + (size_t)x1);
-        } else {
-            const __amdgpu_buffer_rsrc_t rs = volume_rsrc(vol, v);
-            const uint32_t e = (uint32_t)sizeof(T);
-            auto row = [&](int z, int y) {
-                return __umul24(__umul24((uint32_t)z, (uint32_t)v.ny) + (uint32_t)y, (uint32_t)v.nx);
-            };
-            const uint32_t r00 = row(z0, y0), r10 = row(z0, y1), r01 = row(z1, y0), r11 = row(z1, y1);
-            val[0] = buffer_vox(rs, (r00 + (uint32_t)x0) * e, vol);
-            val[1] = buffer_vox(rs, (r10 + (uint32_t)x0) * e, vol);
-            val[2] = buffer_vox(rs, (r00 + (uint32_t)x1) * e, vol);
-            val[3] = buffer_vox(rs, (r10 + (uint32_t)x1) * e, vol);
-            val[4] = buffer_vox(rs, (r01 + (uint32_t)x0) * e, vol);
-            val[5] = buffer_vox(rs, (r11 + (uint32_t)x0) * e, vol);
-            val[6] = buffer_vox(rs, (r01 + (uint32_t)x1) * e, vol);
-            val[7] = buffer_vox(rs, (r11 + (uint32_t)x1) * e, vol);
+            const size_t o = ((size_t)z * (size_t)v.ny + (size_t)y0) * (size_t)v.nx + (size_t)x;
+            return flat_edge(vox(vol, o), vox(vol, o + (size_t)(y1 - y0) * (size_t)v.nx), b, dy);
         }
-        float yA, yB, yC, yD;
-        const float A = flat_edge(val[0], val[1], b, yA), B = flat_edge(val[2], val[3], b, yB);
-        const float C = flat_edge(val[4], val[5], b, yC), D = flat_edge(val[6], val[7], b, yD);
+        const __amdgpu_buffer_rsrc_t rs = volume_rsrc(vol, v);
+        const uint32_t e = (uint32_t)sizeof(T);
+        const uint32_t o = __umul24(__umul24((uint32_t)z, (uint32_t)v.ny) + (uint32_t)y0, (uint32_t)v.nx) + (uint32_t)x;
+        return flat_edge(buffer_vox(rs, o * e, vol), buffer_vox(rs, (o + (uint32_t)(y1 - y0) * (uint32_t)v.nx) * e, vol),
+                         b, dy);
+    };
+    int xf = w.near(d, q0, 0) + 1, zf = w.near(d, q0, 1) + 1;   // the current cell's far indices
+    float yA, yB, yC, yD;
+    float A = edge(xf - 1, zf - 1, yA), B = edge(xf, zf - 1, yB), C = edge(xf - 1, zf, yC), D = edge(xf, zf, yD);
+    const int most = 4 * (int)w.count + 64;   // every step takes samples or advances an axis
+    for (int guard = 1;; guard++) {
         const bool ax = w.kb[0] < w.kb[1];
         float a, c;
         const float m = w.samples(d, ax ? w.kb[0] : w.kb[1], a, c);
         f(A, B, C, D, yA, yB, yC, yD, a, c, m);
         w.advance(d, ax);
+        if (!(guard < most && w.active() && go())) break;
+        xf += ax ? 1 : 0;
+        zf += ax ? 0 : 1;
+        float yN, yE = yD;
+        const float N = edge(ax ? xf : xf - 1, ax ? zf - 1 : zf, yN), E = D;
+        D = edge(xf, zf, yD);
+        A = ax ? B : C;
+        B = ax ? N : E;
+        C = ax ? E : N;
+        yA = ax ? yB : yC;
+        yB = ax ? yN : yE;
+        yC = ax ? yE : yN;
     }
 }
 
