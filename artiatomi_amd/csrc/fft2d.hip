@@ -205,19 +205,21 @@ struct Plan;
         }                                                                                            \
     };
 ARTIA_FFT_PLAN3(128, 8, 8, 8, 2)
-ARTIA_FFT_PLAN3(256, 16, 16, 16, 1)
+ARTIA_FFT_PLAN3(256, 8, 8, 8, 4)
 ARTIA_FFT_PLAN3(512, 8, 8, 8, 8)
 ARTIA_FFT_PLAN3(1024, 16, 16, 16, 4)
 ARTIA_FFT_PLAN3(2048, 16, 16, 16, 8)
 ARTIA_FFT_PLAN3(4096, 16, 16, 16, 16)
 #undef ARTIA_FFT_PLAN3
 
-// Complex transforms (row pairs, or columns) per block: up to 512 threads and 70 KB of LDS, two blocks
-// on a compute unit.
+// Complex transforms (row pairs, or columns) per block: four, or two of 4096 (70 KB of LDS, two blocks on a compute
+// unit).  Blocks of 512 threads left one small image a handful of them, each thread with its points' CTF factors
+// in turn: a 256 x 256 slab filter took 45 us with five blocks of columns, 29.5 with 33 (and eight points a thread
+// instead of 16; 31 with library transforms); 40 images of 1024 x 1024 prepared 466 -> 414 us.
 template <int N>
 struct Shape {
     static constexpr int E = Plan<N>::E, T = Plan<N>::T;
-    static constexpr int F = (512 / T) * padded(N) * 8 > 71000 ? 71000 / (padded(N) * 8) : 512 / T;   // row pairs
+    static constexpr int F = 512 / T < 4 ? 512 / T : 4;   // row pairs
     static constexpr int threads = F * T;
     static constexpr int rows = 2 * F;
     static constexpr int pairs = F / 2;   // pairs of columns per column block
