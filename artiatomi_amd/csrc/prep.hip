@@ -313,7 +313,7 @@ artia_status artia_prepare_projections(artia_ctx* ctx, const artia_prep_params* 
     // Not with a high pass and the mean as divisor, where a frequency 0 filtered to nothing would be divided by.
     const bool fromSpectrum = own && !pp->wbp && width == N && height == N &&
                               (pp->normalization == ARTIA_NORM_STD ||
-                               (pp->normalization == ARTIA_NORM_MEAN && (pp->skip_filter || !(pp->hp > 0.0f))));
+                               (pp->normalization == ARTIA_NORM_MEAN && !(pp->hp > 0.0f)));
     const int waves = fromSpectrum ? fft2d_col_waves(N) : 0;
     // workspace: partial sums of a chunk, then the per-projection state and, behind it, the squares' means
     const size_t partFloats = (size_t)cap * (size_t)std::max(kRedBlocks, std::max(2 * rowBlocks, waves)) * 2;
@@ -337,7 +337,7 @@ artia_status artia_prepare_projections(artia_ctx* ctx, const artia_prep_params* 
                                        ctx->stream),
                    "hipMemcpyAsync(projection state)");
     if (st != ARTIA_OK) return st;
-    const size_t plane = (size_t)N * N, half = (size_t)(N / 2 + 1);
+    const size_t half = (size_t)(N / 2 + 1);
     const size_t istride = (size_t)height * pitch, ostride = (size_t)height * out_pitch;
     const int bx = (N - width) / 2, by = (N - height) / 2;
     const float pixA = pp->pixelsize_nm * 10.0f;

@@ -40,8 +40,8 @@ struct TubePlan {
 // span: the tile's extent in pixels between its outermost sub-rays (7.5 for 8 pixels at offsets
 // 0.25 .. 7.75); slab: cell layers per slab.
 inline bool tube_plan(const VolG& v, const TiltG& g, TubePlan& tp, double span = 7.5, int slab = kSlabCells) {
-    // (nz bounded so that the walk's float box offsets stay exact: |cell z * CXY| < 2^24, CXY being
-    // at most kChunkFloats / 2)
+    // (volumes of more than 6550 layers walk from memory, as they always have; no index of the staged walks asks
+    // for it any more)
     if (v.nx < 2 || v.ny < 2 || v.nz < 2 || (long long)(v.nz + 2) * (kChunkFloats / 2) >= (1LL << 24)) return false;
     if ((long long)v.nx * v.ny >= (1LL << 30)) return false;   // 32-bit byte offsets within a layer
     double sc[3], N[3], dpx[3], dpy[3];

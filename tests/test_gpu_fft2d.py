@@ -218,7 +218,7 @@ def test_ctf_factor_near_its_zeros(ctx):
 def test_prepared_squares_have_no_mean(ctx, N):
     """A square whose mean is 30000 times its deviation: the normalised image has none of it left.  Without
     frequency 0 a pixel's error is a few 2^-24 of the deviation 1, independent of the others' or a bias of that
-    size: gate 1e-6.  (The mean subtracted from float pixels left up to half a unit of its last place, 1e-3.)"""
+    size: gate 1e-6.  (Subtracted from pixels of its size, 2^-9 apart, it left their rounding in the deviation.)"""
     print(f"mean of a prepared square {N}", flush=True)
     img = (30000.3 + white(N, N, 11)).astype(np.float32)
     out = torch.zeros((1, N, N), device="cuda")
