@@ -43,7 +43,8 @@ struct FftBatch {
 
 // The three-kernel filters' state (fft2d.hpp), each buffer allocated when a filter first needs it and kept, where
 // it is, until N changes: twiddles exp(-2 pi i k / N), one half spectrum for single images, cap + 1 for stacks, an
-// N x N image of crop weights and cap slab images that wait to be summed.
+// N x N image of crop weights (with the spectrum of single images too, so that after any of their filters the
+// others allocate nothing and can be captured) and cap slab images that wait to be summed.
 struct FftOwn {
     enum { kOne = 1, kStack = 2, kWeight = 4, kImages = 8 };
     int N = 0, cap = 0;

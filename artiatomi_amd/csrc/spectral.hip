@@ -514,6 +514,7 @@ artia_status FftOwn::ensure(artia_ctx* ctx, int n, int buffers) {
         cap = (int)std::min<size_t>((size_t)kFftBatchMax, std::max<size_t>(1, ((size_t)544 << 20) / spectrum));
     }
     if ((buffers & kOne) && !one) st = check_hip(ctx, hipMalloc(&one, spectrum), "hipMalloc(spectrum)");
+    if (buffers & kOne) buffers |= kWeight;
     if (st == ARTIA_OK && (buffers & kStack) && !spec)
         st = check_hip(ctx, hipMalloc(&spec, (size_t)(cap + 1) * spectrum), "hipMalloc(spectra)");
     if (st == ARTIA_OK && (buffers & kWeight) && !weight)
@@ -564,7 +565,7 @@ artia_status ctf_slab_filter(artia_ctx* ctx, float* img, int W, int H, size_t pi
     const int N = W > H ? W : H;
     if (fft2d_supports(N) && fft2d_fits(H, pitch) && fft2d_fits(H, out_pitch) && ctx->numerics == ARTIA_NUMERICS_EXACT) {
         FftOwn& f = ctx->ffto;
-        const artia_status so = f.ensure(ctx, N, FftOwn::kOne | (corners ? FftOwn::kWeight : 0));
+        const artia_status so = f.ensure(ctx, N, FftOwn::kOne);
         if (so != ARTIA_OK) return so;
         if (corners) {
             launch_crop_border(ctx, W, H, pitch, img, cut, dim, corners);

@@ -258,3 +258,37 @@ def test_filters_take_the_memory_they_use(gpu):
         took = used(c, N, what)
         c.close()
         assert took <= gate << 20, (what, took >> 20)
+
+
+def test_single_image_filters_in_a_captured_graph(gpu):
+    """After one single-image filter the others of its size allocate nothing: captured, and replayed with new images
+    between eager calls, they give the eager results."""
+    N = 256
+    print(f"captured filters {N}", flush=True)
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        c = A.ArtiaContext(0)
+    p, corners = A.ctf_params(pixelsize_nm=0.5), [0, N - 1, N - 1, N - 1, 0, 0, N - 1, 0]
+    img, work, out = (torch.zeros((N, N), device="cuda") for _ in range(3))
+
+    def filters(dst):
+        work.copy_(img)
+        c.wbp_filter(work, dst, 1.0, "ramp")
+        c.ctf_slab_filter(work, dst, corners, p, 3000.0, 3100.0, 0.0, accumulate=True, dim_length=(2.0, 2.0))
+
+    with torch.cuda.stream(stream):
+        c.wbp_filter(work, out, 1.0, "ramp")
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            filters(out)
+        for seed in range(4):
+            img.copy_(torch.from_numpy(white(N, N, seed)).cuda())
+            eager = torch.zeros_like(out)
+            filters(eager)
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert float(eager.abs().max()) > 0
+            assert torch.equal(out, eager)
+    c.close()
