@@ -92,8 +92,8 @@ __device__ __forceinline__ void block_sum3(double& a, double& b, double& c) {
 // it spilled 200 to 320 bytes a lane (40 cubes of 64^3 by 21 tilts, loss and gradient 7.26 -> 5.32 ms, shift gradient
 // 5.47 -> 4.61; 200 of 16^3 by 11 1.23 -> 0.80 and 0.91 -> 0.54).
 // Projections alone (kProject) split a pair's tiles over kPairParts workgroups: shorter ones fill the chip's
-// last round (4100 windows of 80 x 94: 15.3 -> 14.0 ms; two parts 14.4, eight 13.9) and a short list of
-// pairs.  The other modes sum over the pair's pixels in one workgroup.
+// last round (4100 windows of 80 x 94: 15.3 -> 14.0 ms, and 12.3 in a kernel of its own; two parts 14.4, eight
+// 13.9) and a short list of pairs.  The other modes sum over the pair's pixels in one workgroup.
 constexpr int kPairParts = 4;
 // kFlat: the pairs whose rays have no y component (n_y == 0 after flat_beam), otherwise the others.  A kernel for
 // each, because one with both walks spills the registers of the longer one in the other too (4 cubes of 128^3 by
@@ -363,7 +363,7 @@ __global__ void __launch_bounds__(256) pair_adjoint_slab_kernel(PairArgs a, AdjS
 // per voxel and run.  Lanes run along the detector axis on which y changes less, over the pixels of the run, and on
 // along the other: a wave's rays lie a pixel apart and rarely add to one voxel at once.  The planes leave room for one workgroup on a
 // compute unit, so it has sixteen waves to cover the LDS additions (a wave's ds_add_f64 takes nine cycles).
-// 100 cubes of 64^3 by 41 tilts: 19.7 ms (22.2 with eight waves), against 156 ms with z slabs and eight
+// 100 cubes of 64^3 by 41 tilts: 19.5 ms (22.2 with eight waves), against 156 ms with z slabs and eight
 // additions per cell.
 constexpr int kAdjFlatThreads = 1024;
 constexpr int kAdjFlatBytes = 144 << 10;   // LDS for the padded planes
