@@ -429,12 +429,14 @@ __global__ void __launch_bounds__(kAdjFlatThreads) pair_adjoint_flat_kernel(Pair
         }
         // and of each j the `row` pixels i from the first with sub-rays in the run, so that a wave's lanes are rays
         // of the run also where the detector's axes are oblique to y (all ni pixels of a row kept a few of 64
-        // lanes busy at 45 degrees: 12 cubes of 94^3 by 21 tilts 122 ms, 11.6 so; by z slabs 59 ms)
-        const bool part = fabs(gi) > 1e-3;
-        const double inv = part ? 1.0 / gi : 0.0, edge = gi > 0.0 ? lo - oM : hi - om;
-        const int row = wave_uniform(part ? (int)fmax(0.0, fmin((double)ni, floor((hi - lo + (oM - om)) * fabs(inv)) + 1.0)) : ni);
+        // lanes busy at 45 degrees: 12 cubes of 94^3 by 21 tilts 122 ms, 11.6 so; by z slabs 59 ms); all ni where
+        // the run is as wide
+        const double inv = fabs(gi) > 1e-3 ? 1.0 / gi : 0.0, wide = floor((hi - lo + (oM - om)) * fabs(inv)) + 1.0;
+        const bool part = inv != 0.0 && wide < (double)ni;
+        const double edge = part ? (gi > 0.0 ? lo - oM : hi - om) * inv : 0.0, step_j = part ? gj * inv : 0.0;
+        const int row = wave_uniform(part ? (int)fmax(0.0, wide) : ni);
         const int nrow = wave_uniform(j1 - j0 + 1), total = row * nrow * 4;
-        const float start = wave_uniform((float)(edge * inv - gj * inv * j0)), slope = wave_uniform((float)(gj * inv));
+        const float start = wave_uniform((float)(edge - step_j * j0)), slope = wave_uniform((float)step_j);
         j0 = wave_uniform(j0);
         for (int idx = (int)threadIdx.x; idx < total; idx += kAdjFlatThreads) {
             const int rest = idx / row, sub = rest / nrow, jj = rest - sub * nrow, j = j0 + jj;

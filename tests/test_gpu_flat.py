@@ -93,11 +93,12 @@ def test_pair_adjoint_is_the_transpose(ctx, n, psi):
     ps.close()
 
 
-@pytest.mark.parametrize("n", [64, 94, 95])
-@pytest.mark.parametrize("psi", [-45.0, 10.0, 135.0])
-def test_pair_adjoint_rows_oblique_to_the_detector(ctx, n, psi):
-    """Runs of y rows that cross the detector obliquely, with four planes (64), the last size with two (94) and the
-    first without (95)."""
+@pytest.mark.parametrize("n", [16, 40, 64, 94, 95])
+@pytest.mark.parametrize("psi", [0.0, 2.0, 4.0, 10.0, 33.0, -45.0, 87.0, -88.0, 135.0])
+def test_staged_pair_adjoint_is_the_transpose(ctx, n, psi):
+    """The same from runs of y rows in LDS: eight planes of rows (16, 40), four (64), the last size with two (94)
+    and the first without (95); runs along a detector axis, wider and narrower than a window, and oblique."""
+    ctx.set_fp_staging(True)
     test_pair_adjoint_is_the_transpose(ctx, n, psi)
 
 
