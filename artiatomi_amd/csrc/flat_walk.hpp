@@ -160,7 +160,7 @@ __device__ __forceinline__ void flat_walk_direct(const VolG& v, const T* __restr
         const bool ax = w.kb[0] < w.kb[1];
         float a, c;
         const float m = w.samples(d, ax ? w.kb[0] : w.kb[1], a, c);
-        f(A, B, C, D, yA, yB, yC, yD, a, c, m);
+        if (m > 0.0f) f(A, B, C, D, yA, yB, yC, yD, a, c, m);   // (0 times an infinite voxel would be NaN)
         w.advance(d, ax);
         if (!(guard < most && w.active() && go())) break;
         xf += ax ? 1 : 0;

@@ -160,3 +160,20 @@ def test_flat_walk_keeps_its_position(ctx, staged):
     err = float((p.double() - ref).norm() / ref.norm())
     print(f"flat position staged {staged}: {err:.2e}", flush=True)
     assert err <= 2e-7
+
+
+def test_direct_walk_reads_infinite_voxels_only_at_samples(ctx):
+    """From memory, a ray that crosses a cell between two of its samples takes nothing from it: exactly the pixels
+    with a sample beside an infinite voxel are not finite."""
+    nx, ny, nz, W, H = 64, 40, 40, 90, 42
+    vg, vol = A.volume_geometry(nx, ny, nz), positive((nz, ny, nx), 12)
+    at = np.random.default_rng(6).integers([4, 2, 4], [36, 38, 60], (60, 3))
+    vol[at[:, 0], at[:, 1], at[:, 2]] = float("inf")
+    ctx.set_fp_staging(False)
+    for tilt in (61.0, -34.0, 17.0):
+        g = A.tilt_geometry(tilt, W, H, shift=(0.3, 0.2))
+        p, d = torch.zeros((H, W), device="cuda"), torch.zeros((H, W), device="cuda")
+        ctx.fp_march(vg, g, vol, p, d)
+        ref = march_given_samples(vg, g, vol, W, H)
+        assert 0 < int((~ref.isfinite()).sum()) < W * H // 2
+        assert torch.equal(p.isfinite(), ref.isfinite()), tilt
