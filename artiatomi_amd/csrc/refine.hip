@@ -157,8 +157,8 @@ __global__ void __launch_bounds__(256, kMode != kProject && kFlat ? 4 : 5) pair_
             };
             if (P.staged) {   // uniform: the whole block walks the tile's tube through LDS
                 const TubeBox tb = tube_box(v, g, P.tp, pi0 + 0.25, pi0 + 7.75, pj0 + 0.25, pj0 + 7.75, sx, sy);
-                flat_tube_walk<kMode != kProject, kMode == kLossGrad>(v, a.vols + P.vol_offset, chunk, zr, P.tp, tb, dq, s.q0,
-                                                                      s.count, flat_fn);
+                flat_tube_walk<kMode != kProject, kMode == kLossGrad>(v, a.vols + P.vol_offset, chunk, zr, P.tp, tb, dq,
+                                                                      s.q0, s.count, flat_fn);
             } else if (ok) {
                 FlatWalker fw;
                 fw.init(d, s.q0, s.count);
@@ -318,8 +318,9 @@ __global__ void __launch_bounds__(256) pair_adjoint_slab_kernel(PairArgs a, AdjS
             const float fin = (float)(sgn[2] > 0 ? zs : ze), fout = (float)(sgn[2] > 0 ? ze : zs);
             // (the first and last slabs also take what a volume stored in part is sampled at beyond its layers)
             const bool bottom = zs <= -1, top = ze >= v.nz;
-            const int kA = (sgn[2] > 0 ? bottom : top) ? 0 : max(0, min(s.count, (int)ceilf(__builtin_fmaf(fin, inv[2], offz))));
-            const int kB = (sgn[2] > 0 ? top : bottom) ? s.count : max(0, min(s.count, (int)ceilf(__builtin_fmaf(fout, inv[2], offz))));
+            const int kin = max(0, min(s.count, (int)ceilf(__builtin_fmaf(fin, inv[2], offz))));
+            const int kout = max(0, min(s.count, (int)ceilf(__builtin_fmaf(fout, inv[2], offz))));
+            const int kA = (sgn[2] > 0 ? bottom : top) ? 0 : kin, kB = (sgn[2] > 0 ? top : bottom) ? s.count : kout;
             if (kB <= kA) continue;
             CellWalker wk;
             wk.init_from(s.q0, s.dq, sgn, inv, kA, kB);
@@ -360,9 +361,10 @@ __global__ void __launch_bounds__(256) pair_adjoint_slab_kernel(PairArgs a, AdjS
 // and walks exactly the sub-rays of its tilts that lie there, each once and over its whole length (a z
 // slab sets every sub-ray of every tilt up again for each slab, 65 times for 64 layers).  The rows'
 // voxel planes are in LDS in double, padded by the clamp border, and reach the gradient with one atomic
-// per voxel and run.  Lanes run along the detector axis on which y changes less, over the pixels of the run, and on
-// along the other: a wave's rays lie a pixel apart and rarely add to one voxel at once.  The planes leave room for one workgroup on a
-// compute unit, so it has sixteen waves to cover the LDS additions (a wave's ds_add_f64 takes nine cycles).
+// per voxel and run.  Lanes run along the detector axis on which y changes less, over the pixels of the
+// run, and on along the other: a wave's rays lie a pixel apart and rarely add to one voxel at once.  The
+// planes leave room for one workgroup on a compute unit, so it has sixteen waves to cover the LDS
+// additions (a wave's ds_add_f64 takes nine cycles).
 // 100 cubes of 64^3 by 41 tilts: 19.5 ms (22.2 with eight waves), against 156 ms with z slabs and eight
 // additions per cell.
 constexpr int kAdjFlatThreads = 1024;
@@ -416,7 +418,8 @@ __global__ void __launch_bounds__(kAdjFlatThreads) pair_adjoint_flat_kernel(Pair
         // misses it); tol is far above the rounding of texel_y and of the row's first pixel
         constexpr double tol = 1e-2;
         const double lo = (ys <= -1 ? -0.5 : (double)ys) - tol - y00;
-        const double hi = (ys + L >= v.ny ? ((double)v.bbMax[1] - (double)v.bbMin[1]) * ysc - 0.5 : (double)(ys + L)) + tol - y00;
+        const double face = ((double)v.bbMax[1] - (double)v.bbMin[1]) * ysc - 0.5;
+        const double hi = (ys + L >= v.ny ? face : (double)(ys + L)) + tol - y00;
         // a sub-ray's y is i gi + j gj and its offset in the pixel, om .. oM: the j with such sub-rays for some i,
         const double om = fmin(0.25 * gx, 0.75 * gx) + fmin(0.25 * gy, 0.75 * gy);
         const double oM = fmax(0.25 * gx, 0.75 * gx) + fmax(0.25 * gy, 0.75 * gy);
